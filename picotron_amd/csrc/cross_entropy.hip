@@ -236,12 +236,15 @@ struct RowRef {
   bool skip;
 };
 
+template <bool SMALL = false>
 __device__ __forceinline__ RowRef row_ref(int64_t row, int64_t inner, int64_t valid_inner,
                                           int64_t os, int64_t is,
                                           const int64_t* __restrict__ targets, int64_t tos,
                                           int64_t tis, int64_t ignore_index, int64_t gos = 0,
                                           int64_t gis = 0) {
-  const int64_t o = row / inner, ii = row - o * inner;
+  // SMALL: a call has fewer than 2^22 rows (checked on the host), so the decode fits 32 bits
+  const int64_t o = SMALL ? static_cast<uint32_t>(row) / static_cast<uint32_t>(inner) : row / inner;
+  const int64_t ii = row - o * inner;
   RowRef r;
   r.off = o * os + ii * is;
   r.goff = o * gos + ii * gis;
@@ -465,6 +468,168 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kMaxFi
     } else {
       __builtin_amdgcn_raw_buffer_store_b16(static_cast<unsigned short>(one.raw[0] & 0xffffu),
                                             gbuf, toff, 0, kWriteThrough);
+    }
+  }
+}
+
+// Short rows: WPR waves per row (one wave, four rows to a 256-thread workgroup, or one row to a
+// workgroup of WPR waves), VPL 16-byte vectors per lane, the whole row in registers.  A
+// 1024-thread workgroup per row leaves most of its lanes without an element and pays its launch,
+// its barrier and its 16-wave reduction for every row.
+//
+// The row is split into a head of the elements before its first boundary (16 bytes for one wave
+// per row, whose head and tail then fit its 64 lanes; a 128-byte line for several), a body of
+// 16-byte vectors and a tail of fewer than V elements.  The wave's max comes first and every
+// exp is taken against it, so the exps stay in fp32 registers (VPL * V of them) and the gradient
+// is one multiply and one rounding; several waves combine their (max, sum) through LDS behind
+// one barrier.  GRAD: write the gradient; otherwise the loss alone, with the row's log-sum-exp
+// for a deferred one.
+// What bounds it: latency and the number of rows in flight up to about 1 KB a row, HBM from about
+// 8 KB.  Nontemporal stores, since rows that are no multiple of a line share lines with their
+// neighbours in other waves and L2 merges the two halves (write-through: 20.8 against 16.4 us at
+// 520 bytes a row, 15.5 against 17.0 at 1024).  A loss call with its gradient over 16384 bf16
+// rows, graph-replayed, the 1024-thread kernels before and this one now: 64 logits 118 -> 17 us,
+// 260 120 -> 16, 1024 116 -> 21, 2048 118 -> 30, 4096 120 -> 51, 8192 131 -> 93, 12000 177 -> 140;
+// the loss alone 36 -> 13, 42 -> 14, 48 -> 16, 64 -> 20, 65 -> 32, 69 -> 48 (8192).
+template <typename T, int VPL, int WPR, bool GRAD>
+__global__ __launch_bounds__(WPR > 4 ? WPR * 64 : 256) void ce_short_kernel(
+    const T* logits, T* grad, int64_t inner, int64_t valid_inner, int64_t os, int64_t is,
+    int64_t gos, int64_t gis, int vocab, const int64_t* __restrict__ targets, int64_t tos,
+    int64_t tis, int64_t ignore_index, int write_grad, CeWork* __restrict__ ws, int64_t rows) {
+  static_assert(WPR == 1 || WPR >= 4, "a workgroup holds four rows of one wave, or one row");
+  constexpr int V = Elem<T>::VEC;
+  constexpr int LANES = 64 * WPR;
+  constexpr int RPB = WPR == 1 ? 4 : 1;
+  constexpr int kBoundary = WPR == 1 ? 16 : kLineBytes;
+  __shared__ float red_m[WPR];
+  __shared__ float red_s[WPR];
+  __shared__ float s_xt;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / 64);
+  const int lane = threadIdx.x % 64;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * RPB + (WPR == 1 ? wave : 0);
+  const int rl = WPR == 1 ? lane : static_cast<int>(threadIdx.x);
+  if constexpr (WPR == 1) {
+    if (row >= rows) return;  // the last workgroup's spare waves; no barrier below
+  }
+  const RowRef cur =
+      row_ref<true>(row, inner, valid_inner, os, is, targets, tos, tis, ignore_index, gos, gis);
+  const T* p = logits + cur.off;
+  T* g = GRAD ? grad + cur.goff : nullptr;  // in the same 16-byte phase as p (checked on the host)
+  const int lead = static_cast<int>(((kBoundary - (reinterpret_cast<uintptr_t>(p) & (kBoundary - 1))) &
+                                     (kBoundary - 1)) / sizeof(T));
+  const int head = lead < vocab ? lead : vocab;
+  const int nbody = (vocab - head) / V;
+  const int tail_start = head + nbody * V;
+  const int ntail = vocab - tail_start;
+  const auto buf = row_buffer(const_cast<T*>(p) + head, nbody * 16);
+  const auto gbuf = row_buffer(GRAD ? g + head : nullptr, GRAD ? nbody * 16 : 0);
+  // the one head or tail element of this lane, if any
+  const int my_edge = rl < head ? rl : (LANES - 1 - rl < ntail ? tail_start + (LANES - 1 - rl) : -1);
+
+  if (cur.skip) {
+    if constexpr (GRAD) {
+#pragma unroll
+      for (int k = 0; k < VPL; ++k)
+        __builtin_amdgcn_raw_buffer_store_b128(u32x4{0u, 0u, 0u, 0u}, gbuf, (rl + k * LANES) * 16, 0,
+                                               kNonTemporal);
+      if (my_edge >= 0) g[my_edge] = Elem<T>::from_f32(0.0f);
+    }
+    if (rl == 0) row_losses(ws)[row] = 0.0f;
+    return;
+  }
+  Vec16<T> v[VPL];
+#pragma unroll
+  for (int k = 0; k < VPL; ++k)
+    v[k].raw = __builtin_amdgcn_raw_buffer_load_b128(buf, (rl + k * LANES) * 16, 0, kNonTemporal);
+  const float edge = my_edge >= 0 ? Elem<T>::to_f32(p[my_edge]) : -INFINITY;
+  // The target logit: the row's one wave reads it with the row; for several waves thread 0
+  // passes it through LDS, so that it is read before any wave's first store.
+  const bool bad = cur.tgt < 0 || cur.tgt >= vocab;  // NaN loss and status bit 0
+  float xt = NAN;
+  if constexpr (WPR == 1) {
+    if (!bad) xt = Elem<T>::to_f32(p[cur.tgt]);
+  } else {
+    if (rl == 0) s_xt = bad ? NAN : Elem<T>::to_f32(p[cur.tgt]);
+  }
+  if (bad && rl == 0) atomicOr(&ws->status, 1);
+
+  float m = edge;
+#pragma unroll
+  for (int k = 0; k < VPL; ++k) {
+    if (rl + k * LANES >= nbody) {
+      const uint32_t ninf = kNegInfWord<T>;
+      v[k].raw = u32x4{ninf, ninf, ninf, ninf};
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) m = fmaxf(m, Elem<T>::to_f32(v[k].e[i]));
+  }
+  const float mw = wave_max(m);
+  const float ref = mw == -INFINITY ? 0.0f : mw;
+  float e[VPL][V];
+  const float e_edge = exp_shifted(edge, ref);
+  float s = e_edge;
+#pragma unroll
+  for (int k = 0; k < VPL; ++k) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      e[k][i] = exp_shifted(Elem<T>::to_f32(v[k].e[i]), ref);
+      s += e[k][i];
+    }
+  }
+  float M = mw, S = wave_sum(s);
+  if constexpr (WPR > 1) {
+    if (lane == 0) {
+      red_m[wave] = M;
+      red_s[wave] = S;
+    }
+    __syncthreads();
+    xt = s_xt;
+    M = red_m[0];
+#pragma unroll
+    for (int w = 1; w < WPR; ++w) M = fmaxf(M, red_m[w]);
+    const float refM = M == -INFINITY ? 0.0f : M;
+    S = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WPR; ++w) S += red_s[w] * exp_shifted(red_m[w], refM);
+  }
+  if (rl == 0) {
+    row_losses(ws)[row] = row_loss(M, S, xt);
+    if (!GRAD && write_grad == kGradDefer) row_lses(ws, rows)[row] = M + __logf(S);
+  }
+  if constexpr (GRAD) {
+    const float inv_n = inv_n_of(ws);
+    // exp(mw - M) / (S n): 0 for a wave that held only -inf, NaN for a row that did
+    const float f = (WPR > 1 ? exp_shifted(mw, M) : 1.0f) * (inv_n / S);
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+      Vec16<T> out;
+#pragma unroll
+      for (int i = 0; i < V; ++i) out.e[i] = Elem<T>::from_f32(e[k][i] * f);
+      __builtin_amdgcn_raw_buffer_store_b128(out.raw, gbuf, (rl + k * LANES) * 16, 0, kNonTemporal);
+    }
+    if (my_edge >= 0) g[my_edge] = Elem<T>::from_f32(e_edge * f);
+    if (!bad) {
+      // The owner rewrites the target over its own earlier store of that element, through the
+      // same kind of access, so the two stay in program order.
+      const int t = static_cast<int>(cur.tgt);
+      const bool in_body = t >= head && t < tail_start;
+      const int owner = t < head ? t : (in_body ? ((t - head) / V) % LANES : LANES - 1 - (t - tail_start));
+      if (rl == owner) {
+        const T gt = Elem<T>::from_f32(target_grad(M, S, xt, inv_n));
+        if (in_body) {
+          Vec16<T> one;
+          one.e[0] = gt;
+          const int toff = (t - head) * static_cast<int>(sizeof(T));
+          if constexpr (sizeof(T) == 4) {
+            __builtin_amdgcn_raw_buffer_store_b32(one.raw[0], gbuf, toff, 0, kNonTemporal);
+          } else {
+            __builtin_amdgcn_raw_buffer_store_b16(static_cast<unsigned short>(one.raw[0] & 0xffffu),
+                                                  gbuf, toff, 0, kNonTemporal);
+          }
+        } else {
+          g[t] = gt;
+        }
+      }
     }
   }
 }
@@ -935,11 +1100,12 @@ __global__ __launch_bounds__(kThreads) void ce_finish_kernel(CeWork* __restrict_
 // vector, one element per thread.
 constexpr int kScaleVecs = 4;
 
-template <typename T, bool ALIGNED>
+template <typename T, bool ALIGNED, int LANES>
 __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, int64_t inner,
                                                        int64_t valid_inner, int64_t os,
                                                        int64_t is, int64_t sos, int64_t sis,
                                                        int vocab, int64_t items, int64_t chunks,
+                                                       int chunk_vecs,
                                                        const int64_t* __restrict__ targets,
                                                        int64_t tos, int64_t tis,
                                                        int64_t ignore_index,
@@ -953,11 +1119,15 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, 
   } else {
     if (sc == 1.0f) return;
   }
+  constexpr int kGroups = 256 / LANES;  // items that a workgroup takes at a time
+  const int slot =
+      kGroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / LANES);
   const int64_t rows = items / chunks;
   // Item decode in 32 bits when the counts allow it (the usual case; a uniform branch):
   // 64-bit divisions are long scalar sequences ahead of every item's loads.
   const bool small = items <= 0xffffffffLL && inner <= 0xffffffffLL;
-  for (int64_t item = blockIdx.x; item < items; item += gridDim.x) {
+  for (int64_t item = static_cast<int64_t>(blockIdx.x) * kGroups + slot; item < items;
+       item += static_cast<int64_t>(gridDim.x) * kGroups) {
     int64_t row, c, o, ii;
     if (small) {
       const uint32_t r32 = static_cast<uint32_t>(item) / static_cast<uint32_t>(chunks);
@@ -1006,8 +1176,8 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, 
     // the code has no branches, all four loads are in flight together and every gradient
     // is computed before the first store (a load waited for after a store waits for the
     // store too).  Within a row, indexes fit in 32 bits.
-    const int cstart = static_cast<int>(c) * (256 * kScaleVecs);  // first vector of the chunk
-    const int cvecs = nbody - cstart < 256 * kScaleVecs ? nbody - cstart : 256 * kScaleVecs;
+    const int cstart = static_cast<int>(c) * chunk_vecs;  // first vector of the chunk
+    const int cvecs = nbody - cstart < chunk_vecs ? nbody - cstart : chunk_vecs;
     const int cbytes = cvecs > 0 ? cvecs * 16 : 0;
     T* cptr = body + static_cast<int64_t>(cstart) * V;
     const T* qptr = q + lead + static_cast<int64_t>(cstart) * V;
@@ -1017,8 +1187,8 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, 
     // the target's index in the chunk, or -1 when it is not there (ignored, in another
     // chunk, in the head or tail of an unaligned row, or outside the row)
     const int64_t trel64 = tgt - lead - static_cast<int64_t>(cstart) * V;
-    const int trel = (trel64 >= 0 && trel64 < int64_t{256} * kScaleVecs * V) ? static_cast<int>(trel64) : -1;
-    const int tid = static_cast<int>(threadIdx.x);
+    const int trel = (trel64 >= 0 && trel64 < int64_t{LANES} * kScaleVecs * V) ? static_cast<int>(trel64) : -1;
+    const int tid = static_cast<int>(threadIdx.x) % LANES;
     // In a row not on a line, the first item also takes the head elements and the item of
     // the body's last chunk the tail elements (one per thread), so that each end of the row
     // is written by one item; their loads go out with the vector loads, so that their
@@ -1027,7 +1197,7 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, 
     bool has_head = false, has_tail = false;
     const int tail_j = lead + nbody * V + tid;
     if constexpr (!ALIGNED) {
-      const int last_c = nbody > 0 ? (nbody - 1) / (256 * kScaleVecs) : 0;
+      const int last_c = nbody > 0 ? (nbody - 1) / chunk_vecs : 0;
       const bool read = !(kDefer && skip);  // an ignored fp16 row is written as zeros
       has_head = c == 0 && tid < lead;
       has_tail = c == last_c && tid < V && tail_j < vocab;
@@ -1037,7 +1207,7 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, 
     Vec16<T> in[kScaleVecs];
 #pragma unroll
     for (int k = 0; k < kScaleVecs; ++k)
-      in[k].raw = __builtin_amdgcn_raw_buffer_load_b128(lbuf, (k * 256 + tid) * 16, 0, kNonTemporal);
+      in[k].raw = __builtin_amdgcn_raw_buffer_load_b128(lbuf, (k * LANES + tid) * 16, 0, kNonTemporal);
     Vec16<T> out[kScaleVecs];
 #pragma unroll
     for (int k = 0; k < kScaleVecs; ++k) {
@@ -1046,7 +1216,7 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, 
         float y;
         if constexpr (kDefer) {
           y = exp_shifted(Elem<T>::to_f32(in[k].e[i]), lse);
-          if ((k * 256 + tid) * V + i == trel) y -= 1.0f;
+          if ((k * LANES + tid) * V + i == trel) y -= 1.0f;
           y = skip ? 0.0f : y * sc;
         } else {
           y = Elem<T>::to_f32(in[k].e[i]) * sc;
@@ -1059,7 +1229,7 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, 
     }
 #pragma unroll
     for (int k = 0; k < kScaleVecs; ++k)
-      __builtin_amdgcn_raw_buffer_store_b128(out[k].raw, sbuf, (k * 256 + tid) * 16, 0, kWriteThrough);
+      __builtin_amdgcn_raw_buffer_store_b128(out[k].raw, sbuf, (k * LANES + tid) * 16, 0, kWriteThrough);
     if constexpr (!ALIGNED) {
       // The value is rounded to fp32 before the conversion, as in the vector path (left
       // alone, the compiler fuses the last multiply and the fp16 conversion into one rounding).
@@ -1114,12 +1284,48 @@ void launch_rows(const CeRows& d, int write_grad, CeWork* ws, int64_t rows, hipS
 // elements) when every row is 16-byte aligned and, up to 8 vectors per thread, starts on a
 // 128-byte line; other rows take the batched kernel (the element-wise stream only for rows
 // of 2 GB and more).
+template <typename T, int VPL, int WPR>
+void launch_short(const CeRows& d, int write_grad, CeWork* ws, int64_t rows, hipStream_t st) {
+  constexpr int RPB = WPR == 1 ? 4 : 1;
+  const dim3 grid(static_cast<unsigned>((rows + RPB - 1) / RPB)), block(WPR > 4 ? WPR * 64 : 256);
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, static_cast<const T*>(d.logits),
+                       static_cast<T*>(d.grad), d.inner, d.valid_inner, d.os, d.is, d.gos, d.gis,
+                       d.vocab, d.targets, d.tos, d.tis, d.ignore_index, write_grad, ws, rows);
+  };
+  if (write_grad == kGradWrite) {
+    // fp16 never writes its gradient in the forward
+    if constexpr (!std::is_same<T, _Float16>::value) go(ce_short_kernel<T, VPL, WPR, true>);
+  } else {
+    go(ce_short_kernel<T, VPL, WPR, false>);
+  }
+}
+
+// The short-row kernels, by 16-byte vectors per row; false for a longer row.  One wave holds up
+// to 256 vectors (4096 bf16-row bytes: 30 us against 34 for four waves; 6000 bytes 48 against
+// 45).  With a gradient, four waves win up to 1536 vectors (24000 bytes a row: 140 us against 177
+// for the 1024-thread kernel; at 2048 vectors 198 against 190); without one, up to 1024 (the
+// 256-thread lse kernel streams longer rows as fast: 66 us either way at 24000 bytes in fp32).
+template <typename T>
+bool dispatch_short(const CeRows& d, int write_grad, CeWork* ws, int64_t rows, hipStream_t st) {
+  const int64_t nvec = (static_cast<int64_t>(d.vocab) + Elem<T>::VEC - 1) / Elem<T>::VEC;
+  if (nvec <= 64) return launch_short<T, 1, 1>(d, write_grad, ws, rows, st), true;
+  if (nvec <= 128) return launch_short<T, 2, 1>(d, write_grad, ws, rows, st), true;
+  if (nvec <= 256) return launch_short<T, 4, 1>(d, write_grad, ws, rows, st), true;
+  if (nvec <= 512) return launch_short<T, 2, 4>(d, write_grad, ws, rows, st), true;
+  if (nvec <= 1024) return launch_short<T, 4, 4>(d, write_grad, ws, rows, st), true;
+  if (write_grad == kGradWrite && nvec <= 1536)
+    return launch_short<T, 6, 4>(d, write_grad, ws, rows, st), true;
+  return false;
+}
+
 template <typename T>
 void dispatch_rows(bool aligned, bool lines, const CeRows& d, int write_grad, CeWork* ws, int64_t rows,
                    hipStream_t st) {
   const int64_t per_thread = (static_cast<int64_t>(d.vocab) + int64_t{kThreads} * Elem<T>::VEC - 1) /
                              (int64_t{kThreads} * Elem<T>::VEC);
   const int64_t row_bytes = static_cast<int64_t>(d.vocab) * static_cast<int64_t>(sizeof(T));
+  if (dispatch_short<T>(d, write_grad, ws, rows, st)) return;
   if (write_grad != kGradWrite && row_bytes + int64_t{kLseThreads} * kLseBatch * 16 < (int64_t{1} << 31)) {
     hipLaunchKernelGGL(ce_lse_kernel<T>, dim3(static_cast<unsigned>(rows)), dim3(kLseThreads), 0,
                        st, static_cast<const T*>(d.logits), d.inner, d.valid_inner, d.os, d.is,
@@ -1261,14 +1467,19 @@ int ce_run(const char* fn, const CeRows& d, int64_t outer, int64_t inner, int64_
   return check_launch(fn);
 }
 
-template <typename T, bool ALIGNED>
+template <typename T, bool ALIGNED, int LANES>
 void scale_launch_as(const CeRows& d, int64_t rows, const float* grad_output, const CeWork* ws,
                      hipStream_t st) {
-  // (row, chunk of 256 * kScaleVecs body vectors) items; a row's body has at most
+  // (row, chunk of the body) items, the chunks of a row equally long; a row's body has at most
   // vocab / VEC vectors whether or not it is aligned.
-  constexpr int64_t kChunk = 256 * Elem<T>::VEC * kScaleVecs;
-  const int64_t chunks = (d.vocab + kChunk - 1) / kChunk;
+  constexpr int kGroups = 256 / LANES;
+  constexpr int64_t kMost = LANES * kScaleVecs;  // vectors that an item's lanes hold
+  const int64_t nvec = (d.vocab + Elem<T>::VEC - 1) / Elem<T>::VEC;
+  const int64_t chunks = (nvec + kMost - 1) / kMost;
+  constexpr int kLineVecs = kLineBytes / 16;
+  const int chunk_vecs = static_cast<int>(((nvec + chunks - 1) / chunks + kLineVecs - 1) / kLineVecs * kLineVecs);
   const int64_t items = rows * chunks;
+  const int64_t groups = (items + kGroups - 1) / kGroups;
   // fp32 / bf16 scaling: a walk of up to 128 workgroups per CU, at most 4 resident per CU
   // (four 16-byte vectors in flight per thread: [8192, 128256] bf16 761 -> 714 us, vocab
   // 151936 935 -> 846 us); a one-shot grid streams no faster and makes the common
@@ -1282,26 +1493,36 @@ void scale_launch_as(const CeRows& d, int64_t rows, const float* grad_output, co
   static const int64_t walk_blocks = env_int("PT_CE_SCALE_BLOCKS_PER_CU", 128);
   const int64_t cap = (kDefer || walk_blocks <= 0) ? (int64_t{1} << 24) - 1
                                                    : static_cast<int64_t>(num_cus()) * walk_blocks;
-  const unsigned grid = static_cast<unsigned>(items < cap ? items : cap);
+  const unsigned grid = static_cast<unsigned>(groups < cap ? groups : cap);
   static const int walk_per_cu = static_cast<int>(env_int("PT_CE_SCALE_OCCUPANCY", 4));
   static const int defer_per_cu = static_cast<int>(env_int("PT_CE_DEFER_OCCUPANCY", 3));
-  const int per_cu = kDefer ? defer_per_cu : walk_per_cu;
-  const auto kernel = ce_scale_kernel<T, ALIGNED>;
+  // The limits are for items whose lanes hold all their vectors; shorter items run as many more,
+  // so that a CU keeps as much in flight, and one-wave items run unlimited.
+  const int full_per_cu = kDefer ? defer_per_cu : walk_per_cu;
+  const int per_cu = LANES == 64 ? 0 : static_cast<int>(full_per_cu * kMost / chunk_vecs);
+  const auto kernel = ce_scale_kernel<T, ALIGNED, LANES>;
   size_t lds = occupancy_lds(per_cu, 0);
   if (allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds) != PT_OK) lds = 0;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, st, static_cast<T*>(d.logits),
                      static_cast<const T*>(d.grad), d.inner, d.valid_inner, d.os, d.is, d.gos,
-                     d.gis, d.vocab, items, chunks, d.targets, d.tos, d.tis, d.ignore_index,
+                     d.gis, d.vocab, items, chunks, chunk_vecs, d.targets, d.tos, d.tis, d.ignore_index,
                      grad_output, ws);
 }
 
 template <typename T>
 void scale_launch(bool aligned, const CeRows& d, int64_t rows, const float* grad_output,
                   const CeWork* ws, hipStream_t st) {
+  const bool one_wave = (static_cast<int64_t>(d.vocab) + Elem<T>::VEC - 1) / Elem<T>::VEC <= 64 * kScaleVecs;
   if (aligned) {
-    scale_launch_as<T, true>(d, rows, grad_output, ws, st);
+    if (one_wave) {
+      scale_launch_as<T, true, 64>(d, rows, grad_output, ws, st);
+    } else {
+      scale_launch_as<T, true, 256>(d, rows, grad_output, ws, st);
+    }
+  } else if (one_wave) {
+    scale_launch_as<T, false, 64>(d, rows, grad_output, ws, st);
   } else {
-    scale_launch_as<T, false>(d, rows, grad_output, ws, st);
+    scale_launch_as<T, false, 256>(d, rows, grad_output, ws, st);
   }
 }
 

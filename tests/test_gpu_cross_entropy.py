@@ -216,6 +216,29 @@ def test_targets_at_the_splits_of_unaligned_rows(gpu, dtype, vocab):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("vectors", [64, 128, 256, 512, 1024, 1536])
+@pytest.mark.parametrize("extra,offset", [(0, 0), (0, 1), (1, 0), (-1, 3)])
+def test_short_rows_at_the_ends_of_their_kernels(gpu, dtype, vectors, extra, offset):
+    """The one-wave and four-wave row kernels (and, at 1024 and 1536 vectors, the longer-row
+    kernels beyond them) at the last row length that each takes, one logit more and one less,
+    on and off 16-byte boundaries; 7 rows leave a spare wave in the last workgroup.  The
+    backward's items change over at 256 vectors (one wave) and 1024 (one chunk per row)."""
+
+    es = torch.tensor([], dtype=dtype).element_size()
+    rows, vocab = 7, vectors * 16 // es + extra
+    flat = randn((offset + rows * vocab,), dtype, gpu, 31 * vocab + offset, 2.0)
+    logits = flat[offset:].view(rows, vocab)
+    picks = _line_split_targets(logits, rows, vocab, es)
+    picks[3] = -100
+    targets = torch.tensor(picks, device=gpu)
+    buf = _check(logits, targets, dtype)
+    if dtype != torch.float16:  # a scalar other than 1 rescales every kept row
+        scaled = buf.clone()
+        ops.cross_entropy_scale_grad(scaled, targets, torch.full((), 3.0, device=gpu))
+        assert torch.equal(scaled, (buf.float() * 3.0).to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("vocab", [1, 7, 63, 65, 129, 1031, 9001])
 @pytest.mark.parametrize("offset", [0, 1, 3, 8, 17, 31, 32, 47, 63, 64, 71])
 def test_row_starts_in_every_line_phase(gpu, dtype, vocab, offset):
