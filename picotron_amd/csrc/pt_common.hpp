@@ -144,6 +144,51 @@ __device__ __forceinline__ void store16(void* p, u32x4 v) {
   }
 }
 
+// A 16-byte vector at any element address of T: global accesses of the element's alignment, which
+// gfx950 serves at any address (one instruction, a line more when it straddles one).
+typedef unsigned int u32x4_at2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef unsigned int u32x4_at4 __attribute__((ext_vector_type(4), aligned(4)));
+template <typename T>
+struct AnyVec {
+  typedef u32x4_at4 type;
+};
+template <>
+struct AnyVec<_Float16> {
+  typedef u32x4_at2 type;
+};
+template <>
+struct AnyVec<__bf16> {
+  typedef u32x4_at2 type;
+};
+
+template <typename T, bool ALIGNED, bool NT>
+__device__ __forceinline__ u32x4 load_vec(const T* p) {
+  if constexpr (ALIGNED) {
+    return load16<NT>(p);
+  } else {
+    typedef typename AnyVec<T>::type V;
+    if constexpr (NT) {
+      return __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
+    } else {
+      return *reinterpret_cast<const V*>(p);
+    }
+  }
+}
+
+template <typename T, bool ALIGNED, bool NT>
+__device__ __forceinline__ void store_vec(T* p, u32x4 v) {
+  if constexpr (ALIGNED) {
+    store16<NT>(p, v);
+  } else {
+    typedef typename AnyVec<T>::type V;
+    if constexpr (NT) {
+      __builtin_nontemporal_store(static_cast<V>(v), reinterpret_cast<V*>(p));
+    } else {
+      *reinterpret_cast<V*>(p) = static_cast<V>(v);
+    }
+  }
+}
+
 // Loads VEC consecutive elements of storage type T as fp32.  ALIGNED: one 16-byte load
 // (caller guarantees alignment and that all VEC elements are in range); otherwise
 // element-wise loads of the first `valid` elements, zero-filling the rest.
@@ -235,6 +280,21 @@ __device__ __forceinline__ float wave_sum(float v) {
   v += dpp::move<dpp::kRowHalfMirror>(v);
   v += dpp::move<dpp::kRowMirror>(v);
   return ((dpp::lane(v, 0) + dpp::lane(v, 16)) + dpp::lane(v, 32)) + dpp::lane(v, 48);
+}
+
+// Sum over each 16-lane row of the wave, in every lane of it.
+__device__ __forceinline__ float row16_sum(float v) {
+  v += dpp::move<dpp::kQuadSwap1>(v);
+  v += dpp::move<dpp::kQuadSwap2>(v);
+  v += dpp::move<dpp::kRowHalfMirror>(v);
+  v += dpp::move<dpp::kRowMirror>(v);
+  return v;
+}
+
+// Sum of the four lanes l % 16 + {0, 16, 32, 48}, in that order; valid in lanes 0-15.
+__device__ __forceinline__ float quarters_sum(float v) {
+  const float a = __shfl_down(v, 16), b = __shfl_down(v, 32), c = __shfl_down(v, 48);
+  return ((v + a) + b) + c;
 }
 
 __device__ __forceinline__ float wave_max(float v) {

@@ -91,9 +91,9 @@ int fwd_impl(const char* fn, const void* x, int64_t xs, const void* res, int64_t
   a.h_s = hs;
   a.aligned = (cols % vec == 0) && rows_aligned(x_dtype, x, xs) && rows_aligned(x_dtype, y, ys) &&
               (!fused || (rows_aligned(x_dtype, res, res_s) && rows_aligned(x_dtype, h, hs))) &&
-              aligned16(weight) && vector_weight(x_dtype, w_dtype);
-  a.shape = a.aligned ? s : unaligned_shape(cols, vec);
-  a.blocks = fwd_blocks(rows, a.shape, num_cus());
+              aligned16(weight) && vector_weight(x_dtype, w_dtype) && !short_row(cols, vec);
+  a.shape = a.aligned ? s : general_shape(cols, vec, false);
+  a.blocks = fwd_blocks(rows, a.shape, num_cus(), a.aligned);
   a.st = as_stream(stream);
   bool launched;
   if (x_dtype == PT_FLOAT32) {
@@ -128,9 +128,9 @@ int bwd_impl(const char* fn, const void* dy, int64_t dys, const void* dh_in, int
   a.aligned = (cols % vec == 0) && rows_aligned(x_dtype, dy, dys) &&
               rows_aligned(x_dtype, x, xs) && (dx == nullptr || rows_aligned(x_dtype, dx, dxs)) &&
               (dh_in == nullptr || rows_aligned(x_dtype, dh_in, dh_in_s)) && aligned16(weight) &&
-              vector_weight(x_dtype, w_dtype);
-  a.shape = a.aligned ? s : unaligned_shape(cols, vec);
-  a.blocks = bwd_blocks(rows, a.shape);
+              vector_weight(x_dtype, w_dtype) && !short_row(cols, vec);
+  a.shape = a.aligned ? s : general_shape(cols, vec, true);
+  a.blocks = a.aligned ? bwd_blocks(rows, a.shape) : bwd_blocks_general(rows, cols, vec, a.shape);
   float* partial = nullptr;
   if (dweight) {
     const size_t need = static_cast<size_t>(a.blocks) * static_cast<size_t>(cols) * sizeof(float);
@@ -143,7 +143,7 @@ int bwd_impl(const char* fn, const void* dy, int64_t dys, const void* dh_in, int
       return fail(PT_EINVAL, std::string(fn) + ": workspace smaller than pt_rmsnorm_bwd_workspace_bytes()");
     if (!aligned16(workspace)) return fail(PT_EINVAL, std::string(fn) + ": workspace not aligned");
     // LDS combining the row slots' weight-gradient sums holds one fp32 per column.
-    if (bwd_waves(a.shape) / a.shape.wpr > 1 && cols * 4 > 160 * 1024)
+    if (row_slots(a.shape.wpr, bwd_waves(a.shape)) > 1 && cols * 4 > 160 * 1024)
       return fail(PT_EUNSUPPORTED, std::string(fn) + ": hidden size too large for the LDS combine");
     partial = static_cast<float*>(workspace);
   }
@@ -258,10 +258,10 @@ size_t pt_rmsnorm_bwd_workspace_bytes(int64_t rows, int64_t cols, int x_dtype) {
   const int vec = 16 / dtype_size(x_dtype);
   if (!choose_shape(cols, vec, cap_of(bwd_vpl_cap_for(tuning().bwd_vpl_cap, cols, vec)), &s))
     return 0;
-  // Enough for either path (aligned shape or the unaligned subset).
+  // Enough for either path (aligned or general).
   int64_t blocks = bwd_blocks(rows, s);
-  const int64_t ublocks = bwd_blocks(rows, unaligned_shape(cols, vec));
-  if (ublocks > blocks) blocks = ublocks;
+  const int64_t gblocks = bwd_blocks_general(rows, cols, vec, general_shape(cols, vec, true));
+  if (gblocks > blocks) blocks = gblocks;
   return static_cast<size_t>(blocks) * static_cast<size_t>(cols) * sizeof(float);
 }
 

@@ -10,10 +10,18 @@
 //            dW = sum_rows((g * x) * r)
 //
 // Layout: rows are `cols` contiguous elements, consecutive rows `*_row_stride` apart.
-// A row is owned by WPR waves (64*WPR lanes).  Lane `rl` of the row holds the 16-byte
-// vectors rl, rl + 64*WPR, ... (VPL of them), so each wave instruction moves 1 KiB of
-// contiguous memory, and the whole row stays in registers (packed in its storage type)
-// between the reduction and the elementwise pass: x and dy are read from HBM once.
+// A row is owned by WPR waves (64*WPR lanes), or by 16 lanes of a wave that holds four rows
+// (WPR 0).  Lane `rl` of the row holds the 16-byte vectors rl, rl + LANES, ... (VPL of them),
+// so each wave instruction moves 1 KiB of memory, and the whole row stays in registers (packed
+// in its storage type) between the reduction and the elementwise pass: x and dy are read from
+// HBM once.
+//
+// ALIGNED rows are whole 16-byte vectors on 16-byte boundaries.  Other rows -- any hidden size,
+// stride and base -- take the same vectors from the row's first element at whatever address that
+// is (global accesses of the element's alignment, which gfx950 serves unaligned), and the
+// hidden size's remainder of fewer than VEC elements one per lane.  [16383, 1370] bf16: forward
+// 18 us (the bytes at copy speed: 14), backward 31, against 62 and 72 for element-wide accesses
+// of the same lanes (each wave instruction then moves 128 bytes spread over a kilobyte).
 //
 // Backward weight gradient: each block accumulates sum((g*x)*r) for its rows in fp32
 // registers, combines its row slots in LDS in slot order, and writes one fp32 partial
@@ -40,75 +48,31 @@ constexpr bool kLoadNT = true;
 
 // ------------------------------------------------------------------ device helpers
 
-// Loads N consecutive weights starting at element `e` as fp32.
-//   WT == void : runtime dtype `wdt`, element loads (any alignment / type)
-//   VECTOR     : N*sizeof(WT) bytes as 16/32-byte vector loads (aligned)
-template <typename WT, int N, bool VECTOR>
-__device__ __forceinline__ void load_weight(const void* w, int wdt, int64_t e, int valid,
-                                            float (&out)[N]) {
-  if constexpr (std::is_void_v<WT>) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) out[i] = (i < valid) ? load_any(w, e + i, wdt) : 0.0f;
-  } else if constexpr (VECTOR) {
-    const WT* p = reinterpret_cast<const WT*>(w) + e;
-    constexpr int kBytes = N * static_cast<int>(sizeof(WT));
-    static_assert(kBytes == 16 || kBytes == 32, "weight vector size");
-    constexpr int kLoads = kBytes / 16;
-    constexpr int kPer = N / kLoads;
-#pragma unroll
-    for (int l = 0; l < kLoads; ++l) {
-      union {
-        u32x4 raw;
-        WT e[kPer];
-      } u;
-      u.raw = *reinterpret_cast<const u32x4*>(p + l * kPer);
-#pragma unroll
-      for (int i = 0; i < kPer; ++i) out[l * kPer + i] = static_cast<float>(u.e[i]);
-    }
-  } else {
-    const WT* p = reinterpret_cast<const WT*>(w) + e;
-#pragma unroll
-    for (int i = 0; i < N; ++i) out[i] = (i < valid) ? static_cast<float>(p[i]) : 0.0f;
-  }
+// 32 bytes that a lane without a vector of its own reads instead, where a row may be shorter than
+// one vector (its value is never used).
+static __device__ __align__(16) unsigned int kPad[8];
+
+// True if vector k of lane rl lies wholly inside the row.
+template <typename T, int LANES>
+__device__ __forceinline__ bool in_row(int rl, int k, int cols) {
+  return ((rl + k * LANES) + 1) * Elem<T>::VEC <= cols;
 }
 
-// Loads the weights of a lane's VPL vectors as fp32.  Vector path: branch-free -- a vector
-// past the row end loads the row's first weights instead (its products are never stored
-// or summed), so the loads issue back to back and their one wait comes at first use.
-// Element path: zero past the row end.
-template <typename WT, int VPL, int N, bool VECTOR>
-__device__ __forceinline__ void load_lane_weights(const void* w, int wdt, int rl, int lanes,
-                                                  int cols, float (&wv)[VPL][N]) {
-#pragma unroll
-  for (int k = 0; k < VPL; ++k) {
-    const int e = (rl + k * lanes) * N;
-    if constexpr (VECTOR) {
-      load_weight<WT, N, true>(w, wdt, e < cols ? e : 0, N, wv[k]);
-    } else {
-      load_weight<WT, N, false>(w, wdt, e, cols - e, wv[k]);
-    }
-  }
+// The remainder element of this lane (rows that are not whole vectors): its column, or -1.
+template <typename T>
+__device__ __forceinline__ int tail_col(int rl, int cols) {
+  const int tail = cols % Elem<T>::VEC;
+  return rl < tail ? cols - tail + rl : -1;
 }
 
 // A lane's weights kept as loaded and converted to fp32 at each use, which halves their
-// registers for 16-bit weights.  Vector path: 16-byte words, branch-free (a vector past the
-// row end loads the row's first weights; its products are never stored or summed).
-// Element path (runtime weight type): fp32 values, zero past the row end.
-template <typename WT, int VPL, int N, bool VECTOR>
+// registers for 16-bit weights: 16-byte words, branch-free (a vector past the row end loads
+// something else; its products are never stored or summed), so that the loads issue back to back
+// and their one wait comes at first use.  WT == void: a runtime weight type, loaded by elements
+// into fp32, zero past the row end.
+template <typename T, typename WT, int VPL, int LANES, bool ALIGNED>
 struct LaneWeights {
-  float f[VPL][N];
-  __device__ __forceinline__ void load(const void* w, int wdt, int rl, int lanes, int cols) {
-#pragma unroll
-    for (int k = 0; k < VPL; ++k) {
-      const int e = (rl + k * lanes) * N;
-      load_weight<WT, N, false>(w, wdt, e, cols - e, f[k]);
-    }
-  }
-  __device__ __forceinline__ float at(int k, int i) const { return f[k][i]; }
-};
-
-template <typename WT, int VPL, int N>
-struct LaneWeights<WT, VPL, N, true> {
+  static constexpr int N = Elem<T>::VEC;
   static constexpr int kPer = 16 / static_cast<int>(sizeof(WT));  // weights per 16-byte word
   static constexpr int kWords = N / kPer;
   static_assert(kWords * kPer == N, "weights of one vector fill whole 16-byte words");
@@ -117,13 +81,19 @@ struct LaneWeights<WT, VPL, N, true> {
     WT e[kPer];
   };
   Word wd[VPL][kWords];
-  __device__ __forceinline__ void load(const void* w, int, int rl, int lanes, int cols) {
+  float tail;
+  __device__ __forceinline__ void load(const void* w, int, int rl, int cols) {
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
-      const int e = (rl + k * lanes) * N;
-      const WT* p = reinterpret_cast<const WT*>(w) + (e < cols ? e : 0);
+      const WT* p = reinterpret_cast<const WT*>(w) + (rl + k * LANES) * N;
+      if (!in_row<T, LANES>(rl, k, cols))
+        p = ALIGNED ? reinterpret_cast<const WT*>(w) : reinterpret_cast<const WT*>(kPad);
 #pragma unroll
-      for (int l = 0; l < kWords; ++l) wd[k][l].raw = *reinterpret_cast<const u32x4*>(p + l * kPer);
+      for (int l = 0; l < kWords; ++l) wd[k][l].raw = load_vec<WT, ALIGNED, false>(p + l * kPer);
+    }
+    if constexpr (!ALIGNED) {
+      const int c = tail_col<T>(rl, cols);
+      tail = static_cast<float>(reinterpret_cast<const WT*>(w)[c < 0 ? 0 : c]);
     }
   }
   __device__ __forceinline__ float at(int k, int i) const {
@@ -131,10 +101,30 @@ struct LaneWeights<WT, VPL, N, true> {
   }
 };
 
-// The 16-byte vectors of one row held by a lane, packed in the storage type.
+template <typename T, int VPL, int LANES, bool ALIGNED>
+struct LaneWeights<T, void, VPL, LANES, ALIGNED> {
+  static constexpr int N = Elem<T>::VEC;
+  float f[VPL][N];
+  float tail;
+  __device__ __forceinline__ void load(const void* w, int wdt, int rl, int cols) {
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+      const bool in = in_row<T, LANES>(rl, k, cols);
+#pragma unroll
+      for (int i = 0; i < N; ++i) f[k][i] = in ? load_any(w, (rl + k * LANES) * N + i, wdt) : 0.0f;
+    }
+    const int c = tail_col<T>(rl, cols);
+    tail = load_any(w, c < 0 ? 0 : c, wdt);
+  }
+  __device__ __forceinline__ float at(int k, int i) const { return f[k][i]; }
+};
+
+// The 16-byte vectors of one row held by a lane, packed in the storage type, and its remainder
+// element (rows that are not whole vectors).
 template <typename T, int VPL>
 struct RowRegs {
   Vec16<T> v[VPL];
+  T tail;
 
   __device__ __forceinline__ float at(int k, int i) const { return Elem<T>::to_f32(v[k].e[i]); }
 
@@ -170,41 +160,31 @@ struct ResidualGrad {
   int64_t dh_in_stride;
 };
 
-// Loads the lane's VPL vectors of a row.  Aligned path: branch-free and unmasked -- a
-// lane whose vector lies past the row end loads the row's first vector instead, and the
-// caller ignores it (in_row()).  Nothing may consume the loaded registers here: loads
-// under divergent branches, or a select right after them, make the compiler wait for the
-// data at load time and so drain the next row's prefetch.  Element path: out-of-range
-// elements are zero-filled.
+// Loads the lane's part of a row, branch-free and unmasked: a lane whose vector (or remainder
+// element) lies past the row end loads something else instead -- the row's first vector, or
+// kPad where the row may hold none -- and the caller ignores it (in_row(), tail_col()).  Nothing
+// may consume the loaded registers here: loads under divergent branches, or a select right after
+// them, make the compiler wait for the data at load time and so drain the next row's prefetch.
 template <typename T, int VPL, int LANES, bool ALIGNED, bool NT>
 __device__ __forceinline__ void load_row(const T* __restrict__ row, int rl, int cols,
                                          RowRegs<T, VPL>& r) {
-  constexpr int V = Elem<T>::VEC;
 #pragma unroll
   for (int k = 0; k < VPL; ++k) {
-    const int e = (rl + k * LANES) * V;
-    const int valid = cols - e;
-    if constexpr (ALIGNED) {
-      r.v[k].raw = load16<NT>(row + (valid > 0 ? e : 0));
-    } else {
-#pragma unroll
-      for (int i = 0; i < V; ++i) {
-        r.v[k].e[i] = (i < valid) ? row[e + i] : Elem<T>::from_f32(0.0f);
-      }
-    }
+    const T* p = row + (rl + k * LANES) * Elem<T>::VEC;
+    if (!in_row<T, LANES>(rl, k, cols)) p = ALIGNED ? row : reinterpret_cast<const T*>(kPad);
+    r.v[k].raw = load_vec<T, ALIGNED, NT>(p);
+  }
+  if constexpr (!ALIGNED) {
+    const int c = tail_col<T>(rl, cols);
+    r.tail = row[c < 0 ? 0 : c];
   }
 }
 
-// True if vector k of lane rl lies inside the row (aligned path: whole vectors).
-template <typename T, int LANES>
-__device__ __forceinline__ bool in_row(int rl, int k, int cols) {
-  return (rl + k * LANES) * Elem<T>::VEC < cols;
-}
-
-// Stores of one row's 16-byte vectors.  Aligned rows: buffer stores with cache policy
-// POLICY through a resource over the row, whose base is wave-uniform (all lanes of a wave
-// work on the same row); the resource's range check drops vectors past the row end, so the
-// stores need no branch.  Unaligned rows: element stores of the in-range elements.
+// Stores of one row's vectors.  Aligned rows: buffer stores with cache policy POLICY through a
+// resource over the row, whose base is wave-uniform (all lanes of a wave work on the same row);
+// the resource's range check drops vectors past the row end, so the stores need no branch.
+// Other rows: nontemporal global stores of the vectors inside the row and of the remainder
+// elements (the ends of neighbouring rows share lines, which L2 then merges).
 // The forward's stores are write-through (kWriteThrough: 43.9 against 44.3 us per launch at
 // [16384, 4096] bf16), the backward's nontemporal (kNonTemporal: 71.9 against 72.2 us: with
 // two read streams beside it, write-through costs more than it saves).
@@ -219,25 +199,29 @@ struct RowStore {
   __device__ __forceinline__ void store(int rl, int k, const float (&o)[Elem<T>::VEC]) const {
     constexpr int V = Elem<T>::VEC;
     const int e = (rl + k * LANES) * V;
-    if constexpr (ALIGNED) {
-      Vec16<T> v;
+    Vec16<T> v;
 #pragma unroll
-      for (int i = 0; i < V; ++i) v.e[i] = Elem<T>::from_f32(o[i]);
+    for (int i = 0; i < V; ++i) v.e[i] = Elem<T>::from_f32(o[i]);
+    if constexpr (ALIGNED) {
       __builtin_amdgcn_raw_buffer_store_b128(v.raw, rsrc, e * static_cast<int>(sizeof(T)), 0,
                                              POLICY);
-    } else {
-      const int valid = cols - e;
-      if (valid > 0) store_f32<T, false>(row + e, o, valid);
+    } else if (in_row<T, LANES>(rl, k, cols)) {
+      store_vec<T, false, true>(row + e, v.raw);
     }
+  }
+  __device__ __forceinline__ void store_tail(int rl, float o) const {
+    const int c = tail_col<T>(rl, cols);
+    if (c >= 0) row[c] = Elem<T>::from_f32(o);
   }
 };
 
-// Sum over the WPR waves that share a row.  `red` holds 2*WAVES floats; `buf` alternates
-// between consecutive calls so one barrier per row suffices (a wave cannot overwrite a
+// Sum over the WPR waves (or, for WPR 0, the 16 lanes) that share a row.  `red` holds 2*WAVES
+// floats; `buf` alternates between consecutive calls so one barrier per row suffices (a wave cannot overwrite a
 // buffer before every wave has passed the barrier of the call in between).  Waves sum the
 // partials of their row in wave order, so every wave of a row gets the same value.
 template <int WPR, int WAVES>
 __device__ __forceinline__ float row_sum(float v, float* red, int wave, int lane, int buf) {
+  if constexpr (WPR == 0) return row16_sum(v);
   v = wave_sum(v);
   if constexpr (WPR > 1) {
     float* b = red + buf * WAVES;
@@ -252,9 +236,13 @@ __device__ __forceinline__ float row_sum(float v, float* red, int wave, int lane
   return v;
 }
 
+// Lanes of a row and row slots of a workgroup of `waves` waves.
+constexpr __host__ __device__ int row_lanes(int wpr) { return wpr == 0 ? 16 : 64 * wpr; }
+constexpr __host__ __device__ int row_slots(int wpr, int waves) { return waves * 64 / row_lanes(wpr); }
+
 // ------------------------------------------------------------------ forward
 //
-// Row groups: a block has WAVES/WPR row slots; at step `it` block b works on the group of
+// Row groups: a block has row_slots(WPR, WAVES) row slots; at step `it` block b works on the group of
 // rows starting at (it * gridDim.x + b) * slots, so at any moment all blocks work on one
 // compact window of rows (DRAM-friendly, like a non-persistent grid).  With a grid that
 // covers every row once (the default) each wave handles one row; smaller grids loop, and
@@ -272,23 +260,24 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_fwd_kernel(
     const T* __restrict__ x, int64_t xs, const void* __restrict__ w, int wdt, T* __restrict__ y,
     int64_t ys, float* __restrict__ rstd, int64_t rows, int cols, float eps, int iters,
     ResidualIn<T> rin) {
-  static_assert(WAVES % WPR == 0, "row slots must tile the block");
+  static_assert(WPR == 0 ? !ALIGNED : WAVES % WPR == 0, "row slots must tile the block");
   constexpr int V = Elem<T>::VEC;
-  constexpr int RPB = WAVES / WPR;
-  constexpr int LANES = 64 * WPR;
+  constexpr int RPB = row_slots(WPR, WAVES);
+  constexpr int LANES = row_lanes(WPR);
   __shared__ float red[2 * WAVES];
 
   const int wave = threadIdx.x / 64;
   const int lane = threadIdx.x % 64;
-  const int slot = wave / WPR;
-  const int rl = (wave % WPR) * 64 + lane;
+  const int slot = threadIdx.x / LANES;
+  const int rl = threadIdx.x % LANES;
   // iters = ceil(rows / group_stride), computed on the host: the same for every wave.
   const int64_t group_stride = static_cast<int64_t>(gridDim.x) * RPB;
   const int64_t r1 = rows;
   const float inv_cols = 1.0f / static_cast<float>(cols);
+  const bool has_tail = !ALIGNED && tail_col<T>(rl, cols) >= 0;
 
-  LaneWeights<WT, VPL, V, ALIGNED> wv;
-  wv.load(w, wdt, rl, LANES, cols);
+  LaneWeights<T, WT, VPL, LANES, ALIGNED> wv;
+  wv.load(w, wdt, rl, cols);
 
   using ResRegs = std::conditional_t<ADD, RowRegs<T, VPL>, NoRegs>;
   struct Row {
@@ -310,6 +299,10 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_fwd_kernel(
         }
         if (active) hs.store(rl, k, o);
       }
+      if constexpr (!ALIGNED) {
+        xr.tail = Elem<T>::from_f32(Elem<T>::to_f32(xr.tail) + Elem<T>::to_f32(rw.res.tail));
+        if (active) hs.store_tail(rl, Elem<T>::to_f32(xr.tail));
+      }
     }
     float ss = 0.0f;
     if (active) {
@@ -322,6 +315,10 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_fwd_kernel(
           part += f * f;
         }
         ss += in_row<T, LANES>(rl, k, cols) ? part : 0.0f;
+      }
+      if constexpr (!ALIGNED) {
+        const float f = Elem<T>::to_f32(xr.tail);
+        ss += has_tail ? f * f : 0.0f;
       }
     }
     xr.opaque();
@@ -337,6 +334,7 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_fwd_kernel(
       for (int i = 0; i < V; ++i) o[i] = (xr.at(k, i) * r) * wv.at(k, i);
       yst.store(rl, k, o);
     }
+    if constexpr (!ALIGNED) yst.store_tail(rl, (Elem<T>::to_f32(xr.tail) * r) * wv.tail);
   };
 
   // Rows past the end are clamped to the last row for loading (keeping the loads
@@ -434,26 +432,35 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_bwd_kernel(
     const void* __restrict__ w, int wdt, const float* __restrict__ rstd, T* dx,
     int64_t dxs, float* __restrict__ partial, int64_t rows, int cols, int iters,
     ResidualGrad<T> rg) {
-  static_assert(WAVES % WPR == 0, "row slots must tile the block");
+  static_assert(WPR == 0 ? !ALIGNED : WAVES % WPR == 0, "row slots must tile the block");
   constexpr int V = Elem<T>::VEC;
-  constexpr int RPB = WAVES / WPR;
-  constexpr int LANES = 64 * WPR;
+  constexpr int RPB = row_slots(WPR, WAVES);
+  constexpr int LANES = row_lanes(WPR);
   __shared__ float red[2 * WAVES];
   extern __shared__ float lds_dw[];  // [cols] when RPB > 1 and partial != nullptr
 
   const int wave = threadIdx.x / 64;
   const int lane = threadIdx.x % 64;
-  const int slot = wave / WPR;
-  const int rl = (wave % WPR) * 64 + lane;
+  const int slot = threadIdx.x / LANES;
+  const int rl = threadIdx.x % LANES;
   // iters = ceil(rows / group_stride), computed on the host: the same for every wave.
   const int64_t group_stride = static_cast<int64_t>(gridDim.x) * RPB;
   const int64_t r1 = rows;
   const bool want_dw = partial != nullptr;
   const float inv_cols = 1.0f / static_cast<float>(cols);
+  const bool has_tail = !ALIGNED && tail_col<T>(rl, cols) >= 0;
 
-  float wv[VPL][V];
-  load_lane_weights<WT, VPL, V, ALIGNED>(w, wdt, rl, LANES, cols, wv);
-  float acc[VPL][V];
+  float wv[VPL][V], wtail = 0.0f;
+  {
+    LaneWeights<T, WT, VPL, LANES, ALIGNED> lw;
+    lw.load(w, wdt, rl, cols);
+#pragma unroll
+    for (int k = 0; k < VPL; ++k)
+#pragma unroll
+      for (int i = 0; i < V; ++i) wv[k][i] = lw.at(k, i);
+    if constexpr (!ALIGNED) wtail = lw.tail;
+  }
+  float acc[VPL][V], acc_tail = 0.0f;
 #pragma unroll
   for (int k = 0; k < VPL; ++k)
 #pragma unroll
@@ -486,6 +493,10 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_bwd_kernel(
         for (int i = 0; i < V; ++i) part += (bf.g.at(k, i) * wv[k][i]) * bf.x.at(k, i);
         dot += in_row<T, LANES>(rl, k, cols) ? part : 0.0f;
       }
+      if constexpr (!ALIGNED) {
+        const float part = (Elem<T>::to_f32(bf.g.tail) * wtail) * Elem<T>::to_f32(bf.x.tail);
+        dot += has_tail ? part : 0.0f;
+      }
     }
     bf.g.opaque();
     bf.x.opaque();
@@ -507,12 +518,19 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_bwd_kernel(
         }
         dxst.store(rl, k, o);
       }
+      if constexpr (!ALIGNED) {
+        float o = r * (Elem<T>::to_f32(bf.g.tail) * wtail - (Elem<T>::to_f32(bf.x.tail) * r2) * dm);
+        if constexpr (ADD) o += Elem<T>::to_f32(bf.d.tail);
+        dxst.store_tail(rl, o);
+      }
     }
     if (want_dw) {
 #pragma unroll
       for (int k = 0; k < VPL; ++k)
 #pragma unroll
         for (int i = 0; i < V; ++i) acc[k][i] += (bf.g.at(k, i) * bf.x.at(k, i)) * r;
+      if constexpr (!ALIGNED)
+        acc_tail += (Elem<T>::to_f32(bf.g.tail) * Elem<T>::to_f32(bf.x.tail)) * r;
     }
   };
 
@@ -544,6 +562,15 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_bwd_kernel(
   if (!want_dw) return;
 
   float* prow = partial + static_cast<int64_t>(blockIdx.x) * cols;
+  if constexpr (WPR == 0) {
+    // A wave's four rows hold the same columns: lanes 0-15 get their sum.
+#pragma unroll
+    for (int k = 0; k < VPL; ++k)
+#pragma unroll
+      for (int i = 0; i < V; ++i) acc[k][i] = quarters_sum(acc[k][i]);
+    acc_tail = quarters_sum(acc_tail);
+  }
+  const int tail_c = ALIGNED ? -1 : tail_col<T>(rl, cols);
   if constexpr (RPB == 1) {
     // The block's single row slot: each lane owns distinct columns.
 #pragma unroll
@@ -551,20 +578,25 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_bwd_kernel(
       const int e = (rl + k * LANES) * V;
 #pragma unroll
       for (int i = 0; i < V; ++i)
-        if (e + i < cols) prow[e + i] = acc[k][i];
+        if (in_row<T, LANES>(rl, k, cols)) prow[e + i] = acc[k][i];
     }
+    if (tail_c >= 0) prow[tail_c] = acc_tail;
   } else {
-    // Row slots hold the same columns: combine them in LDS in slot order.
-    for (int s = 0; s < RPB; ++s) {
-      if (slot == s) {
+    // Row slots (for WPR 0, the waves) hold the same columns: combine them in LDS in slot order.
+    constexpr int kSums = WPR == 0 ? WAVES : RPB;
+    const int mine = WPR == 0 ? (lane < 16 ? wave : -1) : slot;
+    for (int s = 0; s < kSums; ++s) {
+      if (mine == s) {
 #pragma unroll
         for (int k = 0; k < VPL; ++k) {
           const int e = (rl + k * LANES) * V;
 #pragma unroll
           for (int i = 0; i < V; ++i) {
-            if (e + i < cols) lds_dw[e + i] = (s == 0) ? acc[k][i] : lds_dw[e + i] + acc[k][i];
+            if (in_row<T, LANES>(rl, k, cols))
+              lds_dw[e + i] = (s == 0) ? acc[k][i] : lds_dw[e + i] + acc[k][i];
           }
         }
+        if (tail_c >= 0) lds_dw[tail_c] = (s == 0) ? acc_tail : lds_dw[tail_c] + acc_tail;
       }
       __syncthreads();
     }
@@ -652,19 +684,28 @@ inline bool choose_shape(int64_t cols, int vec, int cap, Shape* s) {
   return true;
 }
 
-// The element-wise (unaligned) path is instantiated for fewer shapes: 4 waves per row
-// with 1..8 vectors per lane, or 16 waves per row with 8 or 16.
-inline Shape unaligned_shape(int64_t cols, int vec) {
+// The general kernels take rows that are not whole aligned vectors, weights of another 16-bit
+// type, and short rows of any alignment: up to kQuarterVecs vectors a row has 16 lanes (four rows
+// to a wave, so one reduction and one wave for four).  Measured per launch, one wave per row
+// against four rows per wave: [131072, 64] bf16 forward 25.5 -> 9.2 us, backward 37.4 -> 17.3;
+// [131072, 128] bf16 29.6 -> 12.9 and 40.4 -> 22.5; [131072, 128] fp32 (32 vectors) 36.5 -> 21.7
+// and 38.2 -> 37.4; at 40 vectors (fp32 160) the backward loses, 15.7 -> 20.9 with the forward equal.
+constexpr int64_t kQuarterVecs = 32;
+
+// Aligned rows that the general kernels take too.
+inline bool short_row(int64_t cols, int vec) { return (cols + vec - 1) / vec <= kQuarterVecs; }
+
+inline Shape general_shape(int64_t cols, int vec, bool backward) {
   const int64_t nvec = (cols + vec - 1) / vec;
-  const int64_t per4 = (nvec + 255) / 256;
-  if (per4 <= 8) return {pow2_at_least(per4), 4};
-  const int64_t per16 = (nvec + 1023) / 1024;
-  return {per16 <= 8 ? 8 : 16, 16};
+  if (nvec <= kQuarterVecs) return {pow2_at_least((nvec + 15) / 16), 0};
+  Shape s;
+  (void)choose_shape(cols, vec, backward ? bwd_vpl_cap_for(0, cols, vec) : fwd_vpl_cap_for(0, vec), &s);
+  return s;
 }
 
 // Calls f.template run<VPL, WPR>() for a runtime shape and returns true, or returns false
-// if that shape is not instantiated.  FULL selects the complete set (vector path);
-// otherwise the element-wise subset.
+// if that shape is not instantiated.  FULL: aligned rows, every shape that a tuning variable can
+// ask for; otherwise those that choose_shape gives for the default caps.
 template <bool FULL, typename F>
 bool dispatch_shape(const Shape& s, const F& f) {
 #define PT_RMS_CASE(V, W)            \
@@ -680,7 +721,17 @@ bool dispatch_shape(const Shape& s, const F& f) {
     PT_RMS_CASE(1, 16) PT_RMS_CASE(2, 16) PT_RMS_CASE(4, 16) PT_RMS_CASE(8, 16)
     PT_RMS_CASE(16, 16)
   } else {
-    PT_RMS_CASE(1, 4) PT_RMS_CASE(2, 4) PT_RMS_CASE(4, 4) PT_RMS_CASE(8, 4)
+    PT_RMS_CASE(1, 0) PT_RMS_CASE(2, 0) PT_RMS_CASE(1, 1)
+    if constexpr (F::kBackward) {
+      PT_RMS_CASE(1, 2) PT_RMS_CASE(1, 4) PT_RMS_CASE(2, 4)
+      PT_RMS_CASE(2, 8) PT_RMS_CASE(2, 16) PT_RMS_CASE(4, 16)
+    } else if constexpr (F::kVec == 8) {
+      PT_RMS_CASE(2, 1) PT_RMS_CASE(4, 1) PT_RMS_CASE(4, 2) PT_RMS_CASE(4, 4) PT_RMS_CASE(4, 8)
+      PT_RMS_CASE(4, 16)
+    } else {
+      PT_RMS_CASE(2, 1) PT_RMS_CASE(4, 1) PT_RMS_CASE(8, 1) PT_RMS_CASE(8, 2) PT_RMS_CASE(8, 4)
+      PT_RMS_CASE(8, 8)
+    }
     PT_RMS_CASE(8, 16) PT_RMS_CASE(16, 16)
   }
 #undef PT_RMS_CASE
@@ -691,20 +742,28 @@ inline int bwd_waves(const Shape& s) { return s.wpr > kBwdWaves ? s.wpr : kBwdWa
 
 // Backward grid = number of weight-gradient partial rows.
 inline int64_t bwd_blocks(int64_t rows, const Shape& s) {
-  const int64_t slots = bwd_waves(s) / s.wpr;
+  const int64_t slots = row_slots(s.wpr, bwd_waves(s));
   int64_t b = (rows + slots - 1) / slots;
   if (b > tuning().bwd_partials) b = tuning().bwd_partials;
   return b < 1 ? 1 : b;
 }
 
+// The general kernels' grid: at least two rows per workgroup up to 2048 vectors a row, which keeps
+// the partial rows of pt_rmsnorm_bwd_noalloc within its scratch at every size that it accepts.
+inline int64_t bwd_blocks_general(int64_t rows, int64_t cols, int vec, const Shape& s) {
+  const int64_t b = bwd_blocks(rows, s);
+  const int64_t pairs = (rows + 1) / 2;
+  return (cols + vec - 1) / vec <= 2048 && b > pairs ? (pairs < 1 ? 1 : pairs) : b;
+}
+
 inline int fwd_waves(const Shape& s) { return s.wpr > kFwdWaves ? s.wpr : kFwdWaves; }
 
 // Forward grid: one row per row slot (non-persistent, measured fastest), optionally capped
-// at PT_RMSNORM_FWD_BLOCKS_PER_CU blocks per CU.
-inline int64_t fwd_blocks(int64_t rows, const Shape& s, int ncu) {
-  const int64_t slots = fwd_waves(s) / s.wpr;
+// at PT_RMSNORM_FWD_BLOCKS_PER_CU blocks per CU (aligned rows; the general kernels do not loop).
+inline int64_t fwd_blocks(int64_t rows, const Shape& s, int ncu, bool aligned) {
+  const int64_t slots = row_slots(s.wpr, fwd_waves(s));
   int64_t b = (rows + slots - 1) / slots;
-  const int64_t per_cu = tuning().fwd_blocks_per_cu;
+  const int64_t per_cu = aligned ? tuning().fwd_blocks_per_cu : 0;
   if (per_cu > 0 && b > static_cast<int64_t>(ncu) * per_cu) b = static_cast<int64_t>(ncu) * per_cu;
   return b < 1 ? 1 : b;
 }
@@ -763,6 +822,8 @@ struct BwdArgs {
 
 template <typename T, typename WT, bool ALIGNED>
 struct FwdLaunch {
+  static constexpr bool kBackward = false;
+  static constexpr int kVec = Elem<T>::VEC;
   const FwdArgs& a;
   template <int VPL, int WPR, bool PERSIST, bool ADD>
   void go(int iters) const {
@@ -779,23 +840,29 @@ struct FwdLaunch {
   template <int VPL, int WPR>
   void run() const {
     constexpr int WAVES = WPR > kFwdWaves ? WPR : kFwdWaves;
-    const int iters = row_iters(a.rows, a.blocks, WAVES / WPR);
-    if (a.res != nullptr) {
-      if (iters == 1) {
-        go<VPL, WPR, false, true>(iters);
-      } else {
-        go<VPL, WPR, true, true>(iters);
+    const int iters = row_iters(a.rows, a.blocks, row_slots(WPR, WAVES));
+    if constexpr (ALIGNED) {
+      if (iters > 1) {
+        if (a.res != nullptr) {
+          go<VPL, WPR, true, true>(iters);
+        } else {
+          go<VPL, WPR, true, false>(iters);
+        }
+        return;
       }
-    } else if (iters == 1) {
-      go<VPL, WPR, false, false>(iters);
+    }
+    if (a.res != nullptr) {
+      go<VPL, WPR, false, true>(iters);
     } else {
-      go<VPL, WPR, true, false>(iters);
+      go<VPL, WPR, false, false>(iters);
     }
   }
 };
 
 template <typename T, typename WT, bool ALIGNED>
 struct BwdLaunch {
+  static constexpr bool kBackward = true;
+  static constexpr int kVec = Elem<T>::VEC;
   const BwdArgs& a;
   template <bool ADD, int VPL, int WPR, int WAVES>
   void go(size_t need, size_t lds, int iters) const {
@@ -810,7 +877,7 @@ struct BwdLaunch {
   template <int VPL, int WPR>
   void run() const {
     constexpr int WAVES = WPR > kBwdWaves ? WPR : kBwdWaves;
-    constexpr int RPB = WAVES / WPR;
+    constexpr int RPB = row_slots(WPR, WAVES);
     const size_t need =
         (RPB > 1 && a.partial != nullptr) ? static_cast<size_t>(a.cols) * sizeof(float) : 0;
     const size_t share = occupancy_lds(tuning().bwd_occupancy, 0);
@@ -824,8 +891,7 @@ struct BwdLaunch {
   }
 };
 
-// True when the 16-byte vector kernels apply: rows aligned (checked by the caller) and a
-// weight type with an instantiated vector path (x's type or fp32).
+// True when the aligned kernels have an instance for the weight type (x's type or fp32).
 inline bool vector_weight(int xdt, int wdt) { return wdt == xdt || wdt == PT_FLOAT32; }
 
 // Per-storage-type launchers; false if no kernel matched the shape (a bug, reported by
@@ -835,6 +901,8 @@ bool launch_fwd(const FwdArgs& a) {
   if (a.aligned && a.wdt == a.xdt) return dispatch_shape<true>(a.shape, FwdLaunch<T, T, true>{a});
   if (a.aligned && a.wdt == PT_FLOAT32)
     return dispatch_shape<true>(a.shape, FwdLaunch<T, float, true>{a});
+  if (a.wdt == a.xdt) return dispatch_shape<false>(a.shape, FwdLaunch<T, T, false>{a});
+  if (a.wdt == PT_FLOAT32) return dispatch_shape<false>(a.shape, FwdLaunch<T, float, false>{a});
   return dispatch_shape<false>(a.shape, FwdLaunch<T, void, false>{a});
 }
 
@@ -843,6 +911,8 @@ bool launch_bwd(const BwdArgs& a) {
   if (a.aligned && a.wdt == a.xdt) return dispatch_shape<true>(a.shape, BwdLaunch<T, T, true>{a});
   if (a.aligned && a.wdt == PT_FLOAT32)
     return dispatch_shape<true>(a.shape, BwdLaunch<T, float, true>{a});
+  if (a.wdt == a.xdt) return dispatch_shape<false>(a.shape, BwdLaunch<T, T, false>{a});
+  if (a.wdt == PT_FLOAT32) return dispatch_shape<false>(a.shape, BwdLaunch<T, float, false>{a});
   return dispatch_shape<false>(a.shape, BwdLaunch<T, void, false>{a});
 }
 

@@ -215,3 +215,39 @@ def test_banner_rows_report_the_hip_kernels(gpu):
     assert rows[0] == ("Triton kernels", "active: rmsnorm, swiglu")
     assert rows[1] == ("Triton status", "rmsnorm=real swiglu=real rope=real "
                        "attention=fallback cross_entropy=real adamw=real")
+
+
+@pytest.mark.parametrize("dtype,wdtype", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32),
+                                          (torch.float16, torch.bfloat16), (torch.float32, torch.float32),
+                                          (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("vectors,extra", [(0, 1), (1, -1), (1, 0), (2, 1), (16, 1), (32, 0), (32, 1), (64, 1), (128, -1),
+                                           (256, 1), (512, 3), (1024, 1)])
+@pytest.mark.parametrize("rows,offset", [(1, 0), (37, 1)])
+def test_general_rows_at_the_ends_of_their_shapes(gpu, dtype, wdtype, vectors, extra, rows, offset):
+    """Rows that are no whole 16-byte vectors, start at any element (offset) or are short, and
+    weights of another 16-bit type, at the row lengths where the lanes per row change (32, 64,
+    128, ... vectors) and below one vector; 37 rows leave spare row slots.  The residual form
+    runs with its result written over the incoming gradient."""
+
+    v = 16 // torch.tensor([], dtype=dtype).element_size()
+    cols = vectors * v + extra
+    seed = 7 * cols + rows
+
+    def make(s, scale=1.0):
+        return randn((offset + rows * cols,), dtype, gpu, seed + s, scale)[offset:].view(rows, cols)
+
+    x, dy, res, dh_in = make(1), make(2), make(3), make(4)
+    w = randn((offset + cols,), wdtype, gpu, seed + 5, 0.02, 1.0)[offset:]
+    _check(x, w, 1e-5, dy, dtype)
+    h, y, rstd = ops.residual_rmsnorm_fwd(x, res, w, 1e-5)
+    assert torch.equal(h, x + res)
+    y2, rstd2 = ops.rmsnorm_fwd(h, w, 1e-5)  # the same kernels without the add
+    assert torch.equal(y, y2) and torch.equal(rstd, rstd2)
+    dx, dw = ops.rmsnorm_bwd(dy, h, w, rstd)
+    dh, dw2 = ops.residual_rmsnorm_bwd(dy, dh_in, h, w, rstd)
+    assert torch.equal(dw, dw2)
+    out = dh_in.contiguous().clone()
+    in_place, _ = ops.residual_rmsnorm_bwd(dy, out, h, w, rstd, out=out)
+    assert torch.equal(in_place, dh)
+    # dx is rounded once more than dh, which adds dh_in before its one rounding
+    close(dh, dx.double() + dh_in.double(), dtype, scale=float(dx.abs().max()) + float(dh_in.abs().max()))
