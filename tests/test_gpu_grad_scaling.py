@@ -122,3 +122,33 @@ def test_fused_step_skips_on_overflow_and_rescales_unowned(gpu):
         assert float(opt.state[p]["step"]) == 1.0
         assert torch.equal(p.detach(), b)
         assert torch.equal(opt.state[p]["exp_avg"], m) and torch.equal(opt.state[p]["exp_avg_sq"], v)
+
+
+@pytest.mark.parametrize("sizes", [[1], [3, 1, 1023, 1025], [4 * 1024 * 3 + 5] * 7 + [2] * 30,
+                                   [12_000_001, 1023, 1, 2, 3, 11_000_003, 1024, 4097, 13_000_000]])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_gradient_walks_over_ranges_that_cross_tensors(gpu, sizes, offset):
+    """The statistics and scaling walks give each workgroup one range of the table's blocks (4
+    blocks each in a small table; 5 and 2 in the largest here, whose ranges end inside tensors
+    and span several): every element is counted and scaled once, gradients that start off a
+    16-byte boundary (offset 1) included, and a non-finite value is found at either end of any
+    tensor."""
+
+    from picotron_amd import ops
+
+    grads = [randn((n + offset,), torch.float32, gpu, 17 * i + n % 1000)[offset:] for i, n in enumerate(sizes)]
+    host, blocks = ops.adamw_table(grads, grads, grads, grads)
+    table = host.to(gpu)
+    total, _, found = ops.grad_stats(table, blocks)
+    ref = torch.sqrt(sum(g.double().square().sum() for g in grads))
+    assert abs(float(total) - float(ref)) <= 1e-6 * float(ref) and int(found) == 0
+    for i in {0, len(sizes) // 2, len(sizes) - 1}:
+        for at in (0, -1):
+            keep = grads[i][at].clone()
+            grads[i][at] = float("inf")
+            assert int(ops.grad_stats(table, blocks)[2]) == 1
+            grads[i][at] = keep
+    before = [g.clone() for g in grads]
+    ops.grad_scale(table, blocks, torch.full((), 0.37, device=gpu))
+    for g, b in zip(grads, before):
+        assert torch.equal(g, b * torch.full((), 0.37, device=gpu))
