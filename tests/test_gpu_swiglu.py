@@ -107,3 +107,20 @@ def test_autograd_surface_and_module(gpu):
     assert not mlp._triton_fallback_warned
     ref = mlp.down_projection(torch.nn.functional.silu(mlp.gate_projection(x)) * mlp.up_projection(x))
     close_fp32(out, ref, rtol=1e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n", [1, 8, 4097, 256 * 4 * 8 + 5])
+@pytest.mark.parametrize("offsets", [(0, 0, 0), (1, 0, 0), (0, 3, 1), (1, 1, 1)])
+def test_tails_and_streams_off_16_byte_boundaries(gpu, dtype, n, offsets):
+    """The elements past the last whole vector share the vectors' launch, and streams that start
+    at any element move the same vectors: the same bits as the aligned streams."""
+
+    g, u, dy = (randn((n + o,), dtype, gpu, 3 * n + i)[o:] for i, o in enumerate(offsets))
+    _check(g, u, dy, dtype)
+    ga, ua, da = g.clone(), u.clone(), dy.clone()
+    assert torch.equal(ops.swiglu_fwd(g, u), ops.swiglu_fwd(ga, ua))
+    for got, ref in zip(ops.swiglu_bwd(dy, g, u), ops.swiglu_bwd(da, ga, ua)):
+        assert torch.equal(got, ref)
+    only_up = ops.swiglu_bwd(dy, g, u, need_dgate=False)
+    assert only_up[0] is None and torch.equal(only_up[1], ops.swiglu_bwd(da, ga, ua)[1])
