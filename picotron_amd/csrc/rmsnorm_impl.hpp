@@ -399,10 +399,20 @@ __device__ __forceinline__ float column_group_sum(const float* __restrict__ part
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) s += v[u];
   }
-  // The remainder (fewer than kUnroll partials per group) in batches of 16 independent
-  // loads, so that it costs a few round trips rather than one per partial.
-#pragma unroll 16
-  for (; i < nparts; i += kFinishGroups) s += p[i * cols];
+  // The remainder (fewer than kUnroll partials per group) in batches of 16 independent loads,
+  // the last one's filled up with the last partial, counted as 0: a few round trips rather than
+  // one per partial ([256, 1024] bf16, 64 partials: the whole backward call 8.1 -> 6.4 us).
+  constexpr int kRest = 16;
+  for (; i < nparts; i += kFinishGroups * kRest) {
+    float v[kRest];
+#pragma unroll
+    for (int u = 0; u < kRest; ++u) {
+      const int64_t at = i + u * kFinishGroups;
+      v[u] = p[(at < nparts ? at : nparts - 1) * cols];
+    }
+#pragma unroll
+    for (int u = 0; u < kRest; ++u) s += i + u * kFinishGroups < nparts ? v[u] : 0.0f;
+  }
   return s;
 }
 
@@ -620,7 +630,7 @@ struct Tuning {
   int fwd_vpl_cap = 0;  // 0: by element size (fwd_vpl_cap_for)
   int bwd_vpl_cap = 0;  // 0: by row length (bwd_vpl_cap_for)
   int64_t fwd_blocks_per_cu = 0;  // 0: no cap (one row per row slot)
-  int64_t bwd_partials = 512;
+  int64_t bwd_partials = 0;  // 0: by the bytes of a row (bwd_partials_for)
   int fwd_occupancy = 0;  // resident forward workgroups per CU (0: no limit)
   int bwd_occupancy = 0;  // resident backward workgroups per CU (0: no limit)
 };
@@ -740,18 +750,39 @@ bool dispatch_shape(const Shape& s, const F& f) {
 
 inline int bwd_waves(const Shape& s) { return s.wpr > kBwdWaves ? s.wpr : kBwdWaves; }
 
-// Backward grid = number of weight-gradient partial rows.
-inline int64_t bwd_blocks(int64_t rows, const Shape& s) {
+// Most weight-gradient partial rows (workgroups) of the backward.
+constexpr int64_t kMostPartials = 512;
+
+// One workgroup per CU keeps HBM busy when its rows are long enough, two streams of the current
+// and the next row group in flight, and half as many partial rows are then written and summed.
+// 512 against 256 workgroups at 16384 rows, us per call (plain, residual form): bf16 2048 38.2 / 41.2
+// and 50.9 / 47.0, 2560 49.5 / 55.4 and 63.4 / 61.4, 4096 73.1 / 69.2 and 96.1 / 91.5, 5120 94.2 / 95.2
+// and 121.6 / 112.7; fp32 768 28.7 / 31.0 and 36.9 / 35.5, 1024 37.1 / 36.4 and 49.1 / 47.0, 2048 70.2 /
+// 67.5 and 92.8 / 88.2.  384 leave half of the CUs with two workgroups and are slower than both.
+// The residual form takes the plain one's count, so that their weight gradients are the same bits.
+inline int64_t bwd_partials_for(int64_t cols, int esize) {
+  if (tuning().bwd_partials > 0) return tuning().bwd_partials;
+  return cols * esize >= (esize == 4 ? 4096 : 8192) ? kMostPartials / 2 : kMostPartials;
+}
+
+// The most that bwd_partials_for gives, for sizing workspaces.
+inline int64_t most_partials() {
+  return tuning().bwd_partials > 0 ? tuning().bwd_partials : kMostPartials;
+}
+
+// Backward grid = number of weight-gradient partial rows, at most `partials`.
+inline int64_t bwd_blocks(int64_t rows, const Shape& s, int64_t partials) {
   const int64_t slots = row_slots(s.wpr, bwd_waves(s));
   int64_t b = (rows + slots - 1) / slots;
-  if (b > tuning().bwd_partials) b = tuning().bwd_partials;
+  if (b > partials) b = partials;
   return b < 1 ? 1 : b;
 }
 
 // The general kernels' grid: at least two rows per workgroup up to 2048 vectors a row, which keeps
 // the partial rows of pt_rmsnorm_bwd_noalloc within its scratch at every size that it accepts.
-inline int64_t bwd_blocks_general(int64_t rows, int64_t cols, int vec, const Shape& s) {
-  const int64_t b = bwd_blocks(rows, s);
+inline int64_t bwd_blocks_general(int64_t rows, int64_t cols, int vec, const Shape& s,
+                                  int64_t partials) {
+  const int64_t b = bwd_blocks(rows, s, partials);
   const int64_t pairs = (rows + 1) / 2;
   return (cols + vec - 1) / vec <= 2048 && b > pairs ? (pairs < 1 ? 1 : pairs) : b;
 }
