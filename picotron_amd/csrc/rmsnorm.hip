@@ -125,25 +125,22 @@ int bwd_impl(const char* fn, const void* dy, int64_t dys, const void* dh_in, int
     return fail(PT_EINVAL, std::string(fn) + ": row stride smaller than cols");
   const int vec = 16 / dtype_size(x_dtype);
   BwdArgs a{};
-  a.aligned = (cols % vec == 0) && rows_aligned(x_dtype, dy, dys) &&
-              rows_aligned(x_dtype, x, xs) && (dx == nullptr || rows_aligned(x_dtype, dx, dxs)) &&
-              (dh_in == nullptr || rows_aligned(x_dtype, dh_in, dh_in_s)) && aligned16(weight) &&
-              vector_weight(x_dtype, w_dtype) && !short_row(cols, vec);
+  const bool vectors = (cols % vec == 0) && rows_aligned(x_dtype, dy, dys) &&
+                       rows_aligned(x_dtype, x, xs) &&
+                       (dx == nullptr || rows_aligned(x_dtype, dx, dxs)) &&
+                       (dh_in == nullptr || rows_aligned(x_dtype, dh_in, dh_in_s)) &&
+                       aligned16(weight) && vector_weight(x_dtype, w_dtype);
+  a.aligned = vectors && !short_row(cols, vec);
   a.shape = a.aligned ? s : general_shape(cols, vec, true);
-  const auto blocks_at = [&](int64_t partials) {
-    return a.aligned ? bwd_blocks(rows, a.shape, partials)
-                     : bwd_blocks_general(rows, cols, vec, a.shape, partials);
-  };
-  a.blocks = blocks_at(bwd_partials_for(cols, dtype_size(x_dtype)));
+  const int64_t bound = bwd_partial_bound(rows, cols, vec, vectors, s);
+  a.blocks = bwd_blocks(rows, a.shape, bwd_partials_for(cols, dtype_size(x_dtype)));
+  if (a.blocks > bound) a.blocks = bound;
   float* partial = nullptr;
   if (dweight) {
-    const size_t need = static_cast<size_t>(a.blocks) * static_cast<size_t>(cols) * sizeof(float);
-    // the allocation-free entry point takes the sizes whose most partial rows fit its scratch
-    const size_t most = static_cast<size_t>(blocks_at(most_partials())) * static_cast<size_t>(cols) *
-                        sizeof(float);
-    if (static_scratch && most > workspace_bytes)
+    const size_t need = static_cast<size_t>(bound) * static_cast<size_t>(cols) * sizeof(float);
+    if (static_scratch && need > workspace_bytes)
       return fail(PT_EUNSUPPORTED,
-                  std::string(fn) + ": the weight-gradient partials need " + std::to_string(most) +
+                  std::string(fn) + ": the weight-gradient partials need " + std::to_string(need) +
                       " bytes, more than the library's static scratch of " +
                       std::to_string(workspace_bytes) + " bytes; use pt_rmsnorm_bwd");
     if (!workspace || workspace_bytes < need)
@@ -265,11 +262,10 @@ size_t pt_rmsnorm_bwd_workspace_bytes(int64_t rows, int64_t cols, int x_dtype) {
   const int vec = 16 / dtype_size(x_dtype);
   if (!choose_shape(cols, vec, cap_of(bwd_vpl_cap_for(tuning().bwd_vpl_cap, cols, vec)), &s))
     return 0;
-  // Enough for either path (aligned or general).
-  int64_t blocks = bwd_blocks(rows, s, most_partials());
-  const int64_t gblocks =
-      bwd_blocks_general(rows, cols, vec, general_shape(cols, vec, true), most_partials());
-  if (gblocks > blocks) blocks = gblocks;
+  // Enough for rows of any alignment.
+  int64_t blocks = bwd_partial_bound(rows, cols, vec, true, s);
+  const int64_t other = bwd_partial_bound(rows, cols, vec, false, s);
+  if (other > blocks) blocks = other;
   return static_cast<size_t>(blocks) * static_cast<size_t>(cols) * sizeof(float);
 }
 

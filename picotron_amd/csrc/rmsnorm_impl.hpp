@@ -778,13 +778,14 @@ inline int64_t bwd_blocks(int64_t rows, const Shape& s, int64_t partials) {
   return b < 1 ? 1 : b;
 }
 
-// The general kernels' grid: at least two rows per workgroup up to 2048 vectors a row, which keeps
-// the partial rows of pt_rmsnorm_bwd_noalloc within its scratch at every size that it accepts.
-inline int64_t bwd_blocks_general(int64_t rows, int64_t cols, int vec, const Shape& s,
-                                  int64_t partials) {
-  const int64_t b = bwd_blocks(rows, s, partials);
-  const int64_t pairs = (rows + 1) / 2;
-  return (cols + vec - 1) / vec <= 2048 && b > pairs ? (pairs < 1 ? 1 : pairs) : b;
+// Partial rows that a workspace has to hold, whatever the grid: the figure of the workspace
+// query, of the workspace check and of pt_rmsnorm_bwd_noalloc's size limit.  Whole aligned vectors
+// (`vectors`): the most workgroups of their shape; other rows: one per two rows up to 2048
+// vectors a row, one per row above.  The grid never exceeds it.
+inline int64_t bwd_partial_bound(int64_t rows, int64_t cols, int vec, bool vectors, const Shape& s) {
+  if (vectors) return bwd_blocks(rows, s, most_partials());
+  const int64_t b = (cols + vec - 1) / vec <= 2048 ? (rows + 1) / 2 : rows;
+  return b < 1 ? 1 : (b < most_partials() ? b : most_partials());
 }
 
 inline int fwd_waves(const Shape& s) { return s.wpr > kFwdWaves ? s.wpr : kFwdWaves; }
