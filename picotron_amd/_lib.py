@@ -1,17 +1,21 @@
-"""ctypes binding of ``libpicotron_hip.so`` (C ABI declared in ``include/picotron_hip.h``).
+"""Binding of ``libpicotron_hip.so`` (C ABI declared in ``include/picotron_hip.h``): ctypes for
+raw arguments, and the ``_native`` extension (``csrc/native.cpp``) for whole calls on tensors.
 
 The library is loaded lazily, once per process.  Loading fails loudly with
-:class:`HipLibraryUnavailable` (never a silent fallback) when the shared object is missing,
-was built for another ABI version, or cannot be opened.
+:class:`HipLibraryUnavailable` (never a silent fallback) when the shared object or the
+extension is missing, was built for another ABI version, or cannot be opened.
 """
 
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 import threading
 from ctypes import c_double, c_float, c_int, c_int64, c_size_t, c_void_p
 from pathlib import Path
+
+from torch import Tensor
 
 LIB_PATH = Path(os.environ.get("PICOTRON_HIP_LIB", Path(__file__).with_name("libpicotron_hip.so")))
 
@@ -146,6 +150,9 @@ class HipKernelError(RuntimeError):
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
+# entry point -> native launcher taking tensors; filled when the library loads
+_launchers: dict[str, object] = {}
+native = None  # the extension module
 _load_error: str | None = None
 
 
@@ -178,8 +185,36 @@ def _load() -> ctypes.CDLL:
         if version != ABI_VERSION:
             _load_error = f"{LIB_PATH} has ABI version {version}, expected {ABI_VERSION}; rebuild it"
             raise HipLibraryUnavailable(_load_error)
+        try:
+            _bind_native(lib)
+        except ImportError as error:
+            _load_error = (f"the native launchers cannot be loaded ({error}); build them with "
+                           "`python -m picotron_amd.build`")
+            raise HipLibraryUnavailable(_load_error) from error
         _lib = lib
         return lib
+
+
+def _bind_native(lib: ctypes.CDLL) -> None:
+    """Gives the extension the addresses of ``lib``'s entry points."""
+
+    global native
+    native = importlib.import_module("picotron_amd._native")
+    for name in native.ENTRY_POINTS:
+        native.bind(name, ctypes.cast(getattr(lib, name), c_void_p).value)
+    _launchers.update(
+        pt_rmsnorm_fwd=native.rmsnorm_fwd,
+        pt_rmsnorm_bwd=native.rmsnorm_bwd,
+        pt_residual_rmsnorm_fwd=native.residual_rmsnorm_fwd,
+        pt_residual_rmsnorm_bwd=native.residual_rmsnorm_bwd,
+        pt_swiglu_fwd=native.swiglu_fwd,
+        pt_swiglu_bwd=native.swiglu_bwd,
+        pt_rope=native.rope,
+        pt_cross_entropy=native.cross_entropy,
+        pt_cross_entropy_shifted=native.cross_entropy,
+        pt_cross_entropy_scale_grad=native.cross_entropy_scale_grad,
+        pt_cross_entropy_shifted_scale_grad=native.cross_entropy_scale_grad,
+    )
 
 
 def lib() -> ctypes.CDLL:
@@ -197,6 +232,8 @@ def is_available() -> bool:
 
 
 def unavailable_reason() -> str | None:
+    if _lib is not None:
+        return None
     try:
         lib()
     except HipLibraryUnavailable as error:
@@ -215,9 +252,9 @@ def check(fn: str, rc: int) -> None:
 _bound: dict[str, object] = {}
 
 
-def call(fn: str, *args) -> None:
-    """Call entry point ``fn`` and raise :class:`HipKernelError` on a nonzero return (the bound
-    function object is looked up once per name)."""
+def raw_call(fn: str, *args) -> None:
+    """Call entry point ``fn`` through ctypes and raise :class:`HipKernelError` on a nonzero
+    return (the bound function object is looked up once per name)."""
 
     f = _bound.get(fn)
     if f is None:
@@ -225,3 +262,21 @@ def call(fn: str, *args) -> None:
     rc = f(*args)
     if rc != PT_OK:
         check(fn, rc)
+
+
+def call(fn: str, *args):
+    """One launch of entry point ``fn``: with raw arguments (integers, addresses) through ctypes;
+    with tensors through its native launcher, which checks them, allocates the outputs and
+    returns them -- or returns None when they are not the plain case that it takes, and the
+    caller goes its general route to :func:`raw_call`."""
+
+    if not isinstance(args[0], Tensor):
+        return raw_call(fn, *args)
+    launcher = _launchers.get(fn)
+    if launcher is None:
+        lib()  # loads the library and fills the table (or raises)
+        launcher = _launchers[fn]
+    out = launcher(*args)
+    if type(out) is int:
+        check(fn, out)
+    return out

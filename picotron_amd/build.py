@@ -1,8 +1,10 @@
 """Build ``libpicotron_hip.so`` for gfx950 (MI355X) from ``picotron_amd/csrc``.
 
 Every ``*.hip`` translation unit is compiled by ``hipcc`` in parallel and linked into one
-shared library next to this file (in-tree, so it travels with the source tree).  The
-build always recompiles; nothing is cached between calls.
+shared library next to this file (in-tree, so it travels with the source tree), and
+``native.cpp`` (the launchers for torch tensors, host code against the installed torch) by the
+C++ compiler into ``_native.so`` beside it.  The build always recompiles; nothing is cached
+between calls.
 
 Usage: ``python -m picotron_amd.build [-j N] [-v]``.
 """
@@ -21,6 +23,8 @@ PACKAGE_DIR = Path(__file__).resolve().parent
 CSRC_DIR = PACKAGE_DIR / "csrc"
 BUILD_DIR = PACKAGE_DIR / "_build"
 LIB_PATH = PACKAGE_DIR / "libpicotron_hip.so"
+NATIVE_SOURCE = CSRC_DIR / "native.cpp"
+NATIVE_PATH = PACKAGE_DIR / "_native.so"
 INCLUDE_DIR = PACKAGE_DIR.parent / "include"
 
 OFFLOAD_ARCH = "gfx950"
@@ -67,6 +71,27 @@ def sources() -> list[Path]:
     return sorted(CSRC_DIR.glob("*.hip"))
 
 
+def build_native() -> Path:
+    """Compile the native launchers against the installed torch; returns the extension's path."""
+
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
+    if not cxx:
+        raise RuntimeError("no C++ compiler found (set CXX)")
+    includes = [*include_paths(), sysconfig.get_paths()["include"]]
+    tmp = NATIVE_PATH.with_suffix(".so.tmp")
+    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          *(arg for path in includes for arg in ("-isystem", path)), str(NATIVE_SOURCE), "-o", str(tmp),
+          *(f"-L{path}" for path in library_paths()), "-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python"])
+    os.replace(tmp, NATIVE_PATH)
+    return NATIVE_PATH
+
+
 def build(jobs: int | None = None, verbose: bool = False) -> Path:
     """Compile every HIP source and link the shared library; returns its path."""
 
@@ -84,10 +109,12 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
 
     objects: list[Path] = []
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
+        native = pool.submit(build_native)
         for obj, log in pool.map(compile_one, srcs):
             objects.append(obj)
             if verbose and log.strip():
                 print(log, file=sys.stderr)
+        native.result()
 
     tmp = LIB_PATH.with_suffix(".so.tmp")
     _run([hipcc, f"--offload-arch={OFFLOAD_ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(tmp)])
@@ -96,10 +123,10 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
 
 
 def ensure_built() -> Path:
-    """The in-tree library, built first when it is not there.  An existing library is used
+    """The in-tree library, built first when it or its launchers are not there.  An existing library is used
     as it is: after changing a source, call :func:`build`."""
 
-    if not LIB_PATH.exists():
+    if not LIB_PATH.exists() or not NATIVE_PATH.exists():
         build()
     return LIB_PATH
 

@@ -12,6 +12,7 @@ import os
 
 import torch
 from torch import Tensor
+from torch.autograd import forward_ad
 
 from picotron_amd import _lib, ops
 
@@ -38,6 +39,20 @@ def _process_reason() -> str:
 @torch.compiler.assume_constant_result
 def _device_supported(index: int) -> bool:
     return ops.device_supported(index)
+
+
+def no_graph(*tensors: Tensor) -> bool:
+    """True when an autograd Function over these inputs would record nothing, so that its forward
+    can be called directly (4 us less of host time): no gradient is asked for, and nothing else
+    looks at the call as a node -- forward-mode differentiation, a functorch transform (both of
+    which a Function refuses, and the caller falls back), jit tracing, torch.compile."""
+
+    if torch.is_grad_enabled():
+        for t in tensors:
+            if t.requires_grad:
+                return False
+    return (forward_ad._current_level < 0 and torch._C._get_tracing_state() is None
+            and not torch._C._are_functorch_transforms_active() and not torch.compiler.is_compiling())
 
 
 def require_hip(exc: type[RuntimeError], op: str, *tensors: Tensor) -> None:

@@ -51,7 +51,7 @@ from torch.autograd.function import once_differentiable
 from torch.nn import functional as F
 
 from picotron_amd import ops
-from picotron_amd.nn.triton_kernels._gate import require_hip
+from picotron_amd.nn.triton_kernels._gate import no_graph, require_hip
 
 IGNORE_INDEX = -100
 _CHECK_ENV = "PICOTRON_HIP_CE_CHECK"
@@ -244,6 +244,9 @@ def triton_cross_entropy(
             _validate(base, targets, ignore_index, True, False, next_targets=True)
             return _FusedShiftedCrossEntropy.apply(base, targets, int(ignore_index), False, True)
     _validate(logits, targets, ignore_index, shift, grad_in_place)
+    if not logits.requires_grad and no_graph(logits):
+        forward = ops.cross_entropy_shifted if shift else ops.cross_entropy
+        return forward(logits, targets, int(ignore_index))[0]
     if shift:
         return _FusedShiftedCrossEntropy.apply(logits, targets, int(ignore_index), bool(inplace),
                                                False)

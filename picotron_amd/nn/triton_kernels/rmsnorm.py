@@ -25,7 +25,7 @@ import torch
 from torch import Tensor
 
 from picotron_amd import _lib, ops
-from picotron_amd.nn.triton_kernels._gate import require_hip
+from picotron_amd.nn.triton_kernels._gate import no_graph, require_hip
 
 
 class TritonRMSNormUnavailable(RuntimeError):
@@ -150,6 +150,8 @@ def triton_rms_norm(hidden_states: Tensor, weight: Tensor, eps: float) -> Tensor
     """
 
     _validate_triton_inputs(hidden_states, weight)
+    if no_graph(hidden_states, weight):
+        return ops.rmsnorm_fwd(hidden_states, weight, eps)[0]
     return _RMSNormAutogradFunction.apply(hidden_states, weight, eps, True)
 
 
@@ -206,4 +208,6 @@ def triton_residual_rms_norm(
         raise TritonRMSNormUnavailable("residual must match hidden_states in shape and dtype.")
     if not residual.is_contiguous():
         raise TritonRMSNormUnavailable("HIP RMSNorm requires contiguous inputs.")
+    if no_graph(hidden_states, residual, weight):
+        return ops.residual_rmsnorm_fwd(hidden_states, residual, weight, eps)[:2]
     return _ResidualRMSNormFunction.apply(hidden_states, residual, weight, eps)

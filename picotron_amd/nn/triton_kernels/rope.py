@@ -16,7 +16,7 @@ import torch
 from torch import Tensor
 
 from picotron_amd import ops
-from picotron_amd.nn.triton_kernels._gate import require_hip
+from picotron_amd.nn.triton_kernels._gate import no_graph, require_hip
 
 
 class TritonRoPEUnavailable(RuntimeError):
@@ -104,6 +104,8 @@ def triton_apply_rotary_embedding(
     """
 
     _validate([states], cosine, sine)
+    if no_graph(states, cosine, sine):
+        return ops.rope(states, cosine.float(), sine.float(), layout=layout)[0]
     return _RoPEFunction.apply(layout, False, cosine.float(), sine.float(), states)[0]
 
 
@@ -113,5 +115,7 @@ def triton_apply_rotary_embedding_pair(
     """Rotate query and key (GQA: head counts may differ) in one kernel launch."""
 
     _validate([query, key], cosine, sine)
+    if no_graph(query, key, cosine, sine):
+        return ops.rope(query, cosine.float(), sine.float(), layout=layout, x1=key)
     out_q, out_k = _RoPEFunction.apply(layout, False, cosine.float(), sine.float(), query, key)
     return out_q, out_k

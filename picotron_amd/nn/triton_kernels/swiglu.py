@@ -15,7 +15,7 @@ from torch import Tensor
 from torch.nn import functional as F
 
 from picotron_amd import ops
-from picotron_amd.nn.triton_kernels._gate import require_hip
+from picotron_amd.nn.triton_kernels._gate import no_graph, require_hip
 
 
 class TritonSwiGLUUnavailable(RuntimeError):
@@ -73,6 +73,8 @@ def triton_swiglu(gate: Tensor, up: Tensor) -> Tensor:
     """Fused SwiGLU activation (HIP forward and backward)."""
 
     _validate_triton_inputs(gate, up)
+    if no_graph(gate, up):
+        return ops.swiglu_fwd(gate, up)
     return _SwiGLUAutogradFunction.apply(gate, up, True)
 
 

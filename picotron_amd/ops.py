@@ -1,5 +1,8 @@
 """Tensor-level launchers for the HIP kernels: shape/stride checks, output allocation,
-and the ctypes call on the caller's current HIP stream.
+and the library call on the caller's current HIP stream.
+
+Dense tensors in the kernels' own layout take a native launcher (``_lib.call`` with tensors), which
+does those steps in one native call; it leaves everything else to the general route below it.
 
 These functions never fall back to PyTorch arithmetic: if the library is missing they
 raise :class:`picotron_amd._lib.HipLibraryUnavailable`, and if an entry point rejects its
@@ -45,6 +48,15 @@ def _stream(device: torch.device) -> int:
     if _raw_stream is not None:
         return _raw_stream(index)
     return torch.cuda.current_stream(index).cuda_stream
+
+
+def _launch(fn: str, first: Tensor, *args):
+    """The native launcher of entry point ``fn`` on the current stream of ``first``'s device: its
+    outputs, or None when the call has to take the general route."""
+
+    if not first.is_cuda:
+        return None
+    return _lib.call(fn, first, *args, _stream(first.device))
 
 
 @functools.lru_cache(maxsize=256)
@@ -101,6 +113,9 @@ def rmsnorm_fwd(x: Tensor, weight: Tensor, eps: float) -> tuple[Tensor, Tensor]:
 
     if _compiling():
         return torch.ops.picotron_amd.rmsnorm_fwd(x, weight, float(eps))
+    out = _launch("pt_rmsnorm_fwd", x, weight, eps)
+    if out is not None:
+        return out
     device = _check_cuda(x, weight)
     cols = x.size(-1)
     if weight.dim() != 1 or weight.numel() != cols:
@@ -111,7 +126,7 @@ def rmsnorm_fwd(x: Tensor, weight: Tensor, eps: float) -> tuple[Tensor, Tensor]:
     y = torch.empty(x.shape, dtype=x.dtype, device=device)
     rstd = torch.empty(x.shape[:-1], dtype=torch.float32, device=device)
     y2 = y.view(-1, cols)
-    _lib.call(
+    _lib.raw_call(
         "pt_rmsnorm_fwd",
         x2.data_ptr(), x2.stride(0) if rows > 1 else cols, weight.data_ptr(), y2.data_ptr(), cols,
         rstd.data_ptr(), rows, cols, float(eps), dtype_code(x.dtype), dtype_code(weight.dtype),
@@ -133,6 +148,9 @@ def rmsnorm_bwd(
     if _compiling():
         dx, dw = torch.ops.picotron_amd.rmsnorm_bwd(dy, x, weight, rstd)
         return (dx if need_dx else None), (dw if need_dw else None)
+    out = _launch("pt_rmsnorm_bwd", dy, x, weight, rstd, bool(need_dx), bool(need_dw))
+    if out is not None:
+        return out
     device = _check_cuda(dy, x, weight, rstd)
     cols = x.size(-1)
     if dy.dtype != x.dtype:
@@ -153,7 +171,7 @@ def rmsnorm_bwd(
         ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=device)
     if not need_dx and not need_dw:
         return None, None
-    _lib.call(
+    _lib.raw_call(
         "pt_rmsnorm_bwd",
         dy2.data_ptr(), dy2.stride(0) if rows > 1 else cols, x2.data_ptr(),
         x2.stride(0) if rows > 1 else cols, weight.data_ptr(), rstd.data_ptr(), _ptr(dx), cols,
@@ -171,6 +189,9 @@ def residual_rmsnorm_fwd(
 
     if _compiling():
         return torch.ops.picotron_amd.residual_rmsnorm_fwd(x, residual, weight, float(eps))
+    out = _launch("pt_residual_rmsnorm_fwd", x, residual, weight, eps)
+    if out is not None:
+        return out
     device = _check_cuda(x, residual, weight)
     cols = x.size(-1)
     if residual.shape != x.shape or residual.dtype != x.dtype:
@@ -184,7 +205,7 @@ def residual_rmsnorm_fwd(
     h = torch.empty(x.shape, dtype=x.dtype, device=device)
     y = torch.empty(x.shape, dtype=x.dtype, device=device)
     rstd = torch.empty(x.shape[:-1], dtype=torch.float32, device=device)
-    _lib.call(
+    _lib.raw_call(
         "pt_residual_rmsnorm_fwd",
         x2.data_ptr(), x2.stride(0) if rows > 1 else cols, r2.data_ptr(),
         r2.stride(0) if rows > 1 else cols, weight.data_ptr(), h.data_ptr(), cols, y.data_ptr(), cols,
@@ -209,6 +230,10 @@ def residual_rmsnorm_bwd(
     if _compiling() and out is None:
         dh, dw = torch.ops.picotron_amd.residual_rmsnorm_bwd(dy, dh_in, h, weight, rstd)
         return dh, (dw if need_dw else None)
+    if out is None:
+        grads = _launch("pt_residual_rmsnorm_bwd", dy, dh_in, h, weight, rstd, bool(need_dw))
+        if grads is not None:
+            return grads
     device = _check_cuda(dy, h, weight, rstd)
     cols = h.size(-1)
     if dy.dtype != h.dtype:
@@ -236,7 +261,7 @@ def residual_rmsnorm_bwd(
     if need_dw:
         ws_bytes = _rmsnorm_ws_bytes(rows, cols, dtype_code(h.dtype))
         ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=device)
-    _lib.call(
+    _lib.raw_call(
         "pt_residual_rmsnorm_bwd",
         dy2.data_ptr(), dy2.stride(0) if rows > 1 else cols, _ptr(d2),
         (d2.stride(0) if rows > 1 else cols) if d2 is not None else 0, h2.data_ptr(),
@@ -259,12 +284,15 @@ def swiglu_fwd(gate: Tensor, up: Tensor) -> Tensor:
 
     if _compiling():
         return torch.ops.picotron_amd.swiglu_fwd(gate, up)
+    out = _launch("pt_swiglu_fwd", gate, up)
+    if out is not None:
+        return out
     device = _check_cuda(gate, up)
     if gate.shape != up.shape or gate.dtype != up.dtype:
         raise ValueError("SwiGLU gate and up must match in shape and dtype")
     gate, up = _flat(gate), _flat(up)
     out = torch.empty_like(gate)
-    _lib.call(
+    _lib.raw_call(
         "pt_swiglu_fwd", gate.data_ptr(), up.data_ptr(), out.data_ptr(), gate.numel(),
         dtype_code(gate.dtype), _stream(device),
     )
@@ -277,13 +305,16 @@ def swiglu_bwd(
     if _compiling():
         dg, du = torch.ops.picotron_amd.swiglu_bwd(dout, gate, up)
         return (dg if need_dgate else None), (du if need_dup else None)
+    out = _launch("pt_swiglu_bwd", dout, gate, up, bool(need_dgate), bool(need_dup))
+    if out is not None:
+        return out
     device = _check_cuda(dout, gate, up)
     if dout.dtype != gate.dtype:
         dout = dout.to(gate.dtype)
     dout, gate, up = _flat(dout), _flat(gate), _flat(up)
     dg = torch.empty_like(gate) if need_dgate else None
     du = torch.empty_like(up) if need_dup else None
-    _lib.call(
+    _lib.raw_call(
         "pt_swiglu_bwd", dout.data_ptr(), gate.data_ptr(), up.data_ptr(), _ptr(dg), _ptr(du),
         gate.numel(), dtype_code(gate.dtype), _stream(device),
     )
@@ -320,6 +351,10 @@ def rope(
             return torch.ops.picotron_amd.rope(x0, cos, sin, layout, bool(inverse)), None
         y0, y1 = torch.ops.picotron_amd.rope_pair(x0, x1, cos, sin, layout, bool(inverse))
         return y0, y1
+    if layout in LAYOUTS:
+        out = _launch("pt_rope", x0, x1, cos, sin, LAYOUTS[layout], bool(inverse))
+        if out is not None:
+            return out
     device = _check_cuda(x0, cos, sin) if x1 is None else _check_cuda(x0, x1, cos, sin)
     if layout not in LAYOUTS:
         raise ValueError(f"layout must be one of {sorted(LAYOUTS)}")
@@ -340,7 +375,7 @@ def rope(
     # comes back with the same memory layout.
     outs = [torch.empty_like(t) for t in tensors]
     descs = [_rope_desc(t, o) for t, o in zip(tensors, outs)]
-    _lib.call(
+    _lib.raw_call(
         "pt_rope",
         x0.data_ptr(), outs[0].data_ptr(), descs[0],
         None if x1 is None else x1.data_ptr(), None if x1 is None else outs[1].data_ptr(),
@@ -405,6 +440,10 @@ def ce_grad_buffer(logits: Tensor, class_dim: int = 1) -> Tensor | None:
     dimension, 1 for (N, C) and (N, C, d) inputs, 2 for the shifted (B, S, V) form.  None when
     the logits rows overlap in memory (an expanded tensor)."""
 
+    if logits.is_cuda and not _compiling() and _lib.is_available():
+        buffer = _lib.native.ce_grad_buffer(logits, class_dim)
+        if buffer is not None:
+            return buffer
     dims = list(zip(logits.shape, logits.stride()))
     rows = [d for i, d in enumerate(dims) if i != class_dim]
     if not rows_disjoint(rows, logits.size(class_dim)):
@@ -432,6 +471,9 @@ def cross_entropy(
     of range), readable with :func:`cross_entropy_status`.
     """
 
+    out = None if _compiling() else _launch("pt_cross_entropy", logits, targets, ignore_index, bool(write_grad), grad, 0)
+    if out is not None:
+        return out
     device = _check_cuda(logits, targets)
     outer, inner, os_, is_, vocab = ce_rows(logits)
     tos, tis = ce_target_strides(targets, outer, inner)
@@ -449,7 +491,7 @@ def cross_entropy(
     ws_bytes = _lib.lib().pt_cross_entropy_workspace_bytes(rows)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
     loss = torch.empty((), dtype=torch.float32, device=device)
-    _lib.call(
+    _lib.raw_call(
         "pt_cross_entropy",
         logits.data_ptr(), outer, inner, os_, is_, vocab, targets.data_ptr(), tos, tis,
         int(ignore_index), loss.data_ptr(), int(write_grad), _ptr(grad), gos, gis, ws.data_ptr(),
@@ -474,6 +516,8 @@ def cross_entropy_scale_grad(
     n_valid in ``workspace`` (the forward's): computed from ``logits`` into ``dlogits`` (rows
     in the same 16-byte phase) when ``logits`` is given, else over ``dlogits`` in place."""
 
+    if not _compiling() and _launch("pt_cross_entropy_scale_grad", dlogits, targets, grad_output, ignore_index, workspace, logits, 0):
+        return
     device = _check_cuda(dlogits, targets, grad_output)
     outer, inner, os_, is_, vocab = ce_rows(dlogits)
     tos, tis = ce_target_strides(targets, outer, inner)
@@ -483,7 +527,7 @@ def cross_entropy_scale_grad(
             raise ValueError("logits must match the gradient buffer")
         _, _, los, lis, _ = ce_rows(logits)
     go = grad_output.detach().to(torch.float32).reshape(())
-    _lib.call(
+    _lib.raw_call(
         "pt_cross_entropy_scale_grad",
         dlogits.data_ptr(), outer, inner, os_, is_, vocab, targets.data_ptr(), tos, tis,
         int(ignore_index), go.data_ptr(), _ptr(logits), los, lis, _ptr(workspace),
@@ -530,6 +574,10 @@ def cross_entropy_shifted(
     given (as in :func:`cross_entropy`), else over the logits.  ``next_targets``:
     ``input_ids`` is already the (B, S - 1) targets (the train loop's ``input_ids[:, 1:]``)."""
 
+    out = None if _compiling() else _launch("pt_cross_entropy_shifted", logits, input_ids, ignore_index, bool(write_grad), grad,
+                  2 if next_targets else 1)
+    if out is not None:
+        return out
     device = _check_cuda(logits, input_ids)
     b, s, bs, ss, v, ibs, iss = _shifted_desc(logits, input_ids, next_targets)
     gbs = gss = 0
@@ -547,7 +595,7 @@ def cross_entropy_shifted(
     ws_bytes = _lib.lib().pt_cross_entropy_workspace_bytes(b * s)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
     loss = torch.empty((), dtype=torch.float32, device=device)
-    _lib.call(
+    _lib.raw_call(
         "pt_cross_entropy_shifted",
         logits.data_ptr(), b, s, bs, ss, v, _ids_ptr(input_ids, next_targets), ibs, iss,
         int(ignore_index), loss.data_ptr(), int(write_grad), _ptr(grad), gbs, gss,
@@ -564,6 +612,9 @@ def cross_entropy_shifted_scale_grad(
     (fp16: as :func:`cross_entropy_scale_grad`, with the forward's ``workspace``, from
     ``logits`` into ``dlogits`` when ``logits`` is given)."""
 
+    if not _compiling() and _launch("pt_cross_entropy_shifted_scale_grad", dlogits, input_ids, grad_output, ignore_index,
+               workspace, logits, 2 if next_targets else 1):
+        return
     device = _check_cuda(dlogits, input_ids, grad_output)
     b, s, bs, ss, v, ibs, iss = _shifted_desc(dlogits, input_ids, next_targets)
     lbs = lss = 0
@@ -572,7 +623,7 @@ def cross_entropy_shifted_scale_grad(
             raise ValueError("logits must match the gradient buffer")
         lbs, lss = logits.stride(0), logits.stride(1)
     go = grad_output.detach().to(torch.float32).reshape(())
-    _lib.call(
+    _lib.raw_call(
         "pt_cross_entropy_shifted_scale_grad",
         dlogits.data_ptr(), b, s, bs, ss, v, _ids_ptr(input_ids, next_targets), ibs, iss,
         int(ignore_index), go.data_ptr(), _ptr(logits), lbs, lss, _ptr(workspace),
