@@ -10,9 +10,12 @@
 // is the backward of the forward.
 //
 // Work item = one 16-byte vector of a row (interleaved: V/2 pairs) or one vector from each
-// half of a row (rotate-half: V pairs).  Rows are the (batch, head, seq) positions of a
+// half of a row (rotate-half: V pairs), for up to kHeads heads of one position: the heads share
+// the item's cos and sin, which are twice the bytes of one head's vectors where those are 16-bit,
+// and the decode of its indices.  Rows are the (batch, head, seq) positions of a
 // strided view whose head_dim is contiguous; the host orders the three row dimensions by
-// decreasing stride so consecutive work items walk memory in address order.  Query and key
+// decreasing stride so consecutive work items walk memory in address order (item c of a
+// position's `chunks` takes heads c, c + chunks, ...).  Query and key
 // are handled by one launch (blocks [0, nb0) and [nb0, nb0 + nb1)).
 #include "pt_common.hpp"
 
@@ -30,35 +33,50 @@ __host__ __device__ constexpr int items_per_row(int head_dim) {
 struct RopeTensor {
   const void* x;
   void* y;
-  int64_t n[3];    // row dimensions, outer to inner (iteration order)
+  int64_t n[3];    // row dimensions, outer to inner (iteration order); the heads' in chunks
   int64_t xs[3];   // x strides of those dimensions (elements)
   int64_t ys[3];   // y strides
   int seq_dim;     // which of the three is the sequence dimension
-  int64_t rows;    // n[0] * n[1] * n[2]
-  int64_t items;   // rows * items_per_row
+  int head_dim;    // and which the heads
+  int heads;
+  int chunks;      // items that share a position's heads
+  int64_t xstep;   // elements from one of an item's heads to the next
+  int64_t ystep;
+  int64_t rows;    // batch * heads * seq
+  int64_t items;   // n[0] * n[1] * n[2] * items_per_row
   int64_t blocks;  // blocks assigned to this tensor
   int64_t ybytes;  // bytes from y to the end of its last row
 };
 
-// One work item in two phases, so that a thread can have several items' loads in flight
-// before it computes and stores any of them (the output may alias the input, so the
-// compiler would not move a later item's loads above an earlier item's stores).  The pair
+// One work item in two phases, so that a thread has every head's loads in flight before it
+// computes and stores any of them (the output may alias the input, so the
+// compiler would not move a later head's loads above an earlier head's stores).  The pair
 // members are held as a[p] (first) and b[p] (second): interleaved rows pair elements
 // (2i, 2i+1) of one vector, rotate-half rows pair element i of the first half with element
 // i of the second.  Item, row and the three row indices fit in 32 bits (pt_rope bounds
 // items by 2^32), so they are decoded with 32-bit divisions; only memory offsets are 64-bit.
 // WT (aligned rows only): stores through a buffer resource over y with the write-through
 // policy instead of nontemporal global stores.
+// Heads per item: two for interleaved rows, whose item is one vector of 16 bytes per head beside 32
+// bytes of cos and sin; one for rotate-half rows (two vectors beside 64 bytes).  Measured per launch
+// on q [8, 2048, 32, 128] + k [8, 2048, 8, 128] bf16 (the bytes at copy speed: 51.5 us): interleaved one
+// head 55.7, two 53.9, four 54.9, and at [1, 2048] 10.1, 8.9, 8.6; rotate-half 54.7, 55.2, 57.2 and
+// 8.6, 8.3, 8.8.
+template <int LAYOUT, bool ALIGNED>
+constexpr int kHeads = ALIGNED && LAYOUT == 0 ? 2 : 1;
+
 template <typename T, int LAYOUT, bool ALIGNED, bool NT, bool WT>
 struct RopeWork {
   static constexpr int V = ALIGNED ? Elem<T>::VEC : 2;
   static constexpr int P = LAYOUT == 0 ? V / 2 : (ALIGNED ? Elem<T>::VEC : 1);  // pairs
+  static constexpr int U = kHeads<LAYOUT, ALIGNED>;
   // Raw storage until store(): converting in load() would wait for the data there.
-  Vec16<T> va, vb;  // aligned: interleaved vector (va) or the two half vectors (va, vb)
+  Vec16<T> va[U], vb[U];  // aligned: interleaved vector (va) or the two half vectors (va, vb)
   T ea[2], eb[2];   // element path: interleaved (ea[0], ea[1]) or rotate-half (ea[0], eb[0])
   float c[P], s[P];
-  T* ya;  // first members (interleaved: the whole vector)
-  T* yb;  // second members (rotate-half)
+  T* ya;            // the first head's first members (interleaved: the whole vector)
+  int64_t ystep;    // from head to head
+  int count;        // heads
 
   __device__ __forceinline__ void load(const RopeTensor& t, uint32_t item, int head_dim,
                                        const float* __restrict__ cos_t,
@@ -75,29 +93,38 @@ struct RopeWork {
     idx[1] = r1 - static_cast<uint32_t>(idx[0]) * n1;
     const int64_t xo = idx[0] * t.xs[0] + idx[1] * t.xs[1] + idx[2] * t.xs[2];
     const int64_t yo = idx[0] * t.ys[0] + idx[1] * t.ys[1] + idx[2] * t.ys[2];
-    const int64_t pos = idx[t.seq_dim];
+    // selects, not an indexed array (which would live in scratch memory)
+    const int64_t pos = t.seq_dim == 0 ? idx[0] : (t.seq_dim == 1 ? idx[1] : idx[2]);
     const T* xr = static_cast<const T*>(t.x) + xo;
-    T* yr = static_cast<T*>(t.y) + yo;
     const int i0 = j * P;  // first pair of the item
-    if constexpr (LAYOUT == 0) {
-      if constexpr (ALIGNED) {
-        va.raw = load16<NT>(xr + j * V);
-      } else {
-        ea[0] = xr[2 * j];
-        ea[1] = xr[2 * j + 1];
+    ya = static_cast<T*>(t.y) + yo + (LAYOUT == 0 ? 2 * i0 : i0);
+    ystep = U > 1 ? t.ystep : 0;
+    count = 1;
+    if constexpr (ALIGNED) {
+      const int64_t xstep = U > 1 ? t.xstep : 0;
+      if constexpr (U > 1) {
+        const int first =
+            static_cast<int>(t.head_dim == 0 ? idx[0] : (t.head_dim == 1 ? idx[1] : idx[2]));
+        count = (t.heads - first + t.chunks - 1) / t.chunks;
       }
-      ya = yr + j * V;
-      yb = ya;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (u == 0 || u < count) {
+          const T* p = xr + u * xstep;
+          if constexpr (LAYOUT == 0) {
+            va[u].raw = load16<NT>(p + j * V);
+          } else {
+            va[u].raw = load16<NT>(p + i0);
+            vb[u].raw = load16<NT>(p + half + i0);
+          }
+        }
+      }
+    } else if constexpr (LAYOUT == 0) {
+      ea[0] = xr[2 * j];
+      ea[1] = xr[2 * j + 1];
     } else {
-      if constexpr (ALIGNED) {
-        va.raw = load16<NT>(xr + i0);
-        vb.raw = load16<NT>(xr + half + i0);
-      } else {
-        ea[0] = xr[j];
-        eb[0] = xr[half + j];
-      }
-      ya = yr + i0;
-      yb = yr + half + i0;
+      ea[0] = xr[j];
+      eb[0] = xr[half + j];
     }
     const float* cr = cos_t + pos * half + i0;
     const float* sr = sin_t + pos * half + i0;
@@ -111,73 +138,68 @@ struct RopeWork {
   template <int N>
   __device__ __forceinline__ static void put(__amdgpu_buffer_rsrc_t buf, const T* ybase, T* p,
                                              const float (&o)[N]) {
-    Vec16<T> v;
+    if constexpr (WT) {
+      Vec16<T> v;
 #pragma unroll
-    for (int i = 0; i < N; ++i) v.e[i] = Elem<T>::from_f32(o[i]);
-    const uint32_t off = static_cast<uint32_t>(reinterpret_cast<const char*>(p) -
-                                               reinterpret_cast<const char*>(ybase));
-    __builtin_amdgcn_raw_buffer_store_b128(v.raw, buf, off, 0, kWriteThrough);
+      for (int i = 0; i < N; ++i) v.e[i] = Elem<T>::from_f32(o[i]);
+      const uint32_t off = static_cast<uint32_t>(reinterpret_cast<const char*>(p) -
+                                                 reinterpret_cast<const char*>(ybase));
+      __builtin_amdgcn_raw_buffer_store_b128(v.raw, buf, off, 0, kWriteThrough);
+    } else {
+      store_f32<T, true, NT>(p, o, N);
+    }
   }
 
-  __device__ __forceinline__ void store(float sign, __amdgpu_buffer_rsrc_t buf,
+  __device__ __forceinline__ void store(float sign, int head_dim, __amdgpu_buffer_rsrc_t buf,
                                         const T* ybase) const {
-    float a[P], b[P];
-    if constexpr (LAYOUT == 0) {
+    const int half = head_dim / 2;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (u > 0 && u >= count) continue;
+      float a[P], b[P];
 #pragma unroll
       for (int p = 0; p < P; ++p) {
-        a[p] = Elem<T>::to_f32(ALIGNED ? va.e[2 * p] : ea[2 * p]);
-        b[p] = Elem<T>::to_f32(ALIGNED ? va.e[2 * p + 1] : ea[2 * p + 1]);
+        if constexpr (LAYOUT == 0) {
+          a[p] = Elem<T>::to_f32(ALIGNED ? va[u].e[2 * p] : ea[2 * p]);
+          b[p] = Elem<T>::to_f32(ALIGNED ? va[u].e[2 * p + 1] : ea[2 * p + 1]);
+        } else {
+          a[p] = Elem<T>::to_f32(ALIGNED ? va[u].e[p] : ea[p]);
+          b[p] = Elem<T>::to_f32(ALIGNED ? vb[u].e[p] : eb[p]);
+        }
       }
-    } else {
+      float oa[P], ob[P];
 #pragma unroll
       for (int p = 0; p < P; ++p) {
-        a[p] = Elem<T>::to_f32(ALIGNED ? va.e[p] : ea[p]);
-        b[p] = Elem<T>::to_f32(ALIGNED ? vb.e[p] : eb[p]);
+        const float sn = sign * s[p];
+        oa[p] = a[p] * c[p] - b[p] * sn;
+        ob[p] = a[p] * sn + b[p] * c[p];
       }
-    }
-    float oa[P], ob[P];
+      T* y = ya + u * ystep;
+      if constexpr (LAYOUT == 0) {
+        float o[V];
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-      const float sn = sign * s[p];
-      oa[p] = a[p] * c[p] - b[p] * sn;
-      ob[p] = a[p] * sn + b[p] * c[p];
-    }
-    if constexpr (LAYOUT == 0) {
-      float o[V];
-#pragma unroll
-      for (int p = 0; p < P; ++p) {
-        o[2 * p] = oa[p];
-        o[2 * p + 1] = ob[p];
-      }
-      if constexpr (ALIGNED && WT) {
-        put(buf, ybase, ya, o);
+        for (int p = 0; p < P; ++p) {
+          o[2 * p] = oa[p];
+          o[2 * p + 1] = ob[p];
+        }
+        if constexpr (ALIGNED) {
+          put(buf, ybase, y, o);
+        } else {
+          y[0] = Elem<T>::from_f32(o[0]);
+          y[1] = Elem<T>::from_f32(o[1]);
+        }
       } else if constexpr (ALIGNED) {
-        store_f32<T, true, NT>(ya, o, V);
+        put(buf, ybase, y, oa);
+        put(buf, ybase, y + half, ob);
       } else {
-        ya[0] = Elem<T>::from_f32(o[0]);
-        ya[1] = Elem<T>::from_f32(o[1]);
-      }
-    } else {
-      if constexpr (ALIGNED && WT) {
-        put(buf, ybase, ya, oa);
-        put(buf, ybase, yb, ob);
-      } else if constexpr (ALIGNED) {
-        store_f32<T, true, NT>(ya, oa, P);
-        store_f32<T, true, NT>(yb, ob, P);
-      } else {
-        ya[0] = Elem<T>::from_f32(oa[0]);
-        yb[0] = Elem<T>::from_f32(ob[0]);
+        y[0] = Elem<T>::from_f32(oa[0]);
+        y[half] = Elem<T>::from_f32(ob[0]);
       }
     }
   }
 };
 
-// A block covers 256 * kItemsPerThread items of one tensor: thread t takes items
-// base + t + 256 * u, all loaded before any is stored.  One item per thread measured best
-// on q [8, 2048, 32, 128] + k [8, 2048, 8, 128] bf16 (54.1 us; two 55.8, four 57.5): more
-// waves beat more loads per wave.
-constexpr int kItemsPerThread = 1;
-
+// Thread t of block b takes item b * 256 + t of its tensor.
 template <typename T, int LAYOUT, bool ALIGNED, bool NT, bool WT>
 __global__ __launch_bounds__(256) void rope_kernel(RopeTensor t0, RopeTensor t1, int head_dim,
                                                    const float* __restrict__ cos_t,
@@ -188,19 +210,13 @@ __global__ __launch_bounds__(256) void rope_kernel(RopeTensor t0, RopeTensor t1,
     b -= static_cast<uint32_t>(t0.blocks);
     t = &t1;
   }
-  const uint32_t base = b * (256u * kItemsPerThread) + threadIdx.x;
-  const uint32_t items = static_cast<uint32_t>(t->items);
-  RopeWork<T, LAYOUT, ALIGNED, NT, WT> w[kItemsPerThread];
-#pragma unroll
-  for (int u = 0; u < kItemsPerThread; ++u) {
-    const uint32_t item = base + 256u * u;
-    if (item < items) w[u].load(*t, item, head_dim, cos_t, sin_t);
-  }
+  const uint32_t item = b * 256u + threadIdx.x;
   // y's span fits a buffer resource whenever WT is set (checked on the host); unused otherwise
   const auto ybuf = uniform_buffer(t->y, WT ? static_cast<int>(t->ybytes) : 0);
-#pragma unroll
-  for (int u = 0; u < kItemsPerThread; ++u)
-    if (base + 256u * u < items) w[u].store(sign, ybuf, static_cast<const T*>(t->y));
+  if (item >= static_cast<uint32_t>(t->items)) return;
+  RopeWork<T, LAYOUT, ALIGNED, NT, WT> w;
+  w.load(*t, item, head_dim, cos_t, sin_t);
+  w.store(sign, head_dim, ybuf, static_cast<const T*>(t->y));
 }
 
 bool parse(const void* x, void* y, const int64_t* d, int64_t head_dim, int64_t table_rows,
@@ -235,7 +251,9 @@ bool parse(const void* x, void* y, const int64_t* d, int64_t head_dim, int64_t t
     t->xs[i] = xs[ord[i]];
     t->ys[i] = ys[ord[i]];
     if (ord[i] == 2) t->seq_dim = i;
+    if (ord[i] == 1) t->head_dim = i;
   }
+  t->heads = static_cast<int>(sz[1]);
   t->rows = sz[0] * sz[1] * sz[2];
   // y's extent in bytes (-1 when a stride is negative): the write-through stores address y
   // through a buffer resource, so they need it to fit 31 bits
@@ -259,20 +277,21 @@ bool parse(const void* x, void* y, const int64_t* d, int64_t head_dim, int64_t t
 
 constexpr int64_t kNontemporalBytes = int64_t{64} << 20;
 
-// Resident workgroups per CU; PT_ROPE_OCCUPANCY overrides it (0: no limit).  One item
-// per thread keeps little in flight, so the limit stays high: at 6 the 4-layer q + k
-// benchmark measured 54.3-54.5 us per launch against 54.7 with the full 8, and 60.5-66.1
-// at 4 and 3.
-int rope_occupancy() {
-  static const int v = static_cast<int>(env_int("PT_ROPE_OCCUPANCY", 6));
-  return v;
+// Resident workgroups per CU (0: no limit); PT_ROPE_OCCUPANCY overrides it.  One item
+// per thread keeps little in flight, so the limit stays high: rotate-half rows at 6 measured
+// 54.3-54.5 us per launch on the 4-layer q + k benchmark against 54.7 with the full 8, and 60.5-66.1
+// at 4 and 3; interleaved rows, with half as much in flight per head, lose at 6 (one head per item 62.6
+// against 55.7 without a limit, two 54.1 against 53.9).
+int rope_occupancy(int layout) {
+  static const int v = static_cast<int>(env_int("PT_ROPE_OCCUPANCY", -1));
+  return v >= 0 ? v : (layout == 0 ? 0 : 6);
 }
 
 template <typename K>
-void launch_limited(K kernel, unsigned grid, hipStream_t st, const RopeTensor& t0,
+void launch_limited(K kernel, int layout, unsigned grid, hipStream_t st, const RopeTensor& t0,
                     const RopeTensor& t1, int head_dim, const float* c, const float* s,
                     float sign) {
-  size_t lds = occupancy_lds(rope_occupancy(), 0);
+  size_t lds = occupancy_lds(rope_occupancy(layout), 0);
   if (allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds) != PT_OK) lds = 0;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, st, t0, t1, head_dim, c, s, sign);
 }
@@ -281,11 +300,18 @@ template <typename T, int LAYOUT, bool ALIGNED>
 void launch(RopeTensor& t0, RopeTensor& t1, int head_dim, const float* c, const float* s,
             float sign, hipStream_t st) {
   const int per_row = items_per_row<T, LAYOUT, ALIGNED>(head_dim);
-  t0.items = t0.rows * per_row;
-  t1.items = t1.rows * per_row;
-  constexpr int64_t kPerBlock = 256 * kItemsPerThread;
-  t0.blocks = (t0.items + kPerBlock - 1) / kPerBlock;
-  t1.blocks = (t1.items + kPerBlock - 1) / kPerBlock;
+  constexpr int kPer = kHeads<LAYOUT, ALIGNED>;
+  for (RopeTensor* t : {&t0, &t1}) {
+    t->chunks = static_cast<int>((t->heads + kPer - 1) / kPer);
+    t->xstep = t->xs[t->head_dim] * t->chunks;
+    t->ystep = t->ys[t->head_dim] * t->chunks;
+    t->items = 0;
+    if (t->rows > 0) {
+      t->n[t->head_dim] = t->chunks;
+      t->items = t->rows / t->heads * t->chunks * per_row;
+    }
+    t->blocks = (t->items + 255) / 256;
+  }
   const int64_t blocks = t0.blocks + t1.blocks;
   if (blocks == 0) return;
   // pt_rope has checked that (rows0 + rows1) * head_dim / 2 + 512 < 2^32, which bounds
@@ -300,14 +326,14 @@ void launch(RopeTensor& t0, RopeTensor& t1, int head_dim, const float* c, const 
   };
   if (bytes > kNontemporalBytes) {
     if (ALIGNED && fits(t0) && fits(t1)) {
-      launch_limited(rope_kernel<T, LAYOUT, ALIGNED, true, ALIGNED>, static_cast<unsigned>(blocks),
+      launch_limited(rope_kernel<T, LAYOUT, ALIGNED, true, ALIGNED>, LAYOUT, static_cast<unsigned>(blocks),
                      st, t0, t1, head_dim, c, s, sign);
     } else {
-      launch_limited(rope_kernel<T, LAYOUT, ALIGNED, true, false>, static_cast<unsigned>(blocks),
+      launch_limited(rope_kernel<T, LAYOUT, ALIGNED, true, false>, LAYOUT, static_cast<unsigned>(blocks),
                      st, t0, t1, head_dim, c, s, sign);
     }
   } else {
-    launch_limited(rope_kernel<T, LAYOUT, ALIGNED, false, false>, static_cast<unsigned>(blocks),
+    launch_limited(rope_kernel<T, LAYOUT, ALIGNED, false, false>, LAYOUT, static_cast<unsigned>(blocks),
                    st, t0, t1, head_dim, c, s, sign);
   }
 }
@@ -361,6 +387,7 @@ int pt_rope(const void* x0, void* y0, const int64_t* desc0, const void* x1, void
   } else {
     t1.n[0] = t1.n[1] = t1.n[2] = 1;
     t1.rows = 0;
+    t1.heads = 1;
   }
   // Empty tensors may carry null data pointers; non-empty ones may not.
   if (t0.rows > 0 && (!x0 || !y0)) return fail(PT_EINVAL, "pt_rope: null first tensor");

@@ -152,3 +152,30 @@ def test_module_shares_one_table_across_sequence_lengths(gpu):
     assert not rope._triton_fallback_warned
     assert len(rope._fp32_tables) == 1
     assert next(iter(rope._fp32_tables.values()))[0].size(0) == 96
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,kv_heads", [(1, 1), (2, 3), (5, 2), (9, 3)])
+@pytest.mark.parametrize("memory", ["bshd", "bhsd", "sbhd"])
+def test_items_of_two_heads(gpu, dtype, heads, kv_heads, memory):
+    """Interleaved rows on 16-byte vectors take two heads per item: odd head counts leave an item
+    with one, and the heads lie at any stride order of the memory."""
+
+    b, s, d = 2, 5, 32
+    order = {"bshd": (0, 2, 1, 3), "bhsd": (0, 1, 2, 3), "sbhd": (1, 2, 0, 3)}[memory]  # (b, h, s, d) from memory
+
+    def make(h, seed):
+        sizes = {"bshd": (b, s, h, d), "bhsd": (b, h, s, d), "sbhd": (s, b, h, d)}[memory]
+        return randn(sizes, dtype, gpu, seed).permute(*order)
+
+    q, k = make(heads, 1), make(kv_heads, 2)
+    cos, sin = randn((s, d // 2), torch.float32, gpu, 3), randn((s, d // 2), torch.float32, gpu, 4)
+    for inverse in (False, True):
+        out = ops.rope(q, cos, sin, inverse=inverse, x1=k)
+        for x, y in zip((q, k), out):
+            assert y.shape == x.shape and y.stride() == x.stride()
+            ref = torch.empty(x.shape, dtype=torch.float64, device=gpu)
+            a, c = x.double()[..., 0::2], cos.double()
+            e, sn = x.double()[..., 1::2], sin.double() * (-1 if inverse else 1)
+            ref[..., 0::2], ref[..., 1::2] = a * c - e * sn, a * sn + e * c
+            close(y, ref, dtype)
