@@ -1092,15 +1092,19 @@ __global__ __launch_bounds__(kThreads) void ce_finish_kernel(CeWork* __restrict_
 // (exp(x - lse) - [j == target]) * (grad_output / n_valid), computed in fp32 and rounded to
 // fp16 once (lse from the forward's workspace).  Ignored rows are zero whatever the
 // scalar is (torch's nll_loss backward leaves them 0).
-// The work items are (row, chunk of 1024 vectors or elements); a grid of up to 128 blocks
+// The work items are (row, chunk of the row's vectors), LANES threads each; a grid of up to 128 blocks
 // per CU walks them (a one-shot grid streams no faster and makes the common
-// grad_output == 1 launch several times dearer).  The body moves in 16-byte vectors (4 per
+// grad_output == 1 launch several times dearer).  The body moves in 16-byte vectors (VECS per
 // thread per chunk, loads nontemporal: touched once); rows that do not start on a 128-byte
 // line (!ALIGNED) split off a head of elements up to the line and a tail of fewer than one
 // vector, one element per thread.
-constexpr int kScaleVecs = 4;
+// Vectors per thread of the 256-thread items: fp16's backward, which always computes, two at 6 workgroups per CU rather
+// than four at 3 (as much in flight from more waves): [8192, 50257] 281 -> 266 us, [8192, 128256]
+// 686 -> 658, [16384, 32000] 338 -> 335; the scaling of fp32 and bf16 loses (bf16 16384: 166 -> 176).
+template <typename T>
+constexpr int kScaleVecs = std::is_same<T, _Float16>::value ? 2 : 4;
 
-template <typename T, bool ALIGNED, int LANES>
+template <typename T, bool ALIGNED, int LANES, int VECS>
 __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, int64_t inner,
                                                        int64_t valid_inner, int64_t os,
                                                        int64_t is, int64_t sos, int64_t sis,
@@ -1173,7 +1177,7 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, 
     };
     // The item's chunk of the body through a raw buffer resource sized to the part of the
     // chunk inside the row: loads past it return zeros and stores past it are dropped, so
-    // the code has no branches, all four loads are in flight together and every gradient
+    // the code has no branches, all its loads are in flight together and every gradient
     // is computed before the first store (a load waited for after a store waits for the
     // store too).  Within a row, indexes fit in 32 bits.
     const int cstart = static_cast<int>(c) * chunk_vecs;  // first vector of the chunk
@@ -1187,7 +1191,7 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, 
     // the target's index in the chunk, or -1 when it is not there (ignored, in another
     // chunk, in the head or tail of an unaligned row, or outside the row)
     const int64_t trel64 = tgt - lead - static_cast<int64_t>(cstart) * V;
-    const int trel = (trel64 >= 0 && trel64 < int64_t{LANES} * kScaleVecs * V) ? static_cast<int>(trel64) : -1;
+    const int trel = (trel64 >= 0 && trel64 < int64_t{LANES} * VECS * V) ? static_cast<int>(trel64) : -1;
     const int tid = static_cast<int>(threadIdx.x) % LANES;
     // In a row not on a line, the first item also takes the head elements and the item of
     // the body's last chunk the tail elements (one per thread), so that each end of the row
@@ -1204,13 +1208,13 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, 
       if (has_head && read) head_v = q[tid];
       if (has_tail && read) tail_v = q[tail_j];
     }
-    Vec16<T> in[kScaleVecs];
+    Vec16<T> in[VECS];
 #pragma unroll
-    for (int k = 0; k < kScaleVecs; ++k)
+    for (int k = 0; k < VECS; ++k)
       in[k].raw = __builtin_amdgcn_raw_buffer_load_b128(lbuf, (k * LANES + tid) * 16, 0, kNonTemporal);
-    Vec16<T> out[kScaleVecs];
+    Vec16<T> out[VECS];
 #pragma unroll
-    for (int k = 0; k < kScaleVecs; ++k) {
+    for (int k = 0; k < VECS; ++k) {
 #pragma unroll
       for (int i = 0; i < V; ++i) {
         float y;
@@ -1228,7 +1232,7 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, 
       }
     }
 #pragma unroll
-    for (int k = 0; k < kScaleVecs; ++k)
+    for (int k = 0; k < VECS; ++k)
       __builtin_amdgcn_raw_buffer_store_b128(out[k].raw, sbuf, (k * LANES + tid) * 16, 0, kWriteThrough);
     if constexpr (!ALIGNED) {
       // The value is rounded to fp32 before the conversion, as in the vector path (left
@@ -1467,13 +1471,13 @@ int ce_run(const char* fn, const CeRows& d, int64_t outer, int64_t inner, int64_
   return check_launch(fn);
 }
 
-template <typename T, bool ALIGNED, int LANES>
+template <typename T, bool ALIGNED, int LANES, int VECS>
 void scale_launch_as(const CeRows& d, int64_t rows, const float* grad_output, const CeWork* ws,
                      hipStream_t st) {
   // (row, chunk of the body) items, the chunks of a row equally long; a row's body has at most
   // vocab / VEC vectors whether or not it is aligned.
   constexpr int kGroups = 256 / LANES;
-  constexpr int64_t kMost = LANES * kScaleVecs;  // vectors that an item's lanes hold
+  constexpr int64_t kMost = LANES * VECS;  // vectors that an item's lanes hold
   const int64_t nvec = (d.vocab + Elem<T>::VEC - 1) / Elem<T>::VEC;
   const int64_t chunks = (nvec + kMost - 1) / kMost;
   constexpr int kLineVecs = kLineBytes / 16;
@@ -1484,9 +1488,9 @@ void scale_launch_as(const CeRows& d, int64_t rows, const float* grad_output, co
   // (four 16-byte vectors in flight per thread: [8192, 128256] bf16 761 -> 714 us, vocab
   // 151936 935 -> 846 us); a one-shot grid streams no faster and makes the common
   // grad_output == 1 launch, which returns at once, several times dearer.  fp16 (the deferred
-  // gradient, always computed): one workgroup per item, at most 3 resident per CU, so that no
-  // item's loads wait behind an earlier item's stores in the same wave ([4 x 2049, 128256]
-  // 711 -> 659 us against the walk; 4 per CU 685 us, 2 per CU 791 us).  The grid stays below
+  // gradient, always computed): one workgroup per item, at most 6 resident per CU, so that no
+  // item's loads wait behind an earlier item's stores in the same wave ([4 x 2049, 128256] with
+  // four vectors per thread at 3 per CU: 711 -> 659 us against the walk; 4 per CU 685, 2 per CU 791).  The grid stays below
   // 2^24 workgroups (the walk covers any remainder).  PT_CE_SCALE_BLOCKS_PER_CU,
   // PT_CE_SCALE_OCCUPANCY and PT_CE_DEFER_OCCUPANCY override the three figures.
   constexpr bool kDefer = std::is_same<T, _Float16>::value;
@@ -1495,12 +1499,12 @@ void scale_launch_as(const CeRows& d, int64_t rows, const float* grad_output, co
                                                    : static_cast<int64_t>(num_cus()) * walk_blocks;
   const unsigned grid = static_cast<unsigned>(groups < cap ? groups : cap);
   static const int walk_per_cu = static_cast<int>(env_int("PT_CE_SCALE_OCCUPANCY", 4));
-  static const int defer_per_cu = static_cast<int>(env_int("PT_CE_DEFER_OCCUPANCY", 3));
+  static const int defer_per_cu = static_cast<int>(env_int("PT_CE_DEFER_OCCUPANCY", 6));
   // The limits are for items whose lanes hold all their vectors; shorter items run as many more,
   // so that a CU keeps as much in flight, and one-wave items run unlimited.
   const int full_per_cu = kDefer ? defer_per_cu : walk_per_cu;
   const int per_cu = LANES == 64 ? 0 : static_cast<int>(full_per_cu * kMost / chunk_vecs);
-  const auto kernel = ce_scale_kernel<T, ALIGNED, LANES>;
+  const auto kernel = ce_scale_kernel<T, ALIGNED, LANES, VECS>;
   size_t lds = occupancy_lds(per_cu, 0);
   if (allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds) != PT_OK) lds = 0;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, st, static_cast<T*>(d.logits),
@@ -1509,20 +1513,28 @@ void scale_launch_as(const CeRows& d, int64_t rows, const float* grad_output, co
                      grad_output, ws);
 }
 
+// Rows of up to 128 and 256 vectors take one wave per row (a launch of 16384 fp16 rows of 256
+// vectors: 22 us, 32 in 256-thread items), longer ones 256 threads per chunk.
+template <typename T, bool ALIGNED>
+void scale_launch(const CeRows& d, int64_t rows, const float* grad_output, const CeWork* ws,
+                  hipStream_t st) {
+  const int64_t nvec = (static_cast<int64_t>(d.vocab) + Elem<T>::VEC - 1) / Elem<T>::VEC;
+  if (nvec <= 128) {
+    scale_launch_as<T, ALIGNED, 64, 2>(d, rows, grad_output, ws, st);
+  } else if (nvec <= 256) {
+    scale_launch_as<T, ALIGNED, 64, 4>(d, rows, grad_output, ws, st);
+  } else {
+    scale_launch_as<T, ALIGNED, 256, kScaleVecs<T>>(d, rows, grad_output, ws, st);
+  }
+}
+
 template <typename T>
 void scale_launch(bool aligned, const CeRows& d, int64_t rows, const float* grad_output,
                   const CeWork* ws, hipStream_t st) {
-  const bool one_wave = (static_cast<int64_t>(d.vocab) + Elem<T>::VEC - 1) / Elem<T>::VEC <= 64 * kScaleVecs;
   if (aligned) {
-    if (one_wave) {
-      scale_launch_as<T, true, 64>(d, rows, grad_output, ws, st);
-    } else {
-      scale_launch_as<T, true, 256>(d, rows, grad_output, ws, st);
-    }
-  } else if (one_wave) {
-    scale_launch_as<T, false, 64>(d, rows, grad_output, ws, st);
+    scale_launch<T, true>(d, rows, grad_output, ws, st);
   } else {
-    scale_launch_as<T, false, 256>(d, rows, grad_output, ws, st);
+    scale_launch<T, false>(d, rows, grad_output, ws, st);
   }
 }
 
