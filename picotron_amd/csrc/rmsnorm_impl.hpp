@@ -647,7 +647,14 @@ inline int bwd_vpl_cap_for(int tuned, int64_t cols, int vec) {
 // eight of fp32 (two waves per 4096-wide row either way); measured at [16384, 4096], 4 layers:
 // bf16 0.4628-0.4639 ms per step against 0.4660-0.4684 with two and 0.4747-0.4763 with eight,
 // fp32 0.8769-0.8777 ms against 0.8868-0.8871 with four.
-inline int fwd_vpl_cap_for(int tuned, int vec) { return tuned > 0 ? tuned : 32 / vec; }
+// Aligned fp32 rows of 257-512 vectors hold four per lane of two waves instead of eight of one:
+// [16384, 2048] 46.7 -> 45.1 us, with the residual add (two such rows per lane) 93.0 -> 88.8
+// (the general kernels lose by it: [16384, 1370] 66.0 -> 67.9 with the add).
+inline int fwd_vpl_cap_for(int tuned, int64_t cols, int vec) {
+  if (tuned > 0) return tuned;
+  const int64_t nvec = (cols + vec - 1) / vec;
+  return vec == 4 && nvec > 256 && nvec <= 512 ? 4 : 32 / vec;
+}
 
 inline int64_t env_positive(const char* name, int64_t fallback) {
   const char* v = std::getenv(name);
@@ -709,7 +716,7 @@ inline Shape general_shape(int64_t cols, int vec, bool backward) {
   const int64_t nvec = (cols + vec - 1) / vec;
   if (nvec <= kQuarterVecs) return {pow2_at_least((nvec + 15) / 16), 0};
   Shape s;
-  (void)choose_shape(cols, vec, backward ? bwd_vpl_cap_for(0, cols, vec) : fwd_vpl_cap_for(0, vec), &s);
+  (void)choose_shape(cols, vec, backward ? bwd_vpl_cap_for(0, cols, vec) : 32 / vec, &s);
   return s;
 }
 
