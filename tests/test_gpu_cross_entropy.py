@@ -216,6 +216,36 @@ def test_targets_at_the_splits_of_unaligned_rows(gpu, dtype, vocab):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("vocab", [40, 3000, 40_001])
+@pytest.mark.parametrize("rows", [1, 1025, 8200])
+def test_targets_counted_by_the_finish_block(gpu, dtype, vocab, rows):
+    """A call that writes no gradient counts and checks its targets with the losses (8192 rows are
+    one batch of the block): kept, ignored and out-of-range targets, each row kernel, over a
+    workspace that held other values."""
+
+    if rows * vocab > 40_000_000:
+        rows = 1025
+    logits = randn((rows, vocab), dtype, gpu, rows + vocab, 2.0)
+    g = torch.Generator(device=gpu).manual_seed(vocab)
+    targets = torch.randint(0, vocab, (rows,), generator=g, device=gpu)
+    targets[1::3] = -100
+    ref, _ = o_ce.forward_backward(logits, targets)
+    for _ in range(2):
+        dirty = torch.full((ops._lib.lib().pt_cross_entropy_workspace_bytes(rows),), 255, dtype=torch.uint8, device=gpu)
+        del dirty  # the next workspace of this size holds its bytes
+        loss, ws = ops.cross_entropy(logits, targets, write_grad=dtype == torch.float16)
+        assert abs(loss.item() - ref.item()) <= LOSS_RTOL * abs(ref.item())
+        assert ops.cross_entropy_status(ws) == 0
+        assert float(ws[:4].view(torch.float32)) == int((targets != -100).sum())
+    for bad in (vocab, -1):
+        targets[rows - 1 - (rows - 1) % 3] = bad
+        loss, ws = ops.cross_entropy(logits, targets)
+        assert math.isnan(loss.item()) and ops.cross_entropy_status(ws) == 1
+    loss, ws = ops.cross_entropy(logits, torch.full_like(targets, -100))
+    assert math.isnan(loss.item()) and ops.cross_entropy_status(ws) == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("vectors", [64, 128, 256, 512, 1024, 1536])
 @pytest.mark.parametrize("extra,offset", [(0, 0), (0, 1), (1, 0), (-1, 3)])
 def test_short_rows_at_the_ends_of_their_kernels(gpu, dtype, vectors, extra, offset):
