@@ -9,7 +9,8 @@
 // as it always did.  A nonzero code of the library comes back as an int, for _lib.call to raise.
 //
 // Entry points come in by address (bind), from the library that _lib loaded.  Nothing is kept
-// between calls.  The library call runs without the GIL, as it does through ctypes.
+// between calls.  Allocations and the library call run without the GIL, as they do through torch and
+// ctypes.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -34,10 +35,14 @@ namespace {
 PT_NATIVE_FNS(PT_DECLARE)
 #undef PT_DECLARE
 
-// Releases the GIL for the library call of a scope.
+// Releases the GIL for the output allocations (which may wait for the device, or free cached
+// memory) and the library call of a scope, up to end() or the scope's end.
 struct NoGil {
   PyThreadState* s = PyEval_SaveThread();
-  ~NoGil() { PyEval_RestoreThread(s); }
+  void end() {
+    if (s != nullptr) PyEval_RestoreThread(std::exchange(s, nullptr));
+  }
+  ~NoGil() { end(); }
 };
 
 int code_of(const at::Tensor& t) {
@@ -148,13 +153,13 @@ PT_FN(rmsnorm_fwd, 4)
   Rows r;
   double eps;
   if (!norm_rows(x, w, &r) || !as_f64(a[2], &eps)) return none();
+  void* const stream = as_stream(a[3]);
+  NoGil nogil;
   at::Tensor y = at::empty(x->sizes(), x->options()), rstd = empty_rstd(*x);
-  int rc;
-  {
-    NoGil g;
-    rc = p_pt_rmsnorm_fwd(ptr(*x), r.cols, ptr(*w), ptr(y), r.cols, static_cast<float*>(ptr(rstd)),
-                          r.rows, r.cols, static_cast<float>(eps), r.code, r.wcode, as_stream(a[3]));
-  }
+  const int rc = p_pt_rmsnorm_fwd(ptr(*x), r.cols, ptr(*w), ptr(y), r.cols,
+                                  static_cast<float*>(ptr(rstd)), r.rows, r.cols,
+                                  static_cast<float>(eps), r.code, r.wcode, stream);
+  nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
   return tuple(y, rstd);
 PT_END
@@ -166,6 +171,8 @@ PT_FN(rmsnorm_bwd, 7)
   const bool need_dx = a[4] == Py_True, need_dw = a[5] == Py_True;
   if (!norm_rows(x, w, &r) || !twin(dy, *x) || !norm_rstd(s, *x, r) || (!need_dx && !need_dw))
     return none();
+  void* const stream = as_stream(a[6]);
+  NoGil nogil;
   std::optional<at::Tensor> dx, dw;
   at::Tensor ws;
   size_t bytes = 0;
@@ -175,14 +182,11 @@ PT_FN(rmsnorm_bwd, 7)
     bytes = p_pt_rmsnorm_bwd_workspace_bytes(r.rows, r.cols, r.code);
     ws = at::empty({static_cast<int64_t>(bytes < 16 ? 16 : bytes)}, x->options().dtype(at::kByte));
   }
-  int rc;
-  {
-    NoGil g;
-    rc = p_pt_rmsnorm_bwd(ptr(*dy), r.cols, ptr(*x), r.cols, ptr(*w),
-                          static_cast<const float*>(ptr(*s)), dx ? ptr(*dx) : nullptr, r.cols,
-                          dw ? ptr(*dw) : nullptr, dw ? ptr(ws) : nullptr, bytes, r.rows, r.cols,
-                          r.code, r.wcode, as_stream(a[6]));
-  }
+  const int rc = p_pt_rmsnorm_bwd(ptr(*dy), r.cols, ptr(*x), r.cols, ptr(*w),
+                                  static_cast<const float*>(ptr(*s)), dx ? ptr(*dx) : nullptr,
+                                  r.cols, dw ? ptr(*dw) : nullptr, dw ? ptr(ws) : nullptr, bytes,
+                                  r.rows, r.cols, r.code, r.wcode, stream);
+  nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
   return tuple(dx, dw);
 PT_END
@@ -193,15 +197,15 @@ PT_FN(residual_rmsnorm_fwd, 5)
   Rows r;
   double eps;
   if (!norm_rows(x, w, &r) || !twin(res, *x) || !as_f64(a[3], &eps)) return none();
+  void* const stream = as_stream(a[4]);
+  NoGil nogil;
   at::Tensor h = at::empty(x->sizes(), x->options()), y = at::empty(x->sizes(), x->options());
   at::Tensor rstd = empty_rstd(*x);
-  int rc;
-  {
-    NoGil g;
-    rc = p_pt_residual_rmsnorm_fwd(ptr(*x), r.cols, ptr(*res), r.cols, ptr(*w), ptr(h), r.cols,
-                                   ptr(y), r.cols, static_cast<float*>(ptr(rstd)), r.rows, r.cols,
-                                   static_cast<float>(eps), r.code, r.wcode, as_stream(a[4]));
-  }
+  const int rc = p_pt_residual_rmsnorm_fwd(ptr(*x), r.cols, ptr(*res), r.cols, ptr(*w), ptr(h),
+                                           r.cols, ptr(y), r.cols, static_cast<float*>(ptr(rstd)),
+                                           r.rows, r.cols, static_cast<float>(eps), r.code, r.wcode,
+                                           stream);
+  nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
   return tuple(h, y, rstd);
 PT_END
@@ -215,6 +219,8 @@ PT_FN(residual_rmsnorm_bwd, 7)
   if (!norm_rows(h, w, &r) || !twin(dy, *h) || !norm_rstd(s, *h, r) ||
       (a[1] != Py_None && !twin(d, *h)))
     return none();
+  void* const stream = as_stream(a[6]);
+  NoGil nogil;
   at::Tensor dh = at::empty(h->sizes(), h->options());
   std::optional<at::Tensor> dw;
   at::Tensor ws;
@@ -224,15 +230,12 @@ PT_FN(residual_rmsnorm_bwd, 7)
     bytes = p_pt_rmsnorm_bwd_workspace_bytes(r.rows, r.cols, r.code);
     ws = at::empty({static_cast<int64_t>(bytes < 16 ? 16 : bytes)}, h->options().dtype(at::kByte));
   }
-  int rc;
-  {
-    NoGil g;
-    rc = p_pt_residual_rmsnorm_bwd(ptr(*dy), r.cols, d ? ptr(*d) : nullptr, d ? r.cols : 0,
-                                   ptr(*h), r.cols, ptr(*w), static_cast<const float*>(ptr(*s)),
-                                   ptr(dh), r.cols, dw ? ptr(*dw) : nullptr,
-                                   dw ? ptr(ws) : nullptr, bytes, r.rows, r.cols, r.code, r.wcode,
-                                   as_stream(a[6]));
-  }
+  const int rc = p_pt_residual_rmsnorm_bwd(ptr(*dy), r.cols, d ? ptr(*d) : nullptr, d ? r.cols : 0,
+                                           ptr(*h), r.cols, ptr(*w),
+                                           static_cast<const float*>(ptr(*s)), ptr(dh), r.cols,
+                                           dw ? ptr(*dw) : nullptr, dw ? ptr(ws) : nullptr, bytes,
+                                           r.rows, r.cols, r.code, r.wcode, stream);
+  nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
   return tuple(dh, dw);
 PT_END
@@ -243,12 +246,11 @@ PT_END
 PT_FN(swiglu_fwd, 3)
   const at::Tensor *g = plain(a[0]), *u = plain(a[1]);
   if (g == nullptr || !g->is_contiguous() || code_of(*g) < 0 || !twin(u, *g)) return none();
+  void* const stream = as_stream(a[2]);
+  NoGil nogil;
   at::Tensor o = at::empty(g->sizes(), g->options());
-  int rc;
-  {
-    NoGil gil;
-    rc = p_pt_swiglu_fwd(ptr(*g), ptr(*u), ptr(o), g->numel(), code_of(*g), as_stream(a[2]));
-  }
+  const int rc = p_pt_swiglu_fwd(ptr(*g), ptr(*u), ptr(o), g->numel(), code_of(*g), stream);
+  nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
   return wrap(o);
 PT_END
@@ -258,15 +260,14 @@ PT_FN(swiglu_bwd, 6)
   const at::Tensor *d = plain(a[0]), *g = plain(a[1]), *u = plain(a[2]);
   if (g == nullptr || !g->is_contiguous() || code_of(*g) < 0 || !twin(u, *g) || !twin(d, *g))
     return none();
+  void* const stream = as_stream(a[5]);
+  NoGil nogil;
   std::optional<at::Tensor> dg, du;
   if (a[3] == Py_True) dg = at::empty(g->sizes(), g->options());
   if (a[4] == Py_True) du = at::empty(g->sizes(), g->options());
-  int rc;
-  {
-    NoGil gil;
-    rc = p_pt_swiglu_bwd(ptr(*d), ptr(*g), ptr(*u), dg ? ptr(*dg) : nullptr,
-                         du ? ptr(*du) : nullptr, g->numel(), code_of(*g), as_stream(a[5]));
-  }
+  const int rc = p_pt_swiglu_bwd(ptr(*d), ptr(*g), ptr(*u), dg ? ptr(*dg) : nullptr,
+                                 du ? ptr(*du) : nullptr, g->numel(), code_of(*g), stream);
+  nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
   return tuple(dg, du);
 PT_END
@@ -297,6 +298,8 @@ PT_FN(rope, 7)
       c->scalar_type() != at::kFloat || s->scalar_type() != at::kFloat || !c->is_contiguous() ||
       !s->is_contiguous() || !same_place(*c, *x0) || !same_place(*s, *x0) || !as_i64(a[4], &layout))
     return none();
+  void* const stream = as_stream(a[6]);
+  NoGil nogil;
   // empty_like keeps a dense input's stride order
   at::Tensor y0 = at::empty_like(*x0);
   std::optional<at::Tensor> y1;
@@ -304,14 +307,11 @@ PT_FN(rope, 7)
   int64_t d0[9], d1[9];
   rope_desc(*x0, y0, d0);
   if (x1 != nullptr) rope_desc(*x1, *y1, d1);
-  int rc;
-  {
-    NoGil g;
-    rc = p_pt_rope(ptr(*x0), ptr(y0), d0, x1 ? ptr(*x1) : nullptr, x1 ? ptr(*y1) : nullptr,
-                   x1 ? d1 : nullptr, x0->size(3), static_cast<const float*>(ptr(*c)),
-                   static_cast<const float*>(ptr(*s)), c->size(0), static_cast<int>(layout),
-                   a[5] == Py_True ? 1 : 0, code_of(*x0), as_stream(a[6]));
-  }
+  const int rc = p_pt_rope(ptr(*x0), ptr(y0), d0, x1 ? ptr(*x1) : nullptr, x1 ? ptr(*y1) : nullptr,
+                           x1 ? d1 : nullptr, x0->size(3), static_cast<const float*>(ptr(*c)),
+                           static_cast<const float*>(ptr(*s)), c->size(0), static_cast<int>(layout),
+                           a[5] == Py_True ? 1 : 0, code_of(*x0), stream);
+  nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
   return tuple(y0, y1);
 PT_END
@@ -407,7 +407,10 @@ PT_FN(ce_grad_buffer, 2)
   if (!rows_disjoint(x->size(0), x->stride(0), other < 0 ? 1 : x->size(other),
                      other < 0 ? 0 : x->stride(other), x->size(dim)))
     return none();
-  return wrap(grad_buffer(*x));
+  NoGil nogil;
+  const at::Tensor buffer = grad_buffer(*x);
+  nogil.end();
+  return wrap(buffer);
 PT_END
 
 // (logits, targets, ignore_index, write_grad, grad or None, shift, stream) -> (loss, workspace)
@@ -428,17 +431,16 @@ PT_FN(cross_entropy, 7)
   }
   if (write && !rows_disjoint(c.outer, grad ? gos : c.os, c.inner, grad ? gis : c.is, c.vocab))
     return none();
+  void* const stream = as_stream(a[6]);
+  NoGil nogil;
   const size_t bytes = p_pt_cross_entropy_workspace_bytes(c.outer * c.inner);
   at::Tensor ws = at::empty({static_cast<int64_t>(bytes)}, x->options().dtype(at::kByte));
   at::Tensor loss = at::empty({}, x->options().dtype(at::kFloat));
   const auto fn = shift != 0 ? p_pt_cross_entropy_shifted : p_pt_cross_entropy;
-  int rc;
-  {
-    NoGil g;
-    rc = fn(ptr(*x), c.outer, c.inner, c.os, c.is, c.vocab, c.targets, c.tos, c.tis, ignore,
-            static_cast<float*>(ptr(loss)), write ? 1 : 0, grad ? ptr(*grad) : nullptr, gos, gis,
-            ptr(ws), bytes, c.code, as_stream(a[6]));
-  }
+  const int rc = fn(ptr(*x), c.outer, c.inner, c.os, c.is, c.vocab, c.targets, c.tos, c.tis, ignore,
+                    static_cast<float*>(ptr(loss)), write ? 1 : 0, grad ? ptr(*grad) : nullptr, gos,
+                    gis, ptr(ws), bytes, c.code, stream);
+  nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
   return tuple(loss, ws);
 PT_END
@@ -463,14 +465,13 @@ PT_FN(cross_entropy_scale_grad, 8)
     los = src->stride(0);
     if (x->dim() == 3) lis = src->stride(3 - c.class_dim);
   }
+  void* const stream = as_stream(a[7]);
+  NoGil nogil;
   const auto fn = shift != 0 ? p_pt_cross_entropy_shifted_scale_grad : p_pt_cross_entropy_scale_grad;
-  int rc;
-  {
-    NoGil g;
-    rc = fn(ptr(*x), c.outer, c.inner, c.os, c.is, c.vocab, c.targets, c.tos, c.tis, ignore,
-            static_cast<const float*>(ptr(*go)), src ? ptr(*src) : nullptr, los, lis,
-            ws ? ptr(*ws) : nullptr, c.code, as_stream(a[7]));
-  }
+  const int rc = fn(ptr(*x), c.outer, c.inner, c.os, c.is, c.vocab, c.targets, c.tos, c.tis, ignore,
+                    static_cast<const float*>(ptr(*go)), src ? ptr(*src) : nullptr, los, lis,
+                    ws ? ptr(*ws) : nullptr, c.code, stream);
+  nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
   Py_RETURN_TRUE;
 PT_END
