@@ -3,8 +3,9 @@
 Every ``*.hip`` translation unit is compiled by ``hipcc`` in parallel and linked into one
 shared library next to this file (in-tree, so it travels with the source tree), and
 ``native.cpp`` (the launchers for torch tensors, host code against the installed torch) by the
-C++ compiler into ``_native.so`` beside it.  The build always recompiles; nothing is cached
-between calls.
+C++ compiler into ``_native.so`` beside it.  The library needs hipcc alone: where torch, its or
+Python's headers or a C++ compiler are missing, the launchers are left out with a note, and calls on
+tensors go through ctypes.  The build always recompiles; nothing is cached between calls.
 
 Usage: ``python -m picotron_amd.build [-j N] [-v]``.
 """
@@ -71,18 +72,28 @@ def sources() -> list[Path]:
     return sorted(CSRC_DIR.glob("*.hip"))
 
 
+class LaunchersNotBuildable(RuntimeError):
+    """Something that the native launchers are compiled with is not installed."""
+
+
 def build_native() -> Path:
     """Compile the native launchers against the installed torch; returns the extension's path."""
 
     import sysconfig
 
-    import torch
-    from torch.utils.cpp_extension import include_paths, library_paths
+    try:
+        import torch
+        from torch.utils.cpp_extension import include_paths, library_paths
+    except ImportError as error:
+        raise LaunchersNotBuildable(f"torch cannot be imported ({error})") from error
 
     cxx = os.environ.get("CXX") or shutil.which("g++") or shutil.which("c++")
     if not cxx:
-        raise RuntimeError("no C++ compiler found (set CXX)")
+        raise LaunchersNotBuildable("no C++ compiler found (set CXX)")
     includes = [*include_paths(), sysconfig.get_paths()["include"]]
+    for header in ("torch/extension.h", "Python.h"):
+        if not any((Path(path) / header).exists() for path in includes):
+            raise LaunchersNotBuildable(f"{header} not found")
     tmp = NATIVE_PATH.with_suffix(".so.tmp")
     _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
@@ -93,7 +104,8 @@ def build_native() -> Path:
 
 
 def build(jobs: int | None = None, verbose: bool = False) -> Path:
-    """Compile every HIP source and link the shared library; returns its path."""
+    """Compile every HIP source and link the shared library, and compile the launchers where that
+    is possible; returns the library's path."""
 
     hipcc = _hipcc()
     BUILD_DIR.mkdir(exist_ok=True)
@@ -114,20 +126,32 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
             objects.append(obj)
             if verbose and log.strip():
                 print(log, file=sys.stderr)
-        native.result()
-
-    tmp = LIB_PATH.with_suffix(".so.tmp")
-    _run([hipcc, f"--offload-arch={OFFLOAD_ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(tmp)])
-    os.replace(tmp, LIB_PATH)
+        tmp = LIB_PATH.with_suffix(".so.tmp")
+        _run([hipcc, f"--offload-arch={OFFLOAD_ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(tmp)])
+        os.replace(tmp, LIB_PATH)
+        _finish_native(native.result)
     return LIB_PATH
 
 
-def ensure_built() -> Path:
-    """The in-tree library, built first when it or its launchers are not there.  An existing library is used
-    as it is: after changing a source, call :func:`build`."""
+def _finish_native(compile_native) -> None:
+    """Runs (or waits for) the launchers' compilation; a note, and no extension of an earlier build
+    left beside a newer library, where they cannot be built here."""
 
-    if not LIB_PATH.exists() or not NATIVE_PATH.exists():
+    try:
+        compile_native()
+    except LaunchersNotBuildable as error:
+        NATIVE_PATH.unlink(missing_ok=True)
+        print(f"{NATIVE_PATH.name} not built: {error}", file=sys.stderr)
+
+
+def ensure_built() -> Path:
+    """The in-tree library, built first when it or its launchers are not there.  What is there is
+    used as it is: after changing a source, call :func:`build`."""
+
+    if not LIB_PATH.exists():
         build()
+    elif not NATIVE_PATH.exists():
+        _finish_native(build_native)
     return LIB_PATH
 
 
