@@ -2,8 +2,10 @@
 raw arguments, and the ``_native`` extension (``csrc/native.cpp``) for whole calls on tensors.
 
 The library is loaded lazily, once per process.  Loading fails loudly with
-:class:`HipLibraryUnavailable` (never a silent fallback) when the shared object or the
-extension is missing, was built for another ABI version, or cannot be opened.
+:class:`HipLibraryUnavailable` (never a silent fallback) when the shared object is missing, was
+built for another ABI version, or cannot be opened.  The extension only saves host time: every call
+has a ctypes route to the same kernels, taken with a warning when the extension is missing or cannot
+be loaded.  This module needs no torch (the extension is bound once torch is there).
 """
 
 from __future__ import annotations
@@ -11,11 +13,11 @@ from __future__ import annotations
 import ctypes
 import importlib
 import os
+import sys
 import threading
+import warnings
 from ctypes import c_double, c_float, c_int, c_int64, c_size_t, c_void_p
 from pathlib import Path
-
-from torch import Tensor
 
 LIB_PATH = Path(os.environ.get("PICOTRON_HIP_LIB", Path(__file__).with_name("libpicotron_hip.so")))
 
@@ -150,9 +152,10 @@ class HipKernelError(RuntimeError):
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
-# entry point -> native launcher taking tensors; filled when the library loads
+# entry point -> native launcher taking tensors; filled with the extension
 _launchers: dict[str, object] = {}
-native = None  # the extension module
+native = None  # the extension module, or None: every call goes through ctypes
+_native_tried = False
 _load_error: str | None = None
 
 
@@ -185,23 +188,30 @@ def _load() -> ctypes.CDLL:
         if version != ABI_VERSION:
             _load_error = f"{LIB_PATH} has ABI version {version}, expected {ABI_VERSION}; rebuild it"
             raise HipLibraryUnavailable(_load_error)
-        try:
+        if sys.modules.get("torch") is not None:
             _bind_native(lib)
-        except ImportError as error:
-            _load_error = (f"the native launchers cannot be loaded ({error}); build them with "
-                           "`python -m picotron_amd.build`")
-            raise HipLibraryUnavailable(_load_error) from error
         _lib = lib
         return lib
 
 
 def _bind_native(lib: ctypes.CDLL) -> None:
-    """Gives the extension the addresses of ``lib``'s entry points."""
+    """Loads the extension, once, and gives it the addresses of ``lib``'s entry points.  Called
+    with the lock held."""
 
-    global native
-    native = importlib.import_module("picotron_amd._native")
-    for name in native.ENTRY_POINTS:
-        native.bind(name, ctypes.cast(getattr(lib, name), c_void_p).value)
+    global native, _native_tried
+    if _native_tried:
+        return
+    _native_tried = True
+    try:
+        found = importlib.import_module("picotron_amd._native")
+    except ImportError as error:
+        warnings.warn(f"the native launchers cannot be loaded ({error}); calls go through ctypes, with "
+                      "more host time each (build them with `python -m picotron_amd.build`)",
+                      RuntimeWarning, stacklevel=2)
+        return
+    for name in found.ENTRY_POINTS:
+        found.bind(name, ctypes.cast(getattr(lib, name), c_void_p).value)
+    native = found
     _launchers.update(
         pt_rmsnorm_fwd=native.rmsnorm_fwd,
         pt_rmsnorm_bwd=native.rmsnorm_bwd,
@@ -264,18 +274,30 @@ def raw_call(fn: str, *args) -> None:
         check(fn, rc)
 
 
+def _load_launcher(fn: str):
+    """The native launcher of ``fn``, loading the library (or raising) and the extension; None when
+    the extension cannot be loaded."""
+
+    loaded = lib()
+    if not _native_tried:
+        with _lock:
+            _bind_native(loaded)
+    return _launchers.get(fn)
+
+
 def call(fn: str, *args):
     """One launch of entry point ``fn``: with raw arguments (integers, addresses) through ctypes;
     with tensors through its native launcher, which checks them, allocates the outputs and
-    returns them -- or returns None when they are not the plain case that it takes, and the
-    caller goes its general route to :func:`raw_call`."""
+    returns them -- or returns None when they are not the plain case that it takes or there is
+    no launcher, and the caller goes its general route to :func:`raw_call`."""
 
-    if not isinstance(args[0], Tensor):
+    if not hasattr(args[0], "data_ptr"):
         return raw_call(fn, *args)
     launcher = _launchers.get(fn)
     if launcher is None:
-        lib()  # loads the library and fills the table (or raises)
-        launcher = _launchers[fn]
+        launcher = _load_launcher(fn)
+        if launcher is None:
+            return None
     out = launcher(*args)
     if type(out) is int:
         check(fn, out)

@@ -192,7 +192,7 @@ def _scan(optimizer: Optimizer) -> _Scan | None:
     within a group.  None for anything else, which then goes through those two and their checks.
     147 tensors take 60 us of host time this way, 640 through Python."""
 
-    if not isinstance(optimizer, torch.optim.AdamW) or not _lib.is_available():
+    if not isinstance(optimizer, torch.optim.AdamW) or not _lib.is_available() or _lib.native is None:
         return None
     groups = optimizer.param_groups
     for group in groups:

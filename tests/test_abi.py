@@ -5,6 +5,8 @@ from __future__ import annotations
 
 import ctypes
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -164,3 +166,29 @@ def test_last_error_is_per_thread():
     assert seen["a_rc"] == _lib.PT_EINVAL and seen["a_msg"].startswith("pt_swiglu_fwd")
     assert seen["b_fail"] == _lib.PT_EINVAL and seen["b_fail_msg"].startswith("pt_copy")
     assert seen["b_ok"] == _lib.PT_OK and seen["b_msg"] == ""
+
+
+def _child(code: str) -> None:
+    proc = subprocess.run([sys.executable, "-W", "error", "-c", f"import sys; sys.path.insert(0, {str(ROOT)!r})\n{code}"],
+                          capture_output=True, text=True, timeout=100)
+    assert proc.returncode == 0, proc.stdout + proc.stderr
+
+
+def test_binding_needs_no_torch():
+    _child("sys.modules['torch'] = None\n"
+           "from picotron_amd import _lib\n"
+           "assert _lib.lib().pt_abi_version() == _lib.ABI_VERSION and _lib.native is None")
+
+
+def test_library_loads_without_the_extension():
+    """A missing extension costs host time and a warning, not the kernels."""
+
+    _child("import warnings, torch\n"
+           "sys.modules['picotron_amd._native'] = None\n"
+           "from picotron_amd import _lib\n"
+           "with warnings.catch_warnings(record=True) as caught:\n"
+           "    warnings.simplefilter('always')\n"
+           "    assert _lib.is_available() and _lib.unavailable_reason() is None\n"
+           "    assert _lib.call('pt_swiglu_fwd', torch.zeros(1), torch.zeros(1), 0) is None\n"
+           "assert [str(w.message)[:20] for w in caught] == ['the native launchers']\n"
+           "assert _lib.native is None and _lib.lib().pt_adamw_block_elems() == 1024")

@@ -272,3 +272,25 @@ def test_a_refused_launch_raises(gpu):
     x = torch.zeros((1, 1 << 22), device=gpu)
     with pytest.raises(_lib.HipKernelError):
         ops.rmsnorm_fwd(x, torch.ones(1 << 22, device=gpu), 1e-5)
+
+
+def test_without_the_extension(gpu, monkeypatch):
+    """Every call has its ctypes route when the extension could not be loaded."""
+
+    x, w = randn((6, 40), torch.float32, gpu, 1), randn((40,), torch.float32, gpu, 2, 0.1, 1.0)
+    t = torch.arange(6, device=gpu)
+
+    def results():
+        logits = x.clone().requires_grad_(True)
+        loss = triton_cross_entropy(logits, t, inplace=False)
+        params, opt = _optimizer(gpu, 5)
+        for p in params[:-1]:
+            p.grad = torch.ones_like(p)
+        triton_adamw_step(opt)
+        return (*ops.rmsnorm_fwd(x, w, 1e-5), ops.swiglu_fwd(x, x), loss, torch.autograd.grad(loss, logits)[0],
+                triton_clip_grad_norm_and_step(opt, 0.1), *params)
+
+    with_it = results()
+    monkeypatch.setattr(_lib, "native", None)
+    monkeypatch.setattr(_lib, "_launchers", {})
+    _same(results(), with_it)
