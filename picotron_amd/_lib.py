@@ -2,8 +2,8 @@
 raw arguments, and the ``_native`` extension (``csrc/native.cpp``) for whole calls on tensors.
 
 The library is loaded lazily, once per process.  Loading fails loudly with
-:class:`HipLibraryUnavailable` (never a silent fallback) when the shared object is missing, was
-built for another ABI version, or cannot be opened.  The extension only saves host time: every call
+:class:`HipLibraryUnavailable` (never a silent fallback) when the shared object is missing or
+cannot be opened, or when it or the extension was built for another ABI version.  The extension only saves host time: every call
 has a ctypes route to the same kernels, taken with a warning when the extension is missing or cannot
 be loaded.  This module needs no torch (the extension is bound once torch is there).
 """
@@ -189,7 +189,11 @@ def _load() -> ctypes.CDLL:
             _load_error = f"{LIB_PATH} has ABI version {version}, expected {ABI_VERSION}; rebuild it"
             raise HipLibraryUnavailable(_load_error)
         if sys.modules.get("torch") is not None:
-            _bind_native(lib)
+            try:
+                _bind_native(lib)
+            except HipLibraryUnavailable as error:
+                _load_error = str(error)
+                raise
         _lib = lib
         return lib
 
@@ -201,14 +205,18 @@ def _bind_native(lib: ctypes.CDLL) -> None:
     global native, _native_tried
     if _native_tried:
         return
-    _native_tried = True
     try:
         found = importlib.import_module("picotron_amd._native")
     except ImportError as error:
         warnings.warn(f"the native launchers cannot be loaded ({error}); calls go through ctypes, with "
                       "more host time each (build them with `python -m picotron_amd.build`)",
                       RuntimeWarning, stacklevel=2)
+        _native_tried = True
         return
+    # bind() casts addresses to the prototypes of the header that the extension was compiled with
+    version = getattr(found, "PT_ABI_VERSION", None)
+    if version != ABI_VERSION:
+        raise HipLibraryUnavailable(f"{found.__file__} has ABI version {version}, expected {ABI_VERSION}; rebuild it")
     for name in found.ENTRY_POINTS:
         found.bind(name, ctypes.cast(getattr(lib, name), c_void_p).value)
     native = found
@@ -225,6 +233,7 @@ def _bind_native(lib: ctypes.CDLL) -> None:
         pt_cross_entropy_scale_grad=native.cross_entropy_scale_grad,
         pt_cross_entropy_shifted_scale_grad=native.cross_entropy_scale_grad,
     )
+    _native_tried = True
 
 
 def lib() -> ctypes.CDLL:

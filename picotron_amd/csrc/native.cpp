@@ -650,5 +650,6 @@ PyMODINIT_FUNC PyInit__native() {
     Py_DECREF(s);
   }
   PyModule_AddObject(m, "ENTRY_POINTS", list);
+  PyModule_AddIntMacro(m, PT_ABI_VERSION);  // of the prototypes that bind() casts to
   return m;
 }

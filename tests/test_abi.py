@@ -192,3 +192,16 @@ def test_library_loads_without_the_extension():
            "    assert _lib.call('pt_swiglu_fwd', torch.zeros(1), torch.zeros(1), 0) is None\n"
            "assert [str(w.message)[:20] for w in caught] == ['the native launchers']\n"
            "assert _lib.native is None and _lib.lib().pt_adamw_block_elems() == 1024")
+
+
+def test_extension_of_another_abi_version_is_refused():
+    """Its launchers would call the library's entry points with the arguments of another header."""
+
+    _child("import torch\n"
+           "from picotron_amd import _native, _lib\n"
+           "assert _native.PT_ABI_VERSION == _lib.ABI_VERSION\n"
+           "_native.PT_ABI_VERSION -= 1\n"
+           "_native.bind = None  # nothing may be bound\n"
+           "for _ in range(2):\n"
+           "    assert not _lib.is_available() and 'ABI version 3, expected 4' in _lib.unavailable_reason()\n"
+           "assert _lib.native is None and not _lib._launchers")
