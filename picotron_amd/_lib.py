@@ -207,6 +207,10 @@ def _bind_native(lib: ctypes.CDLL) -> None:
         return
     try:
         found = importlib.import_module("picotron_amd._native")
+        # the layout of torch's C++ objects is that of the version it was compiled against
+        built, here = getattr(found, "TORCH_VERSION", None), str(sys.modules["torch"].__version__)
+        if built is not None and built != here:
+            raise ImportError(f"compiled against torch {built}, running under {here}")
     except ImportError as error:
         warnings.warn(f"the native launchers cannot be loaded ({error}); calls go through ctypes, with "
                       "more host time each (build them with `python -m picotron_amd.build`)",

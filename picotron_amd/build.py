@@ -97,6 +97,7 @@ def build_native() -> Path:
     tmp = NATIVE_PATH.with_suffix(".so.tmp")
     _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          f'-DPT_TORCH_VERSION="{torch.__version__}"',
           *(arg for path in includes for arg in ("-isystem", path)), str(NATIVE_SOURCE), "-o", str(tmp),
           *(f"-L{path}" for path in library_paths()), "-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python"])
     os.replace(tmp, NATIVE_PATH)

@@ -651,5 +651,6 @@ PyMODINIT_FUNC PyInit__native() {
   }
   PyModule_AddObject(m, "ENTRY_POINTS", list);
   PyModule_AddIntMacro(m, PT_ABI_VERSION);  // of the prototypes that bind() casts to
+  PyModule_AddStringConstant(m, "TORCH_VERSION", PT_TORCH_VERSION);
   return m;
 }

@@ -205,3 +205,17 @@ def test_extension_of_another_abi_version_is_refused():
            "for _ in range(2):\n"
            "    assert not _lib.is_available() and 'ABI version 3, expected 4' in _lib.unavailable_reason()\n"
            "assert _lib.native is None and not _lib._launchers")
+
+
+def test_extension_of_another_torch_is_not_used():
+    """torch's C++ objects have no fixed layout between versions: such an extension counts as one
+    that cannot be loaded."""
+
+    _child("import warnings, torch\n"
+           "from picotron_amd import _native, _lib\n"
+           "assert _native.TORCH_VERSION == str(torch.__version__)\n"
+           "_native.TORCH_VERSION = '1.0'\n"
+           "with warnings.catch_warnings(record=True) as caught:\n"
+           "    warnings.simplefilter('always')\n"
+           "    assert _lib.is_available()\n"
+           "assert 'compiled against torch 1.0' in str(caught[0].message) and _lib.native is None")
