@@ -287,15 +287,15 @@ def raw_call(fn: str, *args) -> None:
         check(fn, rc)
 
 
-def _load_launcher(fn: str):
-    """The native launcher of ``fn``, loading the library (or raising) and the extension; None when
-    the extension cannot be loaded."""
+def extension():
+    """The extension module, loading the library (or raising) and binding the extension when neither
+    has happened yet; None when it cannot be loaded."""
 
-    loaded = lib()
     if not _native_tried:
+        loaded = lib()
         with _lock:
             _bind_native(loaded)
-    return _launchers.get(fn)
+    return native
 
 
 def call(fn: str, *args):
@@ -308,9 +308,9 @@ def call(fn: str, *args):
         return raw_call(fn, *args)
     launcher = _launchers.get(fn)
     if launcher is None:
-        launcher = _load_launcher(fn)
-        if launcher is None:
+        if extension() is None:
             return None
+        launcher = _launchers[fn]
     out = launcher(*args)
     if type(out) is int:
         check(fn, out)

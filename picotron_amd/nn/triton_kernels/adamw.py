@@ -192,14 +192,17 @@ def _scan(optimizer: Optimizer) -> _Scan | None:
     within a group.  None for anything else, which then goes through those two and their checks.
     147 tensors take 60 us of host time this way, 640 through Python."""
 
-    if not isinstance(optimizer, torch.optim.AdamW) or not _lib.is_available() or _lib.native is None:
+    if not isinstance(optimizer, torch.optim.AdamW) or not _lib.is_available():
+        return None
+    native = _lib.extension()
+    if native is None:
         return None
     groups = optimizer.param_groups
     for group in groups:
         _check_group(group)
         if group.get("capturable", False):
             return None
-    found = _lib.native.adamw_scan([group["params"] for group in groups], optimizer.state,
+    found = native.adamw_scan([group["params"] for group in groups], optimizer.state,
                                    ops._adamw_block_elems())
     if found is None:
         return None

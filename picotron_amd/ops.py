@@ -440,8 +440,9 @@ def ce_grad_buffer(logits: Tensor, class_dim: int = 1) -> Tensor | None:
     dimension, 1 for (N, C) and (N, C, d) inputs, 2 for the shifted (B, S, V) form.  None when
     the logits rows overlap in memory (an expanded tensor)."""
 
-    if logits.is_cuda and not _compiling() and _lib.is_available() and _lib.native is not None:
-        buffer = _lib.native.ce_grad_buffer(logits, class_dim)
+    native = _lib.extension() if logits.is_cuda and not _compiling() and _lib.is_available() else None
+    if native is not None:
+        buffer = native.ce_grad_buffer(logits, class_dim)
         if buffer is not None:
             return buffer
     dims = list(zip(logits.shape, logits.stride()))

@@ -219,3 +219,11 @@ def test_extension_of_another_torch_is_not_used():
            "    warnings.simplefilter('always')\n"
            "    assert _lib.is_available()\n"
            "assert 'compiled against torch 1.0' in str(caught[0].message) and _lib.native is None")
+
+
+def test_extension_is_bound_when_torch_comes_after_the_library():
+    _child("from picotron_amd import _lib\n"
+           "_lib.lib()\n"
+           "assert 'torch' not in sys.modules and _lib.native is None\n"
+           "import torch\n"
+           "assert _lib.extension() is not None and _lib.native is _lib.extension()")
