@@ -73,7 +73,10 @@ bool twin(const at::Tensor* t, const at::Tensor& ref) {
          same_place(*t, ref) && t->sizes() == ref.sizes();
 }
 
-void* ptr(const at::Tensor& t) { return const_cast<void*>(t.const_data_ptr()); }
+// The address of a tensor that a call reads, and of one that it writes (which first gives a lazily
+// cloned tensor a storage of its own, as Tensor.data_ptr() does on the general route).
+const void* in(const at::Tensor& t) { return t.const_data_ptr(); }
+void* out(const at::Tensor& t) { return t.mutable_data_ptr(); }
 
 PyObject* none() { Py_RETURN_NONE; }
 PyObject* wrap(const at::Tensor& t) { return THPVariable_Wrap(t); }
@@ -156,8 +159,8 @@ PT_FN(rmsnorm_fwd, 4)
   void* const stream = as_stream(a[3]);
   NoGil nogil;
   at::Tensor y = at::empty(x->sizes(), x->options()), rstd = empty_rstd(*x);
-  const int rc = p_pt_rmsnorm_fwd(ptr(*x), r.cols, ptr(*w), ptr(y), r.cols,
-                                  static_cast<float*>(ptr(rstd)), r.rows, r.cols,
+  const int rc = p_pt_rmsnorm_fwd(in(*x), r.cols, in(*w), out(y), r.cols,
+                                  static_cast<float*>(out(rstd)), r.rows, r.cols,
                                   static_cast<float>(eps), r.code, r.wcode, stream);
   nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
@@ -182,9 +185,9 @@ PT_FN(rmsnorm_bwd, 7)
     bytes = p_pt_rmsnorm_bwd_workspace_bytes(r.rows, r.cols, r.code);
     ws = at::empty({static_cast<int64_t>(bytes < 16 ? 16 : bytes)}, x->options().dtype(at::kByte));
   }
-  const int rc = p_pt_rmsnorm_bwd(ptr(*dy), r.cols, ptr(*x), r.cols, ptr(*w),
-                                  static_cast<const float*>(ptr(*s)), dx ? ptr(*dx) : nullptr,
-                                  r.cols, dw ? ptr(*dw) : nullptr, dw ? ptr(ws) : nullptr, bytes,
+  const int rc = p_pt_rmsnorm_bwd(in(*dy), r.cols, in(*x), r.cols, in(*w),
+                                  static_cast<const float*>(in(*s)), dx ? out(*dx) : nullptr,
+                                  r.cols, dw ? out(*dw) : nullptr, dw ? out(ws) : nullptr, bytes,
                                   r.rows, r.cols, r.code, r.wcode, stream);
   nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
@@ -201,8 +204,8 @@ PT_FN(residual_rmsnorm_fwd, 5)
   NoGil nogil;
   at::Tensor h = at::empty(x->sizes(), x->options()), y = at::empty(x->sizes(), x->options());
   at::Tensor rstd = empty_rstd(*x);
-  const int rc = p_pt_residual_rmsnorm_fwd(ptr(*x), r.cols, ptr(*res), r.cols, ptr(*w), ptr(h),
-                                           r.cols, ptr(y), r.cols, static_cast<float*>(ptr(rstd)),
+  const int rc = p_pt_residual_rmsnorm_fwd(in(*x), r.cols, in(*res), r.cols, in(*w), out(h),
+                                           r.cols, out(y), r.cols, static_cast<float*>(out(rstd)),
                                            r.rows, r.cols, static_cast<float>(eps), r.code, r.wcode,
                                            stream);
   nogil.end();
@@ -230,10 +233,10 @@ PT_FN(residual_rmsnorm_bwd, 7)
     bytes = p_pt_rmsnorm_bwd_workspace_bytes(r.rows, r.cols, r.code);
     ws = at::empty({static_cast<int64_t>(bytes < 16 ? 16 : bytes)}, h->options().dtype(at::kByte));
   }
-  const int rc = p_pt_residual_rmsnorm_bwd(ptr(*dy), r.cols, d ? ptr(*d) : nullptr, d ? r.cols : 0,
-                                           ptr(*h), r.cols, ptr(*w),
-                                           static_cast<const float*>(ptr(*s)), ptr(dh), r.cols,
-                                           dw ? ptr(*dw) : nullptr, dw ? ptr(ws) : nullptr, bytes,
+  const int rc = p_pt_residual_rmsnorm_bwd(in(*dy), r.cols, d ? in(*d) : nullptr, d ? r.cols : 0,
+                                           in(*h), r.cols, in(*w),
+                                           static_cast<const float*>(in(*s)), out(dh), r.cols,
+                                           dw ? out(*dw) : nullptr, dw ? out(ws) : nullptr, bytes,
                                            r.rows, r.cols, r.code, r.wcode, stream);
   nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
@@ -249,7 +252,7 @@ PT_FN(swiglu_fwd, 3)
   void* const stream = as_stream(a[2]);
   NoGil nogil;
   at::Tensor o = at::empty(g->sizes(), g->options());
-  const int rc = p_pt_swiglu_fwd(ptr(*g), ptr(*u), ptr(o), g->numel(), code_of(*g), stream);
+  const int rc = p_pt_swiglu_fwd(in(*g), in(*u), out(o), g->numel(), code_of(*g), stream);
   nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
   return wrap(o);
@@ -265,8 +268,8 @@ PT_FN(swiglu_bwd, 6)
   std::optional<at::Tensor> dg, du;
   if (a[3] == Py_True) dg = at::empty(g->sizes(), g->options());
   if (a[4] == Py_True) du = at::empty(g->sizes(), g->options());
-  const int rc = p_pt_swiglu_bwd(ptr(*d), ptr(*g), ptr(*u), dg ? ptr(*dg) : nullptr,
-                                 du ? ptr(*du) : nullptr, g->numel(), code_of(*g), stream);
+  const int rc = p_pt_swiglu_bwd(in(*d), in(*g), in(*u), dg ? out(*dg) : nullptr,
+                                 du ? out(*du) : nullptr, g->numel(), code_of(*g), stream);
   nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
   return tuple(dg, du);
@@ -307,9 +310,9 @@ PT_FN(rope, 7)
   int64_t d0[9], d1[9];
   rope_desc(*x0, y0, d0);
   if (x1 != nullptr) rope_desc(*x1, *y1, d1);
-  const int rc = p_pt_rope(ptr(*x0), ptr(y0), d0, x1 ? ptr(*x1) : nullptr, x1 ? ptr(*y1) : nullptr,
-                           x1 ? d1 : nullptr, x0->size(3), static_cast<const float*>(ptr(*c)),
-                           static_cast<const float*>(ptr(*s)), c->size(0), static_cast<int>(layout),
+  const int rc = p_pt_rope(in(*x0), out(y0), d0, x1 ? in(*x1) : nullptr, x1 ? out(*y1) : nullptr,
+                           x1 ? d1 : nullptr, x0->size(3), static_cast<const float*>(in(*c)),
+                           static_cast<const float*>(in(*s)), c->size(0), static_cast<int>(layout),
                            a[5] == Py_True ? 1 : 0, code_of(*x0), stream);
   nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
@@ -333,7 +336,7 @@ bool ce_call(const at::Tensor* x, const at::Tensor* t, int64_t shift, CeCall* c)
     return false;
   c->code = code_of(*x);
   if (c->code < 0) return false;
-  c->targets = static_cast<const int64_t*>(ptr(*t));
+  c->targets = static_cast<const int64_t*>(in(*t));
   if (shift != 0) {
     if (x->dim() != 3 || x->stride(2) != 1 || t->dim() != 2 || t->size(0) != x->size(0) ||
         t->size(1) != x->size(1) - (shift == 2 ? 1 : 0))
@@ -392,7 +395,7 @@ at::Tensor grad_buffer(const at::Tensor& x) {
   for (int64_t i = 0; i < x.dim(); ++i) span += (x.size(i) - 1) * x.stride(i);
   const int64_t esize = static_cast<int64_t>(x.element_size());
   at::Tensor flat = at::empty({span + 128 / esize}, x.options());
-  const uintptr_t to = reinterpret_cast<uintptr_t>(ptr(x)), from = reinterpret_cast<uintptr_t>(ptr(flat));
+  const uintptr_t to = reinterpret_cast<uintptr_t>(in(x)), from = reinterpret_cast<uintptr_t>(in(flat));
   return flat.as_strided(x.sizes(), x.strides(), static_cast<int64_t>((to - from) % 128) / esize);
 }
 
@@ -437,9 +440,11 @@ PT_FN(cross_entropy, 7)
   at::Tensor ws = at::empty({static_cast<int64_t>(bytes)}, x->options().dtype(at::kByte));
   at::Tensor loss = at::empty({}, x->options().dtype(at::kFloat));
   const auto fn = shift != 0 ? p_pt_cross_entropy_shifted : p_pt_cross_entropy;
-  const int rc = fn(ptr(*x), c.outer, c.inner, c.os, c.is, c.vocab, c.targets, c.tos, c.tis, ignore,
-                    static_cast<float*>(ptr(loss)), write ? 1 : 0, grad ? ptr(*grad) : nullptr, gos,
-                    gis, ptr(ws), bytes, c.code, stream);
+  // the logits are written only where the gradient goes over them
+  void* const rows = write && grad == nullptr ? out(*x) : const_cast<void*>(in(*x));
+  const int rc = fn(rows, c.outer, c.inner, c.os, c.is, c.vocab, c.targets, c.tos, c.tis, ignore,
+                    static_cast<float*>(out(loss)), write ? 1 : 0, grad ? out(*grad) : nullptr, gos,
+                    gis, out(ws), bytes, c.code, stream);
   nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
   return tuple(loss, ws);
@@ -468,9 +473,9 @@ PT_FN(cross_entropy_scale_grad, 8)
   void* const stream = as_stream(a[7]);
   NoGil nogil;
   const auto fn = shift != 0 ? p_pt_cross_entropy_shifted_scale_grad : p_pt_cross_entropy_scale_grad;
-  const int rc = fn(ptr(*x), c.outer, c.inner, c.os, c.is, c.vocab, c.targets, c.tos, c.tis, ignore,
-                    static_cast<const float*>(ptr(*go)), src ? ptr(*src) : nullptr, los, lis,
-                    ws ? ptr(*ws) : nullptr, c.code, stream);
+  const int rc = fn(out(*x), c.outer, c.inner, c.os, c.is, c.vocab, c.targets, c.tos, c.tis, ignore,
+                    static_cast<const float*>(in(*go)), src ? in(*src) : nullptr, los, lis,
+                    ws ? in(*ws) : nullptr, c.code, stream);
   nogil.end();
   if (rc != PT_OK) return PyLong_FromLong(rc);
   Py_RETURN_TRUE;
@@ -490,7 +495,7 @@ float* host_step(PyObject* o) {
   if (!t.defined() || !t.is_cpu() || t.layout() != at::kStrided || t.scalar_type() != at::kFloat ||
       t.numel() != 1 || !t.has_storage())
     return nullptr;
-  return static_cast<float*>(ptr(t));
+  return static_cast<float*>(out(t));
 }
 
 // A borrowed reference to a dict's item, or null (no exception left).
@@ -550,7 +555,7 @@ PT_FN(adamw_scan, 3)
       g.step = *step;
       g.steps.push_back(so);
       const int64_t n = p->numel(), blocks = (n + per - 1) / per;
-      const auto at = [](const at::Tensor& x) { return reinterpret_cast<int64_t>(ptr(x)); };
+      const auto at = [](const at::Tensor& x) { return reinterpret_cast<int64_t>(out(x)); };
       g.rows.insert(g.rows.end(), {at(*p), at(grad), at(*m), at(*v), n, g.blocks});
       grads.insert(grads.end(), {at(grad), at(grad), at(grad), at(grad), n, all});
       g.blocks += blocks;

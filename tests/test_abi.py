@@ -204,6 +204,10 @@ def test_extension_of_another_abi_version_is_refused():
            "_native.bind = None  # nothing may be bound\n"
            "for _ in range(2):\n"
            "    assert not _lib.is_available() and 'ABI version 3, expected 4' in _lib.unavailable_reason()\n"
+           "try:\n"
+           "    _lib.extension()\n"
+           "except _lib.HipLibraryUnavailable:\n"
+           "    pass\n"
            "assert _lib.native is None and not _lib._launchers")
 
 
@@ -219,6 +223,19 @@ def test_extension_of_another_torch_is_not_used():
            "    warnings.simplefilter('always')\n"
            "    assert _lib.is_available()\n"
            "assert 'compiled against torch 1.0' in str(caught[0].message) and _lib.native is None")
+
+
+def test_advanced_step_counts_leave_a_lazy_clone_alone():
+    """A lazily cloned step tensor shares its storage until it is written: a write through the
+    native pass first gives it its own, as any in-place torch operation does."""
+
+    import torch
+
+    native = _lib.extension()
+    step = torch.tensor(3.0)
+    clone = torch._lazy_clone(step)
+    native.advance_steps([clone])
+    assert float(clone) == 4.0 and float(step) == 3.0
 
 
 def test_extension_is_bound_when_torch_comes_after_the_library():

@@ -294,3 +294,34 @@ def test_without_the_extension(gpu, monkeypatch):
     monkeypatch.setattr(_lib, "native", None)
     monkeypatch.setattr(_lib, "_launchers", {})
     _same(results(), with_it)
+
+
+def test_writes_leave_lazily_cloned_tensors_alone(gpu):
+    """What a call writes gets a storage of its own first (parameters, gradients, moments, step
+    counts, logits and gradient buffers written in place)."""
+
+    logits, t = randn((6, 41), torch.float32, gpu, 1), torch.arange(6, device=gpu)
+    kept = logits.clone()
+    x = torch._lazy_clone(logits)
+    _, ws = ops.cross_entropy(x, t, write_grad=True)
+    assert torch.equal(logits, kept) and not torch.equal(x, kept)
+    scaled = torch._lazy_clone(x)
+    before = x.clone()
+    ops.cross_entropy_scale_grad(scaled, t, torch.full((), 2.0, device=gpu), workspace=ws)
+    assert torch.equal(x, before) and torch.equal(scaled, 2 * before)
+
+    params, opt = _optimizer(gpu, 7)
+    for p in params[:-1]:
+        p.grad = torch.ones_like(p)
+    triton_adamw_step(opt)
+    shared = []
+    for p in params[:-1]:
+        state = opt.state[p]
+        shared += [p.data, p.grad, *state.values()]
+        p.data, p.grad = torch._lazy_clone(p.data), torch._lazy_clone(p.grad)
+        opt.state[p] = {k: torch._lazy_clone(v) for k, v in state.items()}
+    kept = [v.clone() for v in shared]
+    assert adamw._scan(opt) is not None
+    triton_clip_grad_norm_and_step(opt, 0.05)
+    _same(shared, kept)
+    assert float(opt.state[params[0]]["step"]) == 2.0 and not torch.equal(params[0], shared[0])
