@@ -251,8 +251,8 @@ __global__ __launch_bounds__(kThreads) void grad_stats_kernel(const AdamRec* __r
   const float s = inv_scale != nullptr ? *inv_scale : 1.0f;
   float acc = 0.0f;
   bool bad = false;
-  const auto add = [&](float g) {
-    const float x = g * s;
+  const auto add = [&](float g, float scale) {
+    const float x = g * scale;
     acc += x * x;
     bad |= !__builtin_isfinite(g);
   };
@@ -267,12 +267,16 @@ __global__ __launch_bounds__(kThreads) void grad_stats_kernel(const AdamRec* __r
             f32x4, __builtin_amdgcn_raw_buffer_load_b128(
                        buf, base + (u * kThreads + static_cast<int>(threadIdx.x)) * 16, 0, kNonTemporal));
 #pragma unroll
-      for (int u = 0; u < kWalkLoads; ++u)
+      for (int u = 0; u < kWalkLoads; ++u) {
+        // past the run the loads return zeros, which an infinite scale must not meet
+        const int off = base + (u * kThreads + static_cast<int>(threadIdx.x)) * 16;
+        const float scale = off < bytes ? s : 0.0f;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) add(v[u][j]);  // zeros past the run
+        for (int j = 0; j < 4; ++j) add(v[u][j], scale);
+      }
     }
     if (static_cast<int>(threadIdx.x) < tail)
-      add(as_global<float>(g)[static_cast<int64_t>(vectors) * 4 + threadIdx.x]);
+      add(as_global<float>(g)[static_cast<int64_t>(vectors) * 4 + threadIdx.x], s);
   });
   acc = wave_sum(acc);
   const int any_bad = __syncthreads_or(bad ? 1 : 0);

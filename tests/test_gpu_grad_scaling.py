@@ -8,6 +8,7 @@ import torch
 
 from gpu_util import close_fp32, randn
 from oracle import adamw as o_adamw
+from picotron_amd import ops
 from picotron_amd.nn.triton_kernels import (
     triton_unscale_and_check_,
     triton_unscale_clip_and_step,
@@ -46,6 +47,21 @@ def test_unscale_and_check_non_finite_leaves_everything(gpu, bad):
     assert triton_unscale_and_check_(ps, 1024.0) is True
     for p, g in zip(ps, grads):
         assert torch.equal(p.grad.nan_to_num(), g.nan_to_num())
+
+
+@pytest.mark.parametrize("inv_scale", [float("inf"), float("-inf"), 0.0])
+def test_norm_of_finite_gradients_under_an_extreme_scale(gpu, inv_scale):
+    """A loss scale below fp32's range inverts to infinity: the norm of finite, nonzero gradients is
+    then infinite (not NaN) whatever the gradients' sizes are, and the overflow flag stays clear."""
+
+    for n in (1, 4, 5, 1023, 1024, 8192, 8196, 70_001):
+        g = randn((n,), torch.float32, gpu, n, 1e-3)
+        g += torch.where(g == 0, 1.0, 0.0)
+        table, blocks = ops.adamw_table([g], [g], [g], [g])
+        inv = torch.tensor([inv_scale], device=gpu)
+        norm, _, found = ops.grad_stats(table.to(gpu), blocks, inv)
+        assert float(norm) == (0.0 if inv_scale == 0 else float("inf")), n
+        assert int(found) == 0
 
 
 @pytest.mark.parametrize("max_norm", [0.05, 1e4])
