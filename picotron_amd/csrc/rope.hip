@@ -38,8 +38,8 @@ struct RopeTensor {
   int64_t ys[3];   // y strides
   int seq_dim;     // which of the three is the sequence dimension
   int head_dim;    // and which the heads
-  int heads;
-  int chunks;      // items that share a position's heads
+  int64_t heads;
+  int64_t chunks;  // items that share a position's heads
   int64_t xstep;   // elements from one of an item's heads to the next
   int64_t ystep;
   int64_t rows;    // batch * heads * seq
@@ -103,9 +103,11 @@ struct RopeWork {
     if constexpr (ALIGNED) {
       const int64_t xstep = U > 1 ? t.xstep : 0;
       if constexpr (U > 1) {
+        // (a position with whole vectors has fewer than 2^31 heads: pt_rope bounds the pairs by 2^32)
         const int first =
             static_cast<int>(t.head_dim == 0 ? idx[0] : (t.head_dim == 1 ? idx[1] : idx[2]));
-        count = (t.heads - first + t.chunks - 1) / t.chunks;
+        const int heads = static_cast<int>(t.heads), chunks = static_cast<int>(t.chunks);
+        count = (heads - first + chunks - 1) / chunks;
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -253,7 +255,7 @@ bool parse(const void* x, void* y, const int64_t* d, int64_t head_dim, int64_t t
     if (ord[i] == 2) t->seq_dim = i;
     if (ord[i] == 1) t->head_dim = i;
   }
-  t->heads = static_cast<int>(sz[1]);
+  t->heads = sz[1];
   t->rows = sz[0] * sz[1] * sz[2];
   // y's extent in bytes (-1 when a stride is negative): the write-through stores address y
   // through a buffer resource, so they need it to fit 31 bits
@@ -302,7 +304,7 @@ void launch(RopeTensor& t0, RopeTensor& t1, int head_dim, const float* c, const 
   const int per_row = items_per_row<T, LAYOUT, ALIGNED>(head_dim);
   constexpr int kPer = kHeads<LAYOUT, ALIGNED>;
   for (RopeTensor* t : {&t0, &t1}) {
-    t->chunks = static_cast<int>((t->heads + kPer - 1) / kPer);
+    t->chunks = (t->heads + kPer - 1) / kPer;
     t->xstep = t->xs[t->head_dim] * t->chunks;
     t->ystep = t->ys[t->head_dim] * t->chunks;
     t->items = 0;

@@ -92,6 +92,22 @@ def test_rope_at_the_write_through_limit(gpu, s):
         del y
 
 
+def test_rope_past_2_31_heads(gpu):
+    """As many heads as fit the kernel's 2^32 pairs: their count does not fit 31 bits."""
+
+    heads = TWO31 + 24
+    cos, sin = o_rope.tables(2, 2, 500_000.0, device=gpu)
+    x = torch.ones((1, 2 * heads), dtype=torch.bfloat16, device=gpu).view(1, heads, 1, 2)
+    windows = (slice(0, 64), slice(TWO31 - 32, TWO31 + 8), slice(heads - 64, heads))
+    for i, w in enumerate(windows):
+        x[:, w] = _randn(x[:, w].shape, torch.bfloat16, gpu, 40 + i)
+    cos[0], sin[0] = 0.6, 0.8
+    y, _ = ops.rope(x, cos, sin)
+    torch.cuda.synchronize()
+    for w in windows:
+        torch.testing.assert_close(y[:, w].double(), o_rope.rotate(x[:, w], cos, sin, "interleaved"), **BF16)
+
+
 def test_rmsnorm_past_2_31_elements(gpu):
     cols = 4096
     rows = TWO31 // cols + 13  # the last 13 rows start past element 2^31
