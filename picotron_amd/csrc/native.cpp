@@ -13,6 +13,7 @@
 // ctypes.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <ATen/ATen.h>
 
@@ -505,6 +506,12 @@ PyObject* item(PyObject* dict, const char* key) {
   return v;
 }
 
+// A reference of its own to a borrowed object (or null).
+THPObjectPtr owned(PyObject* o) {
+  Py_XINCREF(o);
+  return THPObjectPtr(o);
+}
+
 // scan([params, ...] per group, optimizer.state, elements per block) ->
 // (device index, blocks, gradient table, [(table, rows, blocks, step, steps), ...])
 // for parameters that all have their state in place, with one step count per group: the record
@@ -518,7 +525,7 @@ PT_FN(adamw_scan, 3)
     std::vector<int64_t> rows;
     int64_t blocks = 0;
     float step = 0.0f;
-    std::vector<PyObject*> steps;  // borrowed, from the state
+    THPObjectPtr steps{PyList_New(0)};
   };
   std::vector<Group> groups;
   std::vector<int64_t> grads;
@@ -528,17 +535,22 @@ PT_FN(adamw_scan, 3)
     PyObject* params = PyList_GET_ITEM(a[0], i);
     if (!PyList_Check(params)) return none();
     Group g;
+    if (!g.steps) return nullptr;
     for (Py_ssize_t k = 0; k < PyList_GET_SIZE(params); ++k) {
-      PyObject* o = PyList_GET_ITEM(params, k);
+      // The state's lookup hashes the parameter in Python, where other threads (or a user's code) may
+      // change the lists and the state: what is used afterwards is held by a reference of its own.
+      THPObjectPtr held = owned(PyList_GET_ITEM(params, k));
+      PyObject* o = held.get();
       if (!THPVariable_CheckExact(o)) return none();
-      const at::Tensor& grad = THPVariable_Unpack(o).grad();
+      const at::Tensor grad = THPVariable_Unpack(o).grad();
       if (!grad.defined()) continue;
       const at::Tensor* p = plain_f32(plain(o));
       if (p == nullptr || grad.layout() != at::kStrided || grad.scalar_type() != at::kFloat ||
           !grad.is_contiguous() || !grad.has_storage() || grad.device() != p->device() ||
           grad.numel() != p->numel() || grad.is_neg() || grad.storage().data() == nullptr)
         return none();
-      PyObject* state = PyDict_GetItemWithError(a[1], o);
+      THPObjectPtr entry = owned(PyDict_GetItemWithError(a[1], o));
+      PyObject* state = entry.get();
       if (state == nullptr || !PyDict_Check(state)) {
         PyErr_Clear();
         return none();
@@ -551,9 +563,9 @@ PT_FN(adamw_scan, 3)
           v->device() != p->device() || m->numel() != p->numel() || v->numel() != p->numel())
         return none();
       if (all == 0) device = p->device();
-      if (p->device() != device || (!g.steps.empty() && *step != g.step)) return none();
+      if (p->device() != device || (!g.rows.empty() && *step != g.step)) return none();
       g.step = *step;
-      g.steps.push_back(so);
+      if (PyList_Append(g.steps, so) != 0) return nullptr;
       const int64_t n = p->numel(), blocks = (n + per - 1) / per;
       const auto at = [](const at::Tensor& x) { return reinterpret_cast<int64_t>(out(x)); };
       g.rows.insert(g.rows.end(), {at(*p), at(grad), at(*m), at(*v), n, g.blocks});
@@ -568,18 +580,16 @@ PT_FN(adamw_scan, 3)
     return PyBytes_FromStringAndSize(reinterpret_cast<const char*>(rows.data()),
                                      static_cast<Py_ssize_t>(rows.size() * sizeof(int64_t)));
   };
-  PyObject* list = PyList_New(0);
-  for (const Group& g : groups) {
-    PyObject* steps = PyList_New(0);
-    for (PyObject* s : g.steps) PyList_Append(steps, s);
-    PyObject* entry = Py_BuildValue("(NnLdN)", bytes(g.rows), static_cast<Py_ssize_t>(g.rows.size() / 6),
-                                    static_cast<long long>(g.blocks), static_cast<double>(g.step), steps);
-    if (entry == nullptr) return nullptr;
-    PyList_Append(list, entry);
-    Py_DECREF(entry);
+  THPObjectPtr list{PyList_New(0)};
+  if (!list) return nullptr;
+  for (Group& g : groups) {
+    THPObjectPtr entry{Py_BuildValue("(NnLdO)", bytes(g.rows), static_cast<Py_ssize_t>(g.rows.size() / 6),
+                                     static_cast<long long>(g.blocks), static_cast<double>(g.step),
+                                     g.steps.get())};
+    if (!entry || PyList_Append(list, entry.get()) != 0) return nullptr;
   }
-  return Py_BuildValue("(iLNN)", static_cast<int>(device.index()), static_cast<long long>(all),
-                       bytes(grads), list);
+  return Py_BuildValue("(iLNO)", static_cast<int>(device.index()), static_cast<long long>(all),
+                       bytes(grads), list.get());
 PT_END
 
 // Adds 1 to each fp32 host step tensor of a list, as `step += 1` does.

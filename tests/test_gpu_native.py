@@ -325,3 +325,30 @@ def test_writes_leave_lazily_cloned_tensors_alone(gpu):
     triton_clip_grad_norm_and_step(opt, 0.05)
     _same(shared, kept)
     assert float(opt.state[params[0]]["step"]) == 2.0 and not torch.equal(params[0], shared[0])
+
+
+def test_adamw_scan_outlives_what_a_hash_drops(gpu, monkeypatch):
+    """The scan's dict lookups hash parameters in Python, where other threads run too: step tensors,
+    gradients and states that go away there stay valid until the scan is done with them."""
+
+    params, opt = _optimizer(gpu, 11)
+    for p in params[:-1]:
+        p.grad = torch.ones_like(p)
+    triton_adamw_step(opt)
+    states = [opt.state[p] for p in params[:-1]]
+    hashes = []
+
+    def dropping(self):
+        hashes.append(id(self))
+        self.grad = None  # the parameter's own gradient, which the scan has just read
+        if len(hashes) == 2:
+            states[0].clear()  # and the step count of the parameter before
+        return id(self)
+
+    with monkeypatch.context() as m:
+        m.setattr(torch.Tensor, "__hash__", dropping)
+        found = _lib.extension().adamw_scan([params[:-1]], opt.state, 1024)
+    assert len(hashes) == 5 and found is not None
+    steps = found[3][0][4]
+    assert [float(s) for s in steps] == [1.0] * 5
+    assert found[3][0][1] == 5
