@@ -41,18 +41,28 @@ def _device_supported(index: int) -> bool:
     return ops.device_supported(index)
 
 
+# torch's own names for what no_graph() asks; None in a torch without one of them, where every call
+# then goes through its autograd Function.
+_tracing_state = getattr(torch._C, "_get_tracing_state", None)
+_functorch_active = getattr(torch._C, "_are_functorch_transforms_active", None)
+_CAN_SKIP_FUNCTION = (_tracing_state is not None and _functorch_active is not None
+                      and hasattr(forward_ad, "_current_level"))
+
+
 def no_graph(*tensors: Tensor) -> bool:
     """True when an autograd Function over these inputs would record nothing, so that its forward
     can be called directly (4 us less of host time): no gradient is asked for, and nothing else
     looks at the call as a node -- forward-mode differentiation, a functorch transform (both of
     which a Function refuses, and the caller falls back), jit tracing, torch.compile."""
 
+    if not _CAN_SKIP_FUNCTION:
+        return False
     if torch.is_grad_enabled():
         for t in tensors:
             if t.requires_grad:
                 return False
-    return (forward_ad._current_level < 0 and torch._C._get_tracing_state() is None
-            and not torch._C._are_functorch_transforms_active() and not torch.compiler.is_compiling())
+    return (forward_ad._current_level < 0 and _tracing_state() is None and not _functorch_active()
+            and not torch.compiler.is_compiling())
 
 
 def require_hip(exc: type[RuntimeError], op: str, *tensors: Tensor) -> None:

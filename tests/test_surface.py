@@ -5,6 +5,8 @@ ce_adamw}.py and tests/test_rope.py).  On CPU every fused path must raise its
 
 from __future__ import annotations
 
+import subprocess
+import sys
 import warnings
 
 import pytest
@@ -12,6 +14,7 @@ import torch
 from torch.nn import functional as F
 from torch.optim import AdamW
 
+from conftest import ROOT
 from picotron_amd.config import ConfigValidationError, TritonKernelsConfig
 from picotron_amd.hardware import detect_triton_support, kernel_status_rows
 from picotron_amd.nn import RMSNorm, RotaryEmbedding, SwiGLU, apply_rotary_embedding, rotary_cos_sin
@@ -324,3 +327,20 @@ def test_oracle_not_imported_by_product():
     pkg = pathlib.Path(__file__).resolve().parents[1] / "picotron_amd"
     for path in pkg.rglob("*.py"):
         assert not re.search(r"^\s*(from|import)\s+oracle\b", path.read_text(), flags=re.M), path
+
+
+@pytest.mark.parametrize("name", ["torch._C._get_tracing_state", "torch._C._are_functorch_transforms_active",
+                                  "forward_ad._current_level"])
+def test_graph_free_calls_need_no_private_torch_name(name):
+    """The names that tell a call without a graph are torch's own: without one of them a call goes
+    through its autograd Function instead of failing."""
+
+    code = (f"import sys; sys.path.insert(0, {str(ROOT)!r})\n"
+            "import torch\n"
+            "from torch.autograd import forward_ad\n"
+            "import torch._dynamo  # uses them itself\n"
+            f"del {name}\n"
+            "from picotron_amd.nn.triton_kernels import _gate\n"
+            "assert _gate.no_graph(torch.zeros(2)) is False\n")
+    proc = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert proc.returncode == 0, proc.stdout + proc.stderr
