@@ -399,19 +399,32 @@ __device__ __forceinline__ float column_group_sum(const float* __restrict__ part
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) s += v[u];
   }
-  // The remainder (fewer than kUnroll partials per group) in batches of 16 independent loads,
-  // the last one's filled up with the last partial, counted as 0: a few round trips rather than
-  // one per partial ([256, 1024] bf16, 64 partials: the whole backward call 8.1 -> 6.4 us).
+  // The remainder (fewer than kUnroll partials per group) in batches of 16 independent loads: whole
+  // ones, then one filled up with the group's last partial, counted as 0 -- a few round trips rather than
+  // one per partial.  Whole batches without clamps, and the clamp as a running offset: a multiplied and
+  // selected index for each load costs 0.4 to 0.9 us per call ([16, 2048] and [512, 1024] fp32).
   constexpr int kRest = 16;
-  for (; i < nparts; i += kFinishGroups * kRest) {
+  const int64_t step = static_cast<int64_t>(kFinishGroups) * cols;
+  for (; i + static_cast<int64_t>(kFinishGroups) * (kRest - 1) < nparts;
+       i += static_cast<int64_t>(kFinishGroups) * kRest) {
+    const float* q = p + i * cols;
+    float v[kRest];
+#pragma unroll
+    for (int u = 0; u < kRest; ++u) v[u] = q[u * step];
+#pragma unroll
+    for (int u = 0; u < kRest; ++u) s += v[u];
+  }
+  if (i < nparts) {
+    const int left = static_cast<int>((nparts - 1 - i) / kFinishGroups) + 1;
+    const float* q = p + i * cols;
     float v[kRest];
 #pragma unroll
     for (int u = 0; u < kRest; ++u) {
-      const int64_t at = i + u * kFinishGroups;
-      v[u] = p[(at < nparts ? at : nparts - 1) * cols];
+      if (u > 0) q += u < left ? step : 0;
+      v[u] = *q;
     }
 #pragma unroll
-    for (int u = 0; u < kRest; ++u) s += i + u * kFinishGroups < nparts ? v[u] : 0.0f;
+    for (int u = 0; u < kRest; ++u) s += u < left ? v[u] : 0.0f;
   }
   return s;
 }

@@ -251,3 +251,19 @@ def test_general_rows_at_the_ends_of_their_shapes(gpu, dtype, wdtype, vectors, e
     assert torch.equal(in_place, dh)
     # dx is rounded once more than dh, which adds dh_in before its one rounding
     close(dh, dx.double() + dh_in.double(), dtype, scale=float(dx.abs().max()) + float(dh_in.abs().max()))
+
+
+@pytest.mark.parametrize("partials", [1, 7, 8, 9, 120, 121, 127, 128, 129, 136, 137, 255, 256])
+def test_weight_gradient_over_any_number_of_partials(gpu, partials):
+    """Rows of 5120 bf16 leave one partial each: whole and partly filled batches of the finish's loads,
+    with the last partial standing out, so that counting it twice or not at all shows."""
+
+    x, dy = randn((partials, 5120), torch.bfloat16, gpu, partials), randn((partials, 5120), torch.bfloat16, gpu, 7)
+    dy[-1] *= 64
+    w = torch.ones(5120, device=gpu)
+    _, rstd = ops.rmsnorm_fwd(x, w, 1e-5)
+    _, dw = ops.rmsnorm_bwd(dy, x, w, rstd)
+    _, dw64 = o_rms.backward(dy, x, w, 1e-5)
+    mag = o_rms.backward(dy.abs(), x.abs(), w, 1e-5)[1]
+    # fp32 sums of `partials` products in another order
+    assert bool(((dw.double() - dw64).abs() <= 1e-6 * mag).all())
