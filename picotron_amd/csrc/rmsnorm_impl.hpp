@@ -52,10 +52,12 @@ constexpr bool kLoadNT = true;
 // one vector (its value is never used).
 static __device__ __align__(16) unsigned int kPad[8];
 
-// True if vector k of lane rl lies wholly inside the row.
-template <typename T, int LANES>
+// True if vector k of lane rl lies wholly inside the row.  For rows of whole vectors the test is
+// the one of their loads, so that the compiler keeps one mask for both.
+template <typename T, int LANES, bool ALIGNED>
 __device__ __forceinline__ bool in_row(int rl, int k, int cols) {
-  return ((rl + k * LANES) + 1) * Elem<T>::VEC <= cols;
+  const int e = (rl + k * LANES) * Elem<T>::VEC;
+  return ALIGNED ? e < cols : e + Elem<T>::VEC <= cols;
 }
 
 // The remainder element of this lane (rows that are not whole vectors): its column, or -1.
@@ -85,9 +87,13 @@ struct LaneWeights {
   __device__ __forceinline__ void load(const void* w, int, int rl, int cols) {
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
-      const WT* p = reinterpret_cast<const WT*>(w) + (rl + k * LANES) * N;
-      if (!in_row<T, LANES>(rl, k, cols))
-        p = ALIGNED ? reinterpret_cast<const WT*>(w) : reinterpret_cast<const WT*>(kPad);
+      const int e = (rl + k * LANES) * N;
+      const WT* p = reinterpret_cast<const WT*>(w);
+      if constexpr (ALIGNED) {
+        p += e < cols ? e : 0;
+      } else {
+        p = in_row<T, LANES, ALIGNED>(rl, k, cols) ? p + e : reinterpret_cast<const WT*>(kPad);
+      }
 #pragma unroll
       for (int l = 0; l < kWords; ++l) wd[k][l].raw = load_vec<WT, ALIGNED, false>(p + l * kPer);
     }
@@ -109,7 +115,7 @@ struct LaneWeights<T, void, VPL, LANES, ALIGNED> {
   __device__ __forceinline__ void load(const void* w, int wdt, int rl, int cols) {
 #pragma unroll
     for (int k = 0; k < VPL; ++k) {
-      const bool in = in_row<T, LANES>(rl, k, cols);
+      const bool in = in_row<T, LANES, ALIGNED>(rl, k, cols);
 #pragma unroll
       for (int i = 0; i < N; ++i) f[k][i] = in ? load_any(w, (rl + k * LANES) * N + i, wdt) : 0.0f;
     }
@@ -170,9 +176,13 @@ __device__ __forceinline__ void load_row(const T* __restrict__ row, int rl, int 
                                          RowRegs<T, VPL>& r) {
 #pragma unroll
   for (int k = 0; k < VPL; ++k) {
-    const T* p = row + (rl + k * LANES) * Elem<T>::VEC;
-    if (!in_row<T, LANES>(rl, k, cols)) p = ALIGNED ? row : reinterpret_cast<const T*>(kPad);
-    r.v[k].raw = load_vec<T, ALIGNED, NT>(p);
+    const int e = (rl + k * LANES) * Elem<T>::VEC;
+    if constexpr (ALIGNED) {
+      r.v[k].raw = load16<NT>(row + (e < cols ? e : 0));
+    } else {
+      const T* p = in_row<T, LANES, ALIGNED>(rl, k, cols) ? row + e : reinterpret_cast<const T*>(kPad);
+      r.v[k].raw = load_vec<T, false, NT>(p);
+    }
   }
   if constexpr (!ALIGNED) {
     const int c = tail_col<T>(rl, cols);
@@ -205,7 +215,7 @@ struct RowStore {
     if constexpr (ALIGNED) {
       __builtin_amdgcn_raw_buffer_store_b128(v.raw, rsrc, e * static_cast<int>(sizeof(T)), 0,
                                              POLICY);
-    } else if (in_row<T, LANES>(rl, k, cols)) {
+    } else if (in_row<T, LANES, ALIGNED>(rl, k, cols)) {
       store_vec<T, false, true>(row + e, v.raw);
     }
   }
@@ -314,7 +324,7 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_fwd_kernel(
           const float f = xr.at(k, i);
           part += f * f;
         }
-        ss += in_row<T, LANES>(rl, k, cols) ? part : 0.0f;
+        ss += in_row<T, LANES, ALIGNED>(rl, k, cols) ? part : 0.0f;
       }
       if constexpr (!ALIGNED) {
         const float f = Elem<T>::to_f32(xr.tail);
@@ -514,7 +524,7 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_bwd_kernel(
         float part = 0.0f;
 #pragma unroll
         for (int i = 0; i < V; ++i) part += (bf.g.at(k, i) * wv[k][i]) * bf.x.at(k, i);
-        dot += in_row<T, LANES>(rl, k, cols) ? part : 0.0f;
+        dot += in_row<T, LANES, ALIGNED>(rl, k, cols) ? part : 0.0f;
       }
       if constexpr (!ALIGNED) {
         const float part = (Elem<T>::to_f32(bf.g.tail) * wtail) * Elem<T>::to_f32(bf.x.tail);
@@ -601,7 +611,7 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_bwd_kernel(
       const int e = (rl + k * LANES) * V;
 #pragma unroll
       for (int i = 0; i < V; ++i)
-        if (in_row<T, LANES>(rl, k, cols)) prow[e + i] = acc[k][i];
+        if (in_row<T, LANES, ALIGNED>(rl, k, cols)) prow[e + i] = acc[k][i];
     }
     if (tail_c >= 0) prow[tail_c] = acc_tail;
   } else {
@@ -615,7 +625,7 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_bwd_kernel(
           const int e = (rl + k * LANES) * V;
 #pragma unroll
           for (int i = 0; i < V; ++i) {
-            if (in_row<T, LANES>(rl, k, cols))
+            if (in_row<T, LANES, ALIGNED>(rl, k, cols))
               lds_dw[e + i] = (s == 0) ? acc[k][i] : lds_dw[e + i] + acc[k][i];
           }
         }
