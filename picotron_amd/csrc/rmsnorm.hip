@@ -91,7 +91,8 @@ int fwd_impl(const char* fn, const void* x, int64_t xs, const void* res, int64_t
   a.h_s = hs;
   a.aligned = (cols % vec == 0) && rows_aligned(x_dtype, x, xs) && rows_aligned(x_dtype, y, ys) &&
               (!fused || (rows_aligned(x_dtype, res, res_s) && rows_aligned(x_dtype, h, hs))) &&
-              aligned16(weight) && vector_weight(x_dtype, w_dtype) && !short_row(cols, vec);
+              aligned16(weight) && vector_weight(x_dtype, w_dtype) &&
+              !short_row_fwd(rows, cols, vec, fused);
   a.shape = a.aligned ? s : general_shape(cols, vec, false);
   a.blocks = fwd_blocks(rows, a.shape, num_cus(), a.aligned);
   a.st = as_stream(stream);

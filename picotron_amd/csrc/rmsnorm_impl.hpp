@@ -314,7 +314,10 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_fwd_kernel(
         if (active) hs.store_tail(rl, Elem<T>::to_f32(xr.tail));
       }
     }
-    float ss = 0.0f;
+    // Rows that two kernels take by their count (short_row_fwd) get the same bits from both: 16 lanes
+    // sum each 16 vectors of their row apart and add the sums in order, as one wave does (wave_sum).
+    constexpr int kParts = WPR == 0 ? VPL : 1;
+    float ss[kParts] = {};
     if (active) {
 #pragma unroll
       for (int k = 0; k < VPL; ++k) {
@@ -324,17 +327,19 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_fwd_kernel(
           const float f = xr.at(k, i);
           part += f * f;
         }
-        ss += in_row<T, LANES, ALIGNED>(rl, k, cols) ? part : 0.0f;
+        ss[k % kParts] += in_row<T, LANES, ALIGNED>(rl, k, cols) ? part : 0.0f;
       }
       if constexpr (!ALIGNED) {
         const float f = Elem<T>::to_f32(xr.tail);
-        ss += has_tail ? f * f : 0.0f;
+        ss[0] += has_tail ? f * f : 0.0f;
       }
     }
     xr.opaque();
-    ss = row_sum<WPR, WAVES>(ss, red, wave, lane, buf);
+    float sum = row_sum<WPR, WAVES>(ss[0], red, wave, lane, buf);
+#pragma unroll
+    for (int p = 1; p < kParts; ++p) sum += row_sum<WPR, WAVES>(ss[p], red, wave, lane, buf);
     if (!active) return;
-    const float r = 1.0f / sqrtf(ss * inv_cols + eps);
+    const float r = 1.0f / sqrtf(sum * inv_cols + eps);
     if (rl == 0) rstd[row] = r;
     const RowStore<T, LANES, ALIGNED, kWriteThrough> yst(y + row * ys, cols);
 #pragma unroll
@@ -734,6 +739,16 @@ constexpr int64_t kQuarterVecs = 32;
 
 // Aligned rows that the general kernels take too.
 inline bool short_row(int64_t cols, int vec) { return (cols + vec - 1) / vec <= kQuarterVecs; }
+
+// The forward's: a few rows of nearly 32 vectors are as many waves too few that way, and stay with one
+// wave each.  us, four rows per wave against one: [2048, 256] bf16 2.6 2.3, with the residual add
+// 3.1 2.8, [512, 256] 2.1 2.1 and 2.6 2.3, [2048, 128] fp32 2.5 2.2 and 2.8 2.7; [4096, 256] bf16 2.7 2.8
+// and 3.3 3.8, [4096, 128] fp32 2.6 2.5 and 3.0 3.7, [8192, 256] bf16 3.2 3.9.  At 25 vectors four per
+// wave win at every count ([512, 200] bf16 2.2 2.4, [2048, 100] fp32 2.6 2.7).
+inline bool short_row_fwd(int64_t rows, int64_t cols, int vec, bool fused) {
+  const int64_t nvec = (cols + vec - 1) / vec;
+  return short_row(cols, vec) && (nvec <= 28 || rows > (fused ? 2048 : 4096));
+}
 
 inline Shape general_shape(int64_t cols, int vec, bool backward) {
   const int64_t nvec = (cols + vec - 1) / vec;

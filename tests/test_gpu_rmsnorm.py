@@ -267,3 +267,23 @@ def test_weight_gradient_over_any_number_of_partials(gpu, partials):
     mag = o_rms.backward(dy.abs(), x.abs(), w, 1e-5)[1]
     # fp32 sums of `partials` products in another order
     assert bool(((dw.double() - dw64).abs() <= 1e-6 * mag).all())
+
+
+@pytest.mark.parametrize("dtype,cols", [(torch.float32, 116), (torch.float32, 128), (torch.bfloat16, 232),
+                                        (torch.bfloat16, 256), (torch.float16, 248)])
+def test_a_row_has_the_same_bits_at_every_row_count(gpu, dtype, cols):
+    """The forward's kernel depends on the number of rows (rows of 29-32 vectors); a row's result
+    does not."""
+
+    x, r = randn((4200, cols), dtype, gpu, cols), randn((4200, cols), dtype, gpu, cols + 1)
+    w = randn((cols,), dtype, gpu, cols + 2, 0.02, 1.0)
+    y, rstd = ops.rmsnorm_fwd(x, w, 1e-5)
+    h, yr, rr = ops.residual_rmsnorm_fwd(x, r, w, 1e-5)
+    y64, r64 = o_rms.forward(x, w, 1e-5)
+    close(y, y64, dtype)
+    close_fp32(rstd, r64)
+    for rows in (1, 5, 1023, 1024, 2048, 2049, 4095, 4096, 4097):
+        a, b = ops.rmsnorm_fwd(x[:rows], w, 1e-5)
+        assert torch.equal(a, y[:rows]) and torch.equal(b, rstd[:rows]), rows
+        c, a, b = ops.residual_rmsnorm_fwd(x[:rows], r[:rows], w, 1e-5)
+        assert torch.equal(c, h[:rows]) and torch.equal(a, yr[:rows]) and torch.equal(b, rr[:rows]), rows
