@@ -314,9 +314,11 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_fwd_kernel(
         if (active) hs.store_tail(rl, Elem<T>::to_f32(xr.tail));
       }
     }
-    // Rows that two kernels take by their count (short_row_fwd) get the same bits from both: 16 lanes
-    // sum each 16 vectors of their row apart and add the sums in order, as one wave does (wave_sum).
-    constexpr int kParts = WPR == 0 ? VPL : 1;
+    // Rows that two kernels take by their count (short_row_fwd, fwd_vpl_cap_for) get the same bits from
+    // both: 16 lanes sum each 16 vectors of their row apart and add the sums in order, as one wave
+    // does (wave_sum), and one wave sums every other 64 vectors apart, as two waves do (row_sum).
+    constexpr int kParts =
+        WPR == 0 ? VPL : (ALIGNED && WPR == 1 && VPL == 8 && sizeof(T) == 4 ? 2 : 1);
     float ss[kParts] = {};
     if (active) {
 #pragma unroll
@@ -675,13 +677,18 @@ inline int bwd_vpl_cap_for(int tuned, int64_t cols, int vec) {
 // eight of fp32 (two waves per 4096-wide row either way); measured at [16384, 4096], 4 layers:
 // bf16 0.4628-0.4639 ms per step against 0.4660-0.4684 with two and 0.4747-0.4763 with eight,
 // fp32 0.8769-0.8777 ms against 0.8868-0.8871 with four.
-// Aligned fp32 rows of 257-512 vectors hold four per lane of two waves instead of eight of one:
-// [16384, 2048] 46.7 -> 45.1 us, with the residual add (two such rows per lane) 93.0 -> 88.8
-// (the general kernels lose by it: [16384, 1370] 66.0 -> 67.9 with the add).
-inline int fwd_vpl_cap_for(int tuned, int64_t cols, int vec) {
+// Aligned fp32 rows of 257-512 vectors hold four per lane of two waves instead of eight of one
+// (the general kernels lose by it: [16384, 1370] 66.0 -> 67.9 with the add) where the rows leave CUs
+// with little to do or fill all of them several times; in between one wave per row spreads evenly
+// over the CUs, and the two waves' barrier only costs.  us, one wave against two, 2048 columns:
+// plain / with the residual add 64 rows 2.7 2.5 / 3.9 3.2, 512 3.9 3.6 / 6.0 5.0, 1024 4.4 4.9 / 7.8 7.4,
+// 2048 7.1 7.9 / 12.6 13.4, 3072 9.7 10.5 / 18.6 18.7, 4096 13.5 13.3 / 24.4 24.0, 16384 44.9 43.8 /
+// 89.1 87.2; 1280 columns 512 3.4 3.1, 1024 3.9 4.0, 3072 7.1 8.0, 4096 9.9 9.5.
+inline int fwd_vpl_cap_for(int tuned, int64_t rows, int64_t cols, int vec) {
   if (tuned > 0) return tuned;
   const int64_t nvec = (cols + vec - 1) / vec;
-  return vec == 4 && nvec > 256 && nvec <= 512 ? 4 : 32 / vec;
+  const bool two_waves = rows < 1024 || rows >= 4096;
+  return vec == 4 && nvec > 256 && nvec <= 512 && two_waves ? 4 : 32 / vec;
 }
 
 inline int64_t env_positive(const char* name, int64_t fallback) {

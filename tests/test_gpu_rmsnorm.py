@@ -269,11 +269,12 @@ def test_weight_gradient_over_any_number_of_partials(gpu, partials):
     assert bool(((dw.double() - dw64).abs() <= 1e-6 * mag).all())
 
 
-@pytest.mark.parametrize("dtype,cols", [(torch.float32, 116), (torch.float32, 128), (torch.bfloat16, 232),
+@pytest.mark.parametrize("dtype,cols", [(torch.float32, 1028), (torch.float32, 1540), (torch.float32, 2048),
+                                        (torch.float32, 116), (torch.float32, 128), (torch.bfloat16, 232),
                                         (torch.bfloat16, 256), (torch.float16, 248)])
 def test_a_row_has_the_same_bits_at_every_row_count(gpu, dtype, cols):
-    """The forward's kernel depends on the number of rows (rows of 29-32 vectors); a row's result
-    does not."""
+    """The forward's kernel depends on the number of rows (fp32 rows of 257-512 vectors, rows of 29-32
+    vectors); a row's result does not."""
 
     x, r = randn((4200, cols), dtype, gpu, cols), randn((4200, cols), dtype, gpu, cols + 1)
     w = randn((cols,), dtype, gpu, cols + 2, 0.02, 1.0)
