@@ -134,7 +134,7 @@ int bwd_impl(const char* fn, const void* dy, int64_t dys, const void* dh_in, int
   a.aligned = vectors && !short_row(cols, vec);
   a.shape = a.aligned ? s : general_shape(cols, vec, true);
   const int64_t bound = bwd_partial_bound(rows, cols, vec, vectors, s);
-  a.blocks = bwd_blocks(rows, a.shape, bwd_partials_for(cols, dtype_size(x_dtype)));
+  a.blocks = bwd_blocks(rows, a.shape, bwd_partials_for(rows, cols, dtype_size(x_dtype)));
   if (a.blocks > bound) a.blocks = bound;
   float* partial = nullptr;
   if (dweight) {

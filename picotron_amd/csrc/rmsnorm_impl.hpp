@@ -807,14 +807,22 @@ constexpr int64_t kMostPartials = 512;
 
 // One workgroup per CU keeps HBM busy when its rows are long enough, two streams of the current
 // and the next row group in flight, and half as many partial rows are then written and summed.
-// 512 against 256 workgroups at 16384 rows, us per call (plain, residual form): bf16 2048 38.2 / 41.2
-// and 50.9 / 47.0, 2560 49.5 / 55.4 and 63.4 / 61.4, 4096 73.1 / 69.2 and 96.1 / 91.5, 5120 94.2 / 95.2
-// and 121.6 / 112.7; fp32 768 28.7 / 31.0 and 36.9 / 35.5, 1024 37.1 / 36.4 and 49.1 / 47.0, 2048 70.2 /
-// 67.5 and 92.8 / 88.2.  384 leave half of the CUs with two workgroups and are slower than both.
+// us of the whole call with 512 against 256 workgroups (plain, residual form): bf16 4096 columns 2048 rows
+// 16.6 15.7 and 19.3 18.0, 16384 rows 71.8 69.0 and 95.8 92.4; 8192 columns 512 rows 15.8 11.5 and
+// 17.1 12.4, 16384 rows 139.4 132.8 and 180.7 175.0; fp32 1024 columns 2048 rows 10.0 9.4 and 11.1 10.5,
+// 16384 rows 37.0 36.0 and 49.2 47.3; 4096 columns 16384 rows 132.9 128.6 and 183.6 178.5.  Shorter rows
+// lose ([16384, 2048] bf16 38.2 41.2), and so do many rows that fill two vectors of each of 16 waves'
+// lanes: 16384 rows of 16384 bf16 271.2 277.6 and 373.2 387.4, of 8192 fp32 271.7 277.4 and 376.3 377.4
+// (8192 rows 143.8 138.0 and 193.6 192.6, and 136.6 135.6 and 187.1 190.6); fp32 rows beyond that
+// also (16384 columns 547.8 567.5 and 933.1 927.5), bf16 ones not (32768: 1439 1416).
+// 384 leave half of the CUs with two workgroups and are slower than both.
 // The residual form takes the plain one's count, so that their weight gradients are the same bits.
-inline int64_t bwd_partials_for(int64_t cols, int esize) {
+inline int64_t bwd_partials_for(int64_t rows, int64_t cols, int esize) {
   if (tuning().bwd_partials > 0) return tuning().bwd_partials;
-  return cols * esize >= (esize == 4 ? 4096 : 8192) ? kMostPartials / 2 : kMostPartials;
+  const int64_t bytes = cols * esize;
+  if (bytes < (esize == 4 ? 4096 : 8192)) return kMostPartials;
+  const bool full = bytes > 24576 && (bytes <= 32768 || esize == 4);
+  return full && rows >= 16384 ? kMostPartials : kMostPartials / 2;
 }
 
 // The most that bwd_partials_for gives, for sizing workspaces.
