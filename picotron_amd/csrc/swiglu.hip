@@ -12,7 +12,7 @@
 // use nontemporal loads/stores (they are touched exactly once).  Elements past the last
 // whole vector go one to a thread of the first workgroup, in the same launch (a second launch for
 // them cost 4.1 us forward and 4.5 backward), and streams that are not all 16-byte aligned move the
-// same vectors at the element's alignment.
+// same vectors at the element's alignment (in a short backward, elements).
 #include "pt_common.hpp"
 
 namespace pt {
@@ -130,6 +130,23 @@ __global__ __launch_bounds__(256) void swiglu_bwd_kernel(const T* __restrict__ d
   }
 }
 
+// One element per thread: a short backward of streams that are not all 16-byte aligned.
+template <typename T>
+__global__ __launch_bounds__(256) void swiglu_bwd_elem_kernel(const T* __restrict__ dy,
+                                                              const T* __restrict__ g,
+                                                              const T* __restrict__ u,
+                                                              T* __restrict__ dg,
+                                                              T* __restrict__ du, int n) {
+  const int i = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+  if (i >= n) return;
+  SwigluGrad r = swiglu_grad(Elem<T>::to_f32(dy[i]), Elem<T>::to_f32(g[i]), Elem<T>::to_f32(u[i]));
+  // Rounded to fp32 before the conversion, as in the vector kernels: left alone, the compiler fuses a
+  // lone element's last multiply and its fp16 conversion into one rounding.
+  asm volatile("" : "+v"(r.g), "+v"(r.u));
+  if (dg != nullptr) dg[i] = Elem<T>::from_f32(r.g);
+  if (du != nullptr) du[i] = Elem<T>::from_f32(r.u);
+}
+
 // Vectors per stream per thread.  The backward (3 streams read, 2 written) keeps two in
 // flight and runs 2 workgroups per CU: [16384, 14336] bf16 366-367 us, against 383 us with
 // four vectors at full occupancy and 395-399 us with two at full occupancy.  The forward
@@ -142,6 +159,19 @@ constexpr int kFwdUnroll = 4;
 constexpr int kBwdUnroll = 2;
 // Streams above this many bytes bypass cache retention (nontemporal).
 constexpr int64_t kNontemporalBytes = int64_t{64} << 20;
+
+// Streams that are not all 16-byte aligned.  A small call is bound by what one thread does after its
+// loads, so it spreads the elements over more threads: the forward takes one vector per thread up to 4 MB a
+// stream, the backward one element per thread up to 393216 elements.  Above, the forward and the fp32
+// backward take the large aligned streams' shape at every size (nontemporal), the 16-bit backward one vector
+// per thread, plain accesses and no limit on resident workgroups.  us at one element's offset, four (two)
+// nontemporal vectors per thread against the shape taken: forward bf16 10007 elements 2.84 1.87, 100003 3.00
+// 1.95, 1000003 3.99 2.86, 2000003 4.31 3.87 (4000003 6.91 6.80, 32000011 34.1 34.3), fp32 100003 2.36 1.88,
+// 600011 3.12 2.85 (2000003 5.65 6.02); backward bf16 10007 2.75 1.89, 300007 3.51 2.47, 600011 3.66 3.27,
+// 16000003 35.1 29.7, 64000003 130 110, fp32 100003 2.85 2.25, 300007 3.06 3.02 (600011 4.35 against 4.57 by
+// elements and 4.08 by one vector, 4000003 15.8 and 17.1).
+constexpr int64_t kAnyFwdBytes = int64_t{4} << 20;
+constexpr int64_t kAnyBwdElems = 3 << 17;
 
 // Resident workgroups per CU of the vector kernels (0: no limit); PT_SWIGLU_FWD_OCCUPANCY
 // and PT_SWIGLU_BWD_OCCUPANCY override them.
@@ -178,16 +208,20 @@ void launch_fwd(const void* g, const void* u, void* o, int64_t n, hipStream_t st
   const int tail = static_cast<int>(n % V);
   const bool nt = n * static_cast<int64_t>(sizeof(T)) > kNontemporalBytes;
   const unsigned grid = grid_for(nvec, 256 * kFwdUnroll);
-  const auto go = [&](auto kernel) {
-    launch_limited(kernel, fwd_occupancy(), grid, st, static_cast<const T*>(g),
+  const auto go = [&](auto kernel, unsigned blocks) {
+    launch_limited(kernel, fwd_occupancy(), blocks, st, static_cast<const T*>(g),
                    static_cast<const T*>(u), static_cast<T*>(o), nvec, tail);
   };
   if (!(aligned16(g) && aligned16(u) && aligned16(o))) {
-    go(swiglu_fwd_kernel<T, kFwdUnroll, true, false>);
+    if (n * static_cast<int64_t>(sizeof(T)) <= kAnyFwdBytes) {
+      go(swiglu_fwd_kernel<T, 1, false, false>, grid_for(nvec, 256));
+    } else {
+      go(swiglu_fwd_kernel<T, kFwdUnroll, true, false>, grid);
+    }
   } else if (nt) {
-    go(swiglu_fwd_kernel<T, kFwdUnroll, true, true>);
+    go(swiglu_fwd_kernel<T, kFwdUnroll, true, true>, grid);
   } else {
-    go(swiglu_fwd_kernel<T, kFwdUnroll, false, true>);
+    go(swiglu_fwd_kernel<T, kFwdUnroll, false, true>, grid);
   }
 }
 
@@ -206,7 +240,15 @@ void launch_bwd(const void* dy, const void* g, const void* u, void* dg, void* du
                    static_cast<const T*>(g), static_cast<const T*>(u), static_cast<T*>(dg),
                    static_cast<T*>(du), nvec, tail);
   };
-  if (!aligned) {
+  if (!aligned && n <= kAnyBwdElems) {
+    hipLaunchKernelGGL(swiglu_bwd_elem_kernel<T>, dim3(grid_for(n, 256)), dim3(256), 0, st,
+                       static_cast<const T*>(dy), static_cast<const T*>(g), static_cast<const T*>(u),
+                       static_cast<T*>(dg), static_cast<T*>(du), static_cast<int>(n));
+  } else if (!aligned && sizeof(T) == 2) {
+    hipLaunchKernelGGL((swiglu_bwd_kernel<T, 1, false, false, false>), dim3(grid_for(nvec, 256)),
+                       dim3(256), 0, st, static_cast<const T*>(dy), static_cast<const T*>(g),
+                       static_cast<const T*>(u), static_cast<T*>(dg), static_cast<T*>(du), nvec, tail);
+  } else if (!aligned) {
     go(swiglu_bwd_kernel<T, kBwdUnroll, true, false, false>);
   } else if (nt && nvec <= 0x7fffffff / 16) {
     go(swiglu_bwd_kernel<T, kBwdUnroll, true, true, true>);

@@ -72,7 +72,7 @@ def test_sizes(gpu, dtype, n):
 
 def test_unaligned_and_special_values(gpu):
     base = randn((4099,), torch.bfloat16, gpu, 5)
-    g, u, dy = base[1:4000], base[2:4001], base[3:4002]  # 2-byte offsets: element path
+    g, u, dy = base[1:4000], base[2:4001], base[3:4002]  # 2-byte offsets: unaligned vectors, a backward by elements
     _check(g, u, dy, torch.bfloat16)
     special = torch.tensor([0.0, -0.0, 1e-30, -100.0, 100.0, -88.0, 88.0, 1.0], device=gpu)
     ones = torch.ones_like(special)
@@ -124,3 +124,22 @@ def test_tails_and_streams_off_16_byte_boundaries(gpu, dtype, n, offsets):
         assert torch.equal(got, ref)
     only_up = ops.swiglu_bwd(dy, g, u, need_dgate=False)
     assert only_up[0] is None and torch.equal(only_up[1], ops.swiglu_bwd(da, ga, ua)[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n", [(3 << 17) - 1, 3 << 17, (3 << 17) + 1, (1 << 20) + 1, 1 << 21, (1 << 21) + 9])
+def test_streams_off_16_byte_boundaries_at_the_ends_of_their_rules(gpu, dtype, n):
+    """Backward by elements, by one vector and by two; forward by one vector and by four."""
+
+    g, u, dy = (randn((n + 1,), dtype, gpu, n + i)[1:] for i in range(3))
+    ga, ua, da = g.clone(), u.clone(), dy.clone()
+    assert torch.equal(ops.swiglu_fwd(g, u), ops.swiglu_fwd(ga, ua))
+    for need in ((True, True), (True, False), (False, True)):
+        for got, ref in zip(ops.swiglu_bwd(dy, g, u, *need), ops.swiglu_bwd(da, ga, ua)):
+            assert got is None or torch.equal(got, ref)
+    tail = slice(n - 20, n)
+    close(ops.swiglu_fwd(g, u)[tail], o_swiglu.forward(g[tail], u[tail]), dtype)
+    dg64, du64 = o_swiglu.backward(dy[tail], g[tail], u[tail])
+    dg, du = ops.swiglu_bwd(dy, g, u)
+    close(dg[tail], dg64, dtype)
+    close(du[tail], du64, dtype)
