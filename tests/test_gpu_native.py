@@ -39,20 +39,34 @@ def _same(a, b):
     assert torch.equal(a, b)
 
 
-def _both(monkeypatch, call):
-    """The result (or the exception's type) of a call as it is and through the general route."""
+def _both(monkeypatch, call, native=None, raises=None):
+    """The result of a call as it is and through the general route (or the type of the exception
+    `raises`, which both then have to raise).  `native`: whether the first one's launches all took
+    (True) or all left (False) the native route; None where the form decides."""
+
+    taken = []
+    launch = ops._launch
+
+    def recording(*args):
+        out = launch(*args)
+        taken.append(out is not None)
+        return out
 
     def attempt():
-        try:
+        if raises is None:
             return call()
-        except Exception as error:
-            return type(error)
+        with pytest.raises(raises) as caught:
+            call()
+        return caught.type
 
-    out = attempt()
     with monkeypatch.context() as m:
+        m.setattr(ops, "_launch", recording)
+        out = attempt()
         m.setattr(ops, "_launch", lambda *args: None)
         ref = attempt()
-    if isinstance(out, type) or isinstance(ref, type):
+    if native is not None:
+        assert taken and all(t is native for t in taken), taken
+    if raises is not None:
         assert out is ref
     else:
         _same(out, ref)
@@ -60,16 +74,17 @@ def _both(monkeypatch, call):
 
 
 def _layouts(shape, dtype, gpu, seed):
-    """Tensors of one shape in the layouts that reach the launchers."""
+    """(tensor, the launchers take it) in the layouts that reach the launchers, of one shape and
+    dtype; then another dtype and an empty tensor."""
 
     t = randn(shape, dtype, gpu, seed)
-    yield t
-    yield randn((*shape[:-1], shape[-1] + 3), dtype, gpu, seed + 1)[..., :-3]
-    yield randn(tuple(reversed(shape)), dtype, gpu, seed + 2).permute(*range(len(shape) - 1, -1, -1))
-    yield randn((1,) * len(shape), dtype, gpu, seed + 3).expand(shape)
-    yield randn((t.numel() + 1,), dtype, gpu, seed + 4)[1:].view(shape)
-    yield t.float() if dtype != torch.float32 else t.bfloat16()
-    yield t[:0]
+    yield t, True
+    yield randn((*shape[:-1], shape[-1] + 3), dtype, gpu, seed + 1)[..., :-3], False
+    yield randn(tuple(reversed(shape)), dtype, gpu, seed + 2).permute(*range(len(shape) - 1, -1, -1)), False
+    yield randn((1,) * len(shape), dtype, gpu, seed + 3).expand(shape), False
+    yield randn((t.numel() + 1,), dtype, gpu, seed + 4)[1:].view(shape), True
+    yield t.float() if dtype != torch.float32 else t.bfloat16(), False
+    yield t[:0], False
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -78,21 +93,24 @@ def test_norm_and_swiglu_forms(gpu, monkeypatch, dtype):
     w = randn((70,), dtype, gpu, 1, 0.1, 1.0)
     base = randn(shape, dtype, gpu, 2)
     _, rstd = ops.rmsnorm_fwd(base, w, 1e-5)
-    for i, t in enumerate(_layouts(shape, dtype, gpu, 10)):
-        _both(monkeypatch, lambda: ops.rmsnorm_fwd(t, w, 1e-5))
-        _both(monkeypatch, lambda: ops.residual_rmsnorm_fwd(base, t, w, 1e-5))
-        _both(monkeypatch, lambda: ops.swiglu_fwd(base, t))
+    for t, plain in _layouts(shape, dtype, gpu, 10):
+        # a norm takes rows of any of its types; two inputs of one call have to match
+        _both(monkeypatch, lambda: ops.rmsnorm_fwd(t, w, 1e-5), native=plain or t.dtype != dtype)
+        pair = dict(native=plain) if t.shape == base.shape and t.dtype == dtype else dict(raises=ValueError)
+        _both(monkeypatch, lambda: ops.residual_rmsnorm_fwd(base, t, w, 1e-5), **pair)
+        _both(monkeypatch, lambda: ops.swiglu_fwd(base, t), **pair)
         if t.numel():  # a gradient has its output's shape
             for need in ((True, True), (True, False), (False, True), (False, False)):
-                _both(monkeypatch, lambda: ops.rmsnorm_bwd(t, base, w, rstd, *need))
-                _both(monkeypatch, lambda: ops.swiglu_bwd(t, base, base, *need))
-            _both(monkeypatch, lambda: ops.residual_rmsnorm_bwd(t, None, base, w, rstd))
-            _both(monkeypatch, lambda: ops.residual_rmsnorm_bwd(base, t, base, w, rstd, need_dw=False))
-    for bad in (w[:-1], w.view(1, 70), w.double(), w.cpu(), w[::2]):
-        _both(monkeypatch, lambda: ops.rmsnorm_fwd(base, bad, 1e-5))
-    assert _both(monkeypatch, lambda: ops.swiglu_fwd(base, base[:, :2])) is ValueError
-    assert _both(monkeypatch, lambda: ops.rmsnorm_fwd(base.cpu(), w.cpu(), 1e-5)) is ValueError
-    assert _both(monkeypatch, lambda: ops.rmsnorm_bwd(base, base, w, rstd.view(-1)[1:])) is ValueError
+                _both(monkeypatch, lambda: ops.rmsnorm_bwd(t, base, w, rstd, *need), native=plain and any(need))
+                _both(monkeypatch, lambda: ops.swiglu_bwd(t, base, base, *need), native=plain)
+            _both(monkeypatch, lambda: ops.residual_rmsnorm_bwd(t, None, base, w, rstd), native=plain)
+            _both(monkeypatch, lambda: ops.residual_rmsnorm_bwd(base, t, base, w, rstd, need_dw=False), native=plain)
+    for bad in (w[:-1], w.view(1, 70), w.cpu(), w[::2]):
+        _both(monkeypatch, lambda: ops.rmsnorm_fwd(base, bad, 1e-5), raises=ValueError)
+    _both(monkeypatch, lambda: ops.rmsnorm_fwd(base, w.double(), 1e-5), raises=TypeError)
+    _both(monkeypatch, lambda: ops.swiglu_fwd(base, base[:, :2]), raises=ValueError)
+    _both(monkeypatch, lambda: ops.rmsnorm_fwd(base.cpu(), w.cpu(), 1e-5), raises=ValueError)
+    _both(monkeypatch, lambda: ops.rmsnorm_bwd(base, base, w, rstd.view(-1)[1:]), raises=ValueError)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -102,14 +120,19 @@ def test_rope_forms(gpu, monkeypatch, dtype, layout):
     q = randn((2, 7, 4, 16), dtype, gpu, 3).transpose(1, 2)
     keys = [randn((2, 7, 2, 16), dtype, gpu, 4).transpose(1, 2), randn((2, 2, 7, 16), dtype, gpu, 5),
             randn((2, 2, 7, 20), dtype, gpu, 6)[..., 2:18], randn((1, 1, 1, 16), dtype, gpu, 7).expand(2, 2, 7, 16),
-            None, randn((2, 2, 16, 7), dtype, gpu, 8).transpose(2, 3), randn((2, 2, 7, 14), dtype, gpu, 9)]
-    for k in keys:
-        for inverse in (False, True):
-            _both(monkeypatch, lambda: ops.rope(q, cos, sin, layout=layout, inverse=inverse, x1=k))
-    for c, s in ((cos[:3], sin[:3]), (cos.double(), sin.double()), (cos[:, :4], sin[:, :4]), (cos.t(), sin.t()),
-                 (randn((16, 9), torch.float32, gpu, 10)[:8].t(), sin)):
-        _both(monkeypatch, lambda: ops.rope(q, c, s, layout=layout))
-    assert _both(monkeypatch, lambda: ops.rope(q, cos, sin, layout="other")) is ValueError
+            None]
+    bad = [randn((2, 2, 16, 7), dtype, gpu, 8).transpose(2, 3), randn((2, 2, 7, 14), dtype, gpu, 9)]
+    for inverse in (False, True):
+        for k in keys:
+            _both(monkeypatch, lambda: ops.rope(q, cos, sin, layout=layout, inverse=inverse, x1=k), native=True)
+        for k in bad:
+            _both(monkeypatch, lambda: ops.rope(q, cos, sin, layout=layout, inverse=inverse, x1=k), raises=ValueError)
+    for c, s in ((cos.double(), sin.double()), (cos[:, :4], sin[:, :4]), (cos.t(), sin.t())):
+        _both(monkeypatch, lambda: ops.rope(q, c, s, layout=layout), raises=ValueError)
+    _both(monkeypatch, lambda: ops.rope(q, cos[:3], sin[:3], layout=layout), raises=_lib.HipKernelError)
+    strided = randn((16, 9), torch.float32, gpu, 10)[:8].t()
+    _both(monkeypatch, lambda: ops.rope(q, strided, sin, layout=layout), native=False)
+    _both(monkeypatch, lambda: ops.rope(q, cos, sin, layout="other"), raises=ValueError)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -145,13 +168,16 @@ def test_cross_entropy_forms(gpu, monkeypatch, dtype):
     calls = [(logits, ids, 1), (wide, ids, 1), (logits, ids[:, 1:], 2), (wide, ids[:, 1:], 2),
              (logits.transpose(0, 1).contiguous().transpose(0, 1), ids, 1),
              (logits.view(-1, v), ids.view(-1), 0), (logits.transpose(1, 2), ids, 0),
-             (wide.transpose(1, 2), ids, 0), (logits[:, 0], ids[:, 0], 0), (logits.view(-1, v), ids.view(-1)[::1][:5], 0),
-             (logits, ids[:, :3], 1), (logits, ids.int(), 1), (logits.transpose(0, 2).contiguous(), ids, 1)]
-    for x, t, shift in calls:
-        for write, form in ((False, "in"), (True, "in"), (True, "out")):
-            _both(monkeypatch, lambda: loss_of(x, t, shift, write, form))
+             (wide.transpose(1, 2), ids, 0), (logits[:, 0], ids[:, 0], 0)]
+    bad = [(logits.view(-1, v), ids.view(-1)[:5], 0), (logits, ids[:, :3], 1), (logits, ids.int(), 1),
+           (logits.transpose(0, 2).contiguous(), ids, 1)]
+    for write, form in ((False, "in"), (True, "in"), (True, "out")):
+        for x, t, shift in calls:
+            _both(monkeypatch, lambda: loss_of(x, t, shift, write, form), native=True)
+        for x, t, shift in bad:
+            _both(monkeypatch, lambda: loss_of(x, t, shift, write, form), raises=ValueError)
     expanded = logits[:1].expand(b, s, v)
-    assert _both(monkeypatch, lambda: loss_of(expanded, ids, 1, True, "expanded")) is ValueError
+    _both(monkeypatch, lambda: loss_of(expanded, ids, 1, True, "expanded"), raises=ValueError)
     for x in (logits, wide, expanded):  # the gradient buffer itself: same strides and phase
         got = ops.ce_grad_buffer(x, 2)
         if x is expanded:
