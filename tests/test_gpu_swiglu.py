@@ -143,3 +143,22 @@ def test_streams_off_16_byte_boundaries_at_the_ends_of_their_rules(gpu, dtype, n
     dg, du = ops.swiglu_bwd(dy, g, u)
     close(dg[tail], dg64, dtype)
     close(du[tail], du64, dtype)
+
+
+@pytest.mark.parametrize("dtype,n", [(torch.float16, 16383 * 2731), (torch.float32, (1 << 24) + 3)])
+def test_large_streams_with_a_tail(gpu, dtype, n):
+    """Aligned streams above 64 MB (nontemporal forward, write-through backward) whose last elements
+    are no whole vector: the tail, written by the first workgroup, and a sample of the body."""
+
+    g, u, dy = (randn((n,), dtype, gpu, n + i) for i in range(3))
+    y = ops.swiglu_fwd(g, u)
+    dg, du = ops.swiglu_bwd(dy, g, u)
+    none, only_up = ops.swiglu_bwd(dy, g, u, need_dgate=False)
+    assert none is None and torch.equal(only_up, du)
+    per = 16 // g.element_size()
+    assert n % per
+    for part in (slice(0, 64), slice(n // 2, n // 2 + 4096), slice(n - 3 * per, n)):
+        close(y[part], o_swiglu.forward(g[part], u[part]), dtype)
+        dg64, du64 = o_swiglu.backward(dy[part], g[part], u[part])
+        close(dg[part], dg64, dtype)
+        close(du[part], du64, dtype)
