@@ -172,9 +172,13 @@ struct RopeWork {
       float oa[P], ob[P];
 #pragma unroll
       for (int p = 0; p < P; ++p) {
+        // Written out, since the compiler's own choice of the product that it rounds differs from
+        // instance to instance: every instance the same.  (For fp16 it may
+        // still fuse the last operation with the conversion, one rounding in place of two.)
         const float sn = sign * s[p];
-        oa[p] = a[p] * c[p] - b[p] * sn;
-        ob[p] = a[p] * sn + b[p] * c[p];
+        oa[p] = __builtin_fmaf(a[p], c[p], -(b[p] * sn));
+        ob[p] = LAYOUT == 0 && ALIGNED ? __builtin_fmaf(a[p], sn, b[p] * c[p])
+                                       : __builtin_fmaf(b[p], c[p], a[p] * sn);
       }
       T* y = ya + u * ystep;
       if constexpr (LAYOUT == 0) {

@@ -179,3 +179,22 @@ def test_items_of_two_heads(gpu, dtype, heads, kv_heads, memory):
             e, sn = x.double()[..., 1::2], sin.double() * (-1 if inverse else 1)
             ref[..., 0::2], ref[..., 1::2] = a * c - e * sn, a * sn + e * c
             close(y, ref, dtype)
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("shape,offset", [((1, 5, 7, 64), 0), ((1, 5, 7, 64), 1), ((2, 32, 1100, 128), 0)])
+def test_products_round_in_one_order(gpu, layout, shape, offset):
+    """The product that is rounded before the other is added does not depend on the instance: the
+    second member's a * sin in general, b * cos on interleaved rows of whole vectors."""
+
+    n = shape[0] * shape[1] * shape[2] * shape[3]
+    x = randn((n + offset,), torch.bfloat16, gpu, 1)[offset:].view(shape)
+    cos, sin = randn((shape[2], shape[3] // 2), torch.float32, gpu, 2), randn((shape[2], shape[3] // 2), torch.float32, gpu, 3)
+    y, _ = ops.rope(x, cos, sin, layout=layout)
+    half = shape[3] // 2
+    first, second = (slice(0, None, 2), slice(1, None, 2)) if layout == "interleaved" else (slice(0, half), slice(half, None))
+    a, b, c, s = x.double()[..., first], x.double()[..., second], cos.double(), sin.double()
+    rounded = lambda t: t.float().double()  # the products are exact in fp64, and no sum here rounds twice
+    assert torch.equal(y[..., first], (a * c - rounded(b * s)).float().bfloat16())
+    other = a * s + rounded(b * c) if layout == "interleaved" and not offset else b * c + rounded(a * s)
+    assert torch.equal(y[..., second], other.float().bfloat16())
