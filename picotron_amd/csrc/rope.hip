@@ -48,6 +48,25 @@ struct RopeTensor {
   int64_t ybytes;  // bytes from y to the end of its last row
 };
 
+// What the kernel reads of a RopeTensor.  A small call is bound by the chain of scalar loads that fetches
+// these arguments: as the host's struct, behind the tables' pointers, they cost it 0.1 us of 2.1.
+struct RopeArgs {
+  const void* x;
+  void* y;
+  int64_t xs[3];
+  int64_t ys[3];
+  int64_t xstep;
+  int64_t ystep;
+  uint32_t n1, n2;  // n[1], n[2]
+  uint32_t heads;
+  uint32_t chunks;
+  uint32_t items;
+  uint32_t blocks;
+  int seq_dim;
+  int head_dim;
+  int ybytes;  // write-through stores only
+};
+
 // One work item in two phases, so that a thread has every head's loads in flight before it
 // computes and stores any of them (the output may alias the input, so the
 // compiler would not move a later head's loads above an earlier head's stores).  The pair
@@ -57,19 +76,19 @@ struct RopeTensor {
 // items by 2^32), so they are decoded with 32-bit divisions; only memory offsets are 64-bit.
 // WT (aligned rows only): stores through a buffer resource over y with the write-through
 // policy instead of nontemporal global stores.
-// Heads per item: two for interleaved rows, whose item is one vector of 16 bytes per head beside 32
+// Heads per item (U): two for interleaved rows, whose item is one vector of 16 bytes per head beside 32
 // bytes of cos and sin; one for rotate-half rows (two vectors beside 64 bytes).  Measured per launch
 // on q [8, 2048, 32, 128] + k [8, 2048, 8, 128] bf16 (the bytes at copy speed: 51.5 us): interleaved one
 // head 55.7, two 53.9, four 54.9, and at [1, 2048] 10.1, 8.9, 8.6; rotate-half 54.7, 55.2, 57.2 and
-// 8.6, 8.3, 8.8.
-template <int LAYOUT, bool ALIGNED>
-constexpr int kHeads = ALIGNED && LAYOUT == 0 ? 2 : 1;
+// 8.6, 8.3, 8.8.  Calls of fewer than 65536 vectors (a decode step) are one wave's chain of loads, which the
+// second head only lengthens: interleaved, mean over the sizes up to 16384 vectors two heads 2.16 us
+// and one 2.06, up to 65536 2.24 and 2.14; up to 262144 3.15 and 3.18, up to 1048576 5.84 and 6.15.
+constexpr int64_t kTwoHeadVectors = 65536;
 
-template <typename T, int LAYOUT, bool ALIGNED, bool NT, bool WT>
+template <typename T, int LAYOUT, bool ALIGNED, bool NT, bool WT, int U>
 struct RopeWork {
   static constexpr int V = ALIGNED ? Elem<T>::VEC : 2;
   static constexpr int P = LAYOUT == 0 ? V / 2 : (ALIGNED ? Elem<T>::VEC : 1);  // pairs
-  static constexpr int U = kHeads<LAYOUT, ALIGNED>;
   // Raw storage until store(): converting in load() would wait for the data there.
   Vec16<T> va[U], vb[U];  // aligned: interleaved vector (va) or the two half vectors (va, vb)
   T ea[2], eb[2];   // element path: interleaved (ea[0], ea[1]) or rotate-half (ea[0], eb[0])
@@ -78,19 +97,18 @@ struct RopeWork {
   int64_t ystep;    // from head to head
   int count;        // heads
 
-  __device__ __forceinline__ void load(const RopeTensor& t, uint32_t item, int head_dim,
+  __device__ __forceinline__ void load(const RopeArgs& t, uint32_t item, int head_dim,
                                        const float* __restrict__ cos_t,
                                        const float* __restrict__ sin_t) {
     const int half = head_dim / 2;
     const uint32_t per_row = static_cast<uint32_t>(items_per_row<T, LAYOUT, ALIGNED>(head_dim));
     const uint32_t row = item / per_row;
     const int j = static_cast<int>(item - row * per_row);
-    const uint32_t n2 = static_cast<uint32_t>(t.n[2]), n1 = static_cast<uint32_t>(t.n[1]);
     int64_t idx[3];
-    const uint32_t r1 = row / n2;
-    idx[2] = row - r1 * n2;
-    idx[0] = r1 / n1;
-    idx[1] = r1 - static_cast<uint32_t>(idx[0]) * n1;
+    const uint32_t r1 = row / t.n2;
+    idx[2] = row - r1 * t.n2;
+    idx[0] = r1 / t.n1;
+    idx[1] = r1 - static_cast<uint32_t>(idx[0]) * t.n1;
     const int64_t xo = idx[0] * t.xs[0] + idx[1] * t.xs[1] + idx[2] * t.xs[2];
     const int64_t yo = idx[0] * t.ys[0] + idx[1] * t.ys[1] + idx[2] * t.ys[2];
     // selects, not an indexed array (which would live in scratch memory)
@@ -103,11 +121,11 @@ struct RopeWork {
     if constexpr (ALIGNED) {
       const int64_t xstep = U > 1 ? t.xstep : 0;
       if constexpr (U > 1) {
-        // (a position with whole vectors has fewer than 2^31 heads: pt_rope bounds the pairs by 2^32)
-        const int first =
-            static_cast<int>(t.head_dim == 0 ? idx[0] : (t.head_dim == 1 ? idx[1] : idx[2]));
-        const int heads = static_cast<int>(t.heads), chunks = static_cast<int>(t.chunks);
-        count = (heads - first + chunks - 1) / chunks;
+        static_assert(U == 2 && ALIGNED, "an item's heads are first and first + chunks");
+        // below 2^31: pt_rope bounds the pairs by 2^32, and these rows have at least two vectors
+        const uint32_t first =
+            static_cast<uint32_t>(t.head_dim == 0 ? idx[0] : (t.head_dim == 1 ? idx[1] : idx[2]));
+        count = first + t.chunks < t.heads ? 2 : 1;
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -173,7 +191,7 @@ struct RopeWork {
 #pragma unroll
       for (int p = 0; p < P; ++p) {
         // Written out, since the compiler's own choice of the product that it rounds differs from
-        // instance to instance: every instance the same.  (For fp16 it may
+        // instance to instance: the same bits from every number of heads per item.  (For fp16 it may
         // still fuse the last operation with the conversion, one rounding in place of two.)
         const float sn = sign * s[p];
         oa[p] = __builtin_fmaf(a[p], c[p], -(b[p] * sn));
@@ -206,21 +224,24 @@ struct RopeWork {
 };
 
 // Thread t of block b takes item b * 256 + t of its tensor.
-template <typename T, int LAYOUT, bool ALIGNED, bool NT, bool WT>
-__global__ __launch_bounds__(256) void rope_kernel(RopeTensor t0, RopeTensor t1, int head_dim,
-                                                   const float* __restrict__ cos_t,
-                                                   const float* __restrict__ sin_t, float sign) {
+template <typename T, int LAYOUT, bool ALIGNED, bool NT, bool WT, int U>
+__global__ __launch_bounds__(256) void rope_kernel(const float* __restrict__ cos_t,
+                                                   const float* __restrict__ sin_t, int head_dim,
+                                                   float sign, RopeArgs t0, RopeArgs t1) {
   uint32_t b = blockIdx.x;
-  const RopeTensor* t = &t0;
+  const RopeArgs* t = &t0;
   if (b >= t0.blocks) {
-    b -= static_cast<uint32_t>(t0.blocks);
+    b -= t0.blocks;
     t = &t1;
   }
   const uint32_t item = b * 256u + threadIdx.x;
   // y's span fits a buffer resource whenever WT is set (checked on the host); unused otherwise
-  const auto ybuf = uniform_buffer(t->y, WT ? static_cast<int>(t->ybytes) : 0);
-  if (item >= static_cast<uint32_t>(t->items)) return;
-  RopeWork<T, LAYOUT, ALIGNED, NT, WT> w;
+  const auto ybuf = uniform_buffer(t->y, WT ? t->ybytes : 0);
+  if (item >= t->items) return;
+  // Fetches the table pointers with the other arguments (left alone, the compiler loads them only after
+  // the states' loads, and the tables' loads wait for one more round trip).
+  asm volatile("" : : "s"(cos_t), "s"(sin_t));
+  RopeWork<T, LAYOUT, ALIGNED, NT, WT, U> w;
   w.load(*t, item, head_dim, cos_t, sin_t);
   w.store(sign, head_dim, ybuf, static_cast<const T*>(t->y));
 }
@@ -294,21 +315,20 @@ int rope_occupancy(int layout) {
 }
 
 template <typename K>
-void launch_limited(K kernel, int layout, unsigned grid, hipStream_t st, const RopeTensor& t0,
-                    const RopeTensor& t1, int head_dim, const float* c, const float* s,
+void launch_limited(K kernel, int layout, unsigned grid, hipStream_t st, const RopeArgs& t0,
+                    const RopeArgs& t1, int head_dim, const float* c, const float* s,
                     float sign) {
   size_t lds = occupancy_lds(rope_occupancy(layout), 0);
   if (allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds) != PT_OK) lds = 0;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, st, t0, t1, head_dim, c, s, sign);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, st, c, s, head_dim, sign, t0, t1);
 }
 
-template <typename T, int LAYOUT, bool ALIGNED>
+template <typename T, int LAYOUT, bool ALIGNED, int U>
 void launch(RopeTensor& t0, RopeTensor& t1, int head_dim, const float* c, const float* s,
             float sign, hipStream_t st) {
   const int per_row = items_per_row<T, LAYOUT, ALIGNED>(head_dim);
-  constexpr int kPer = kHeads<LAYOUT, ALIGNED>;
   for (RopeTensor* t : {&t0, &t1}) {
-    t->chunks = (t->heads + kPer - 1) / kPer;
+    t->chunks = (t->heads + U - 1) / U;
     t->xstep = t->xs[t->head_dim] * t->chunks;
     t->ystep = t->ys[t->head_dim] * t->chunks;
     t->items = 0;
@@ -330,17 +350,29 @@ void launch(RopeTensor& t0, RopeTensor& t1, int head_dim, const float* c, const 
   const auto fits = [](const RopeTensor& t) {
     return t.rows == 0 || (t.ybytes > 0 && t.ybytes <= 0x7fffffff);
   };
-  if (bytes > kNontemporalBytes) {
-    if (ALIGNED && fits(t0) && fits(t1)) {
-      launch_limited(rope_kernel<T, LAYOUT, ALIGNED, true, ALIGNED>, LAYOUT, static_cast<unsigned>(blocks),
-                     st, t0, t1, head_dim, c, s, sign);
-    } else {
-      launch_limited(rope_kernel<T, LAYOUT, ALIGNED, true, false>, LAYOUT, static_cast<unsigned>(blocks),
-                     st, t0, t1, head_dim, c, s, sign);
-    }
+  const auto args = [](const RopeTensor& t) {
+    RopeArgs a{t.x, t.y, {t.xs[0], t.xs[1], t.xs[2]}, {t.ys[0], t.ys[1], t.ys[2]}, t.xstep, t.ystep};
+    a.n1 = static_cast<uint32_t>(t.n[1]);
+    a.n2 = static_cast<uint32_t>(t.n[2]);
+    a.heads = static_cast<uint32_t>(t.heads);
+    a.chunks = static_cast<uint32_t>(t.chunks);
+    a.items = static_cast<uint32_t>(t.items);
+    a.blocks = static_cast<uint32_t>(t.blocks);
+    a.seq_dim = t.seq_dim;
+    a.head_dim = t.head_dim;
+    a.ybytes = static_cast<int>(t.ybytes);
+    return a;
+  };
+  const auto go = [&](auto kernel) {
+    launch_limited(kernel, LAYOUT, static_cast<unsigned>(blocks), st, args(t0), args(t1), head_dim, c, s,
+                   sign);
+  };
+  if (bytes <= kNontemporalBytes) {
+    go(rope_kernel<T, LAYOUT, ALIGNED, false, false, U>);
+  } else if (ALIGNED && fits(t0) && fits(t1)) {
+    go(rope_kernel<T, LAYOUT, ALIGNED, true, ALIGNED, U>);
   } else {
-    launch_limited(rope_kernel<T, LAYOUT, ALIGNED, false, false>, LAYOUT, static_cast<unsigned>(blocks),
-                   st, t0, t1, head_dim, c, s, sign);
+    go(rope_kernel<T, LAYOUT, ALIGNED, true, false, U>);
   }
 }
 
@@ -348,16 +380,18 @@ template <typename T>
 void launch_t(int layout, bool aligned, RopeTensor& t0, RopeTensor& t1, int head_dim,
               const float* c, const float* s, float sign, hipStream_t st) {
   if (layout == 0) {
-    if (aligned) {
-      launch<T, 0, true>(t0, t1, head_dim, c, s, sign, st);
+    if (!aligned) {
+      launch<T, 0, false, 1>(t0, t1, head_dim, c, s, sign, st);
+    } else if ((t0.rows + t1.rows) * head_dim / Elem<T>::VEC < kTwoHeadVectors) {
+      launch<T, 0, true, 1>(t0, t1, head_dim, c, s, sign, st);
     } else {
-      launch<T, 0, false>(t0, t1, head_dim, c, s, sign, st);
+      launch<T, 0, true, 2>(t0, t1, head_dim, c, s, sign, st);
     }
   } else {
     if (aligned) {
-      launch<T, 1, true>(t0, t1, head_dim, c, s, sign, st);
+      launch<T, 1, true, 1>(t0, t1, head_dim, c, s, sign, st);
     } else {
-      launch<T, 1, false>(t0, t1, head_dim, c, s, sign, st);
+      launch<T, 1, false, 1>(t0, t1, head_dim, c, s, sign, st);
     }
   }
 }

@@ -198,3 +198,35 @@ def test_products_round_in_one_order(gpu, layout, shape, offset):
     assert torch.equal(y[..., first], (a * c - rounded(b * s)).float().bfloat16())
     other = a * s + rounded(b * c) if layout == "interleaved" and not offset else b * c + rounded(a * s)
     assert torch.equal(y[..., second], other.float().bfloat16())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("heads,kv_heads", [(1, 1), (2, 3), (5, 2), (9, 3)])
+@pytest.mark.parametrize("memory", ["bshd", "bhsd", "sbhd"])
+def test_one_and_two_heads_per_item_agree(gpu, dtype, heads, kv_heads, memory):
+    """Interleaved calls of 65536 vectors or more take two heads per item, smaller ones one: the same
+    bits (in fp16 but for ties of the last rounding, which the compiler may fuse with the one
+    before), with odd head counts and the heads at any stride order of the memory."""
+
+    b, d = 2, 32
+    per_position = b * (heads + kv_heads) * d * torch.tensor([], dtype=dtype).element_size() // 16
+    s = 65536 // per_position + 1  # two heads; a position less leaves one
+    order = {"bshd": (0, 2, 1, 3), "bhsd": (0, 1, 2, 3), "sbhd": (1, 2, 0, 3)}[memory]  # (b, h, s, d) from memory
+
+    def make(h, seed):
+        sizes = {"bshd": (b, s, h, d), "bhsd": (b, h, s, d), "sbhd": (s, b, h, d)}[memory]
+        return randn(sizes, dtype, gpu, seed).permute(*order)
+
+    q, k = make(heads, 1), make(kv_heads, 2)
+    cos, sin = randn((s, d // 2), torch.float32, gpu, 3), randn((s, d // 2), torch.float32, gpu, 4)
+    for inverse in (False, True):
+        two = ops.rope(q, cos, sin, inverse=inverse, x1=k)
+        cut = s // 2
+        one = ops.rope(q[:, :, :cut], cos, sin, inverse=inverse, x1=k[:, :, :cut])
+        for x, y, z in zip((q, k), two, one):
+            assert y.stride() == x.stride()
+            differing = int((y[:, :, :cut] != z).sum())
+            assert differing <= (z.numel() * 1e-3 + 2 if dtype == torch.float16 else 0)
+            close(z, y[:, :, :cut], dtype)
+            ref = o_rope.rotate(x, cos, -sin if inverse else sin, "interleaved")
+            close(y, ref, dtype, scale=float(x.abs().max()) * float(cos.abs().max()))
