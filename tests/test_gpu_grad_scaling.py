@@ -168,3 +168,27 @@ def test_gradient_walks_over_ranges_that_cross_tensors(gpu, sizes, offset):
     ops.grad_scale(table, blocks, torch.full((), 0.37, device=gpu))
     for g, b in zip(grads, before):
         assert torch.equal(g, b * torch.full((), 0.37, device=gpu))
+
+
+@pytest.mark.parametrize("sizes", [[1], [1024], [1025], [3, 1024, 5], [768] * 9, [1023, 1025, 2047, 2049, 4097],
+                                   [33_554_432], [33_554_433], [33_550_000, 7, 9000]])
+def test_statistics_and_scaling_by_waves_and_by_workgroups(gpu, sizes):
+    """Up to 32768 blocks (on 256 CUs) every wave takes one block of the table, above a workgroup takes
+    a range: norm, overflow flag and scaled gradients over blocks of one, of whole and of broken
+    vectors, with the bad value in each tensor's last element."""
+
+    grads = [randn((n + i % 3,), torch.float32, gpu, n + i, 0.5)[i % 3:] for i, n in enumerate(sizes)]
+    table, blocks = ops.adamw_table(grads, grads, grads, grads)
+    table = table.to(gpu)
+    inv = torch.tensor([0.25], device=gpu)
+    norm, _, found = ops.grad_stats(table, blocks, inv)
+    ref = torch.stack([(g.double() * 0.25).square().sum() for g in grads]).sum().sqrt()
+    assert abs(float(norm) - float(ref)) <= 1e-6 * float(ref) and int(found) == 0
+    before = [g.clone() for g in grads]
+    ops.grad_scale(table, blocks, inv)
+    for g, old in zip(grads, before):
+        assert torch.equal(g, old * 0.25)
+    for g in grads:
+        g[-1] = float("inf")
+        assert int(ops.grad_stats(table, blocks, inv)[2]) == 1
+        g[-1] = 0.0
