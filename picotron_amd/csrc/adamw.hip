@@ -127,17 +127,13 @@ __device__ __forceinline__ void device_step_scalars(AdamScalars& s, const DevSte
 // leaves a skipped step's gradients (the caller advances no step count then).
 template <bool SCALED, bool DEVSTEP>
 __global__ __launch_bounds__(kThreads) void adamw_kernel(const AdamRec* __restrict__ table,
-                                                         int64_t ntensors, AdamScalars s,
+                                                         int64_t ntensors, uint32_t last, AdamScalars s,
                                                          const float* __restrict__ grad_scale,
                                                          int write_grad, DevStep ds,
                                                          const int* __restrict__ found,
                                                          const float* __restrict__ inv_scale) {
-  // SCALED steps follow the gradient statistics, whose last-read gradients are still in the
-  // Infinity Cache: they take the blocks from the end, those gradients first.  Clip + step, one
-  // process, alternated: 1.04e9 parameters 6535 -> 6427 and 6449 -> 6346 us (two sets of buffers),
-  // 4.3e8 2500 -> 2426 and 2446 -> 2405, 9.4e7 528 -> 526 and 522 -> 515.  (With plain instead of
-  // nontemporal loads in the statistics the large lists gain half of that.)
-  const int64_t blk = SCALED ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+  // `last` > 0 (the grid's last block): the blocks are taken from the end (launch_step).
+  const int64_t blk = SCALED && last > 0 ? last - blockIdx.x : blockIdx.x;
   const int64_t row = find_tensor(table, ntensors, blk);
   const AdamRec r = table[row];
   const int64_t start = (blk - r.first_block) * kBlockElems;
@@ -417,8 +413,15 @@ int launch_step(const int64_t* table, int64_t n_tensors, int64_t total_blocks, A
   const auto kernel = adamw_kernel<SCALED, DEVSTEP>;
   size_t lds = occupancy_lds(step_occupancy(), 0);
   if (allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds) != PT_OK) lds = 0;
+  // A scaled step follows the gradient statistics, whose last-read gradients are still in the
+  // Infinity Cache: a large one takes the blocks from the end, those gradients first.  Clip + step,
+  // forward against reversed, us: 1.07e9 parameters 6420-6440 and 6367-6372 (three alternated runs), 4.3e8
+  // 2448 and 2452, 2.7e8 1636 and 1634 in one tensor, 1487 and 1512 in 64, 1e8 576 and 585, 1.7e7 103.6 and
+  // 105.1.
+  constexpr int64_t kReverseBlocks = int64_t{1} << 19;  // 5.4e8 elements
+  const uint32_t last = total_blocks >= kReverseBlocks ? static_cast<uint32_t>(total_blocks - 1) : 0;
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(total_blocks)), dim3(kThreads), lds,
-                     as_stream(stream), reinterpret_cast<const AdamRec*>(table), n_tensors, s,
+                     as_stream(stream), reinterpret_cast<const AdamRec*>(table), n_tensors, last, s,
                      grad_scale, write_grad, d, found, inv_scale);
   return check_launch(fn);
 }

@@ -92,6 +92,26 @@ def test_rope_at_the_write_through_limit(gpu, s):
         del y
 
 
+def test_scaled_adamw_step_in_reverse_order(gpu):
+    """From 2^19 blocks on a scaled step takes its blocks from the end: the same bits as smaller steps
+    over parts of the same tensors."""
+
+    sizes = [(1 << 28) + 5, (1 << 28) - 1024, 3000]
+    tensors = [[_randn(n, torch.float32, gpu, 60 + 4 * i + k, 0.1).abs_() for k in range(4)] for i, n in enumerate(sizes)]
+    parts = [[t.clone() for t in quad] for quad in tensors]
+    hyper = dict(lr=1e-2, beta1=0.9, beta2=0.95, eps=1e-8, weight_decay=0.1, step=3.0)
+    scale = torch.tensor([0.5], device=gpu)
+    table, blocks = ops.adamw_table(*zip(*tensors))
+    assert blocks >= 1 << 19
+    ops.adamw_step_scaled(table.to(gpu), blocks, scale, write_grad=True, **hyper)
+    for quad, want in zip(tensors, parts):
+        table, blocks = ops.adamw_table(*([t] for t in want))
+        assert blocks < 1 << 19
+        ops.adamw_step_scaled(table.to(gpu), blocks, scale, write_grad=True, **hyper)
+        for got, ref in zip(quad, want):
+            assert torch.equal(got, ref)
+
+
 def test_rope_past_2_31_heads(gpu):
     """As many heads as fit the kernel's 2^32 pairs: their count does not fit 31 bits."""
 
