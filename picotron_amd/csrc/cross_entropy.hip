@@ -1228,10 +1228,11 @@ __global__ __launch_bounds__(256) void ce_scale_kernel(T* logits, const T* src, 
     bool has_head = false, has_tail = false;
     const int tail_j = lead + nbody * V + tid;
     if constexpr (!ALIGNED) {
-      const int last_c = nbody > 0 ? (nbody - 1) / chunk_vecs : 0;
       const bool read = !(kDefer && skip);  // an ignored fp16 row is written as zeros
+      // the body's last chunk, or the first of a row without a body
+      const bool last = (cstart < nbody || c == 0) && nbody - cstart <= chunk_vecs;
       has_head = c == 0 && tid < lead;
-      has_tail = c == last_c && tid < V && tail_j < vocab;
+      has_tail = last && tid < V && tail_j < vocab;
       if (has_head && read) head_v = q[tid];
       if (has_tail && read) tail_v = q[tail_j];
     }
