@@ -12,20 +12,25 @@
 // device-scope fences:
 //   1. ce_prepare (before a gradient): one block counts the non-ignored targets (n_valid) into the
 //      workspace and clears the status word.
-//   2. ce_rows: one 1024-thread workgroup per row.  The row is loaded once into registers
-//      (VPT 16-byte vectors per thread, raw buffer loads whose hardware range check drops
-//      the ragged end) and reduced by an online max / sum of exp(x - max) as the vectors
-//      arrive; each exp is kept in the registers in place of its logit, so the gradient
-//      softmax / n_valid is written from registers with one multiply per element and no
-//      second exponential: HBM sees one read and one write of the logits.  The target
-//      element's gradient (softmax_t - 1) / n_valid comes from the exact fp32 target logit.
-//      Longer or unaligned rows use ce_rows_batched (two passes, batches of loads in flight,
-//      the second pass served largely by the Infinity Cache).
-//      Each row's fp32 loss goes to the workspace.  When no gradient is written in the
-//      forward -- the loss alone, or fp16 logits, which are left as they are -- aligned rows
-//      take ce_lse instead: a read-only stream, 256-thread workgroups several to a CU, that
-//      also keeps the row's log-sum-exp for fp16, whose backward (ce_scale) then writes the
-//      gradient with grad_output applied, rounding to fp16 once.
+//   2. one row kernel, by the row's length and alignment, which leaves each row's fp32 loss in the
+//      workspace and, for fp32 and bf16 with a gradient, writes it; HBM sees one read and one write of
+//      the logits:
+//      - ce_short: rows of up to 1536 16-byte vectors with a gradient, 1024 without, at any
+//        alignment.  One wave or four per row, the row and its exps in registers.
+//      - ce_lse: longer rows without a gradient in the forward -- the loss alone, or fp16 logits, which
+//        are left as they are.  A read-only stream at any alignment, 256-thread workgroups several to a
+//        CU.  Like ce_short it keeps the row's log-sum-exp for fp16, whose backward (ce_scale)
+//        writes the gradient with grad_output applied, rounding to fp16 once.
+//      - ce_rows: longer rows with a gradient that start on a line, up to 16 vectors for each of a
+//        1024-thread workgroup's threads.  The row is loaded once into registers (raw buffer loads
+//        whose hardware range check drops the ragged end) and reduced by an online max / sum of
+//        exp(x - max) as the vectors arrive; each exp is kept in the registers in place of its logit,
+//        so the gradient softmax / n_valid is written from registers with one multiply per element and no
+//        second exponential.  The target element's gradient (softmax_t - 1) / n_valid comes from
+//        the exact fp32 target logit.
+//      - ce_rows_batched: the other rows with a gradient (unaligned, or longer, whose second pass
+//        is served largely by the Infinity Cache).
+//      - ce_rows_stream: rows of 2 GB and more.
 //   3. ce_finish: one block sums the per-row losses in a fixed order and divides by
 //      n_valid (which it counts itself where ce_prepare did not run), so the loss is bitwise
 //      reproducible.
@@ -304,7 +309,7 @@ constexpr uint32_t kNegInfWord = std::is_same<T, float>::value      ? 0xff800000
 //      vector store of that address, the target element (softmax_t - 1) / n_valid.
 // Keeping e rounds the softmax twice in 16-bit storage (once as e, once as the gradient),
 // a relative error of at most 2 units of the storage type's last place.
-// The launch picks the smallest VPT of 1, 2, 3, 4, 6, 7, 8, 10, 12, 14, 16 that covers the
+// The launch picks the smallest VPT of 2, 3, 4, 6, 7, 8, 10, 12, 14, 16 that covers the
 // row; each is at most twice the one before, so the vectors of chunks k < VPT / 2 are always
 // inside it.
 // Up to 64 VGPRs a CU holds two of these workgroups, one loading while the other reduces or
@@ -1312,10 +1317,6 @@ void launch_rows(const CeRows& d, int write_grad, CeWork* ws, int64_t rows, hipS
                      d.ignore_index, write_grad, ws);
 }
 
-// Register-resident rows for up to 16 vectors per thread (131072 fp16/bf16 or 65536 fp32
-// elements) when every row is 16-byte aligned and, up to 8 vectors per thread, starts on a
-// 128-byte line; other rows take the batched kernel (the element-wise stream only for rows
-// of 2 GB and more).
 template <typename T, int VPL, int WPR>
 void launch_short(const CeRows& d, int write_grad, CeWork* ws, int64_t rows, hipStream_t st) {
   constexpr int RPB = WPR == 1 ? 4 : 1;
@@ -1351,6 +1352,10 @@ bool dispatch_short(const CeRows& d, int write_grad, CeWork* ws, int64_t rows, h
   return false;
 }
 
+// Short rows first (dispatch_short), then rows that the forward does not write.  The others:
+// register-resident for up to 16 vectors per thread (131072 bf16 or 65536 fp32 elements) when every row
+// is 16-byte aligned and starts on a 128-byte line; other rows take the batched kernel (the
+// element-wise stream only for rows of 2 GB and more).
 template <typename T>
 void dispatch_rows(bool aligned, bool lines, const CeRows& d, int write_grad, CeWork* ws, int64_t rows,
                    hipStream_t st) {
@@ -1376,7 +1381,6 @@ void dispatch_rows(bool aligned, bool lines, const CeRows& d, int write_grad, Ce
     launch_rows<T, N>(d, write_grad, ws, rows, st);    \
     return;                                            \
   }
-      PT_CE_CASE(1)
       PT_CE_CASE(2)
       PT_CE_CASE(3)
       PT_CE_CASE(4)
@@ -1390,7 +1394,7 @@ void dispatch_rows(bool aligned, bool lines, const CeRows& d, int write_grad, Ce
 #undef PT_CE_CASE
     }
     if (row_bytes + kStreamBatchBytes < (int64_t{1} << 31)) {
-      // Rows whose body fits in 1, 2, 4, 6, 7, 8, 10, 12, 14 or 16 kept chunks are read
+      // Rows whose body fits in 2, 4, 6, 7, 8, 10, 12, 14 or 16 kept chunks are read
       // once; longer rows keep kKeepChunks and stream the rest twice.  Up to 8 kept chunks
       // leave room for two workgroups per CU.
 #define PT_CE_BATCHED(K)                                                                        \
@@ -1400,9 +1404,7 @@ void dispatch_rows(bool aligned, bool lines, const CeRows& d, int write_grad, Ce
                      static_cast<const T*>(d.logits), static_cast<T*>(d.grad), d.inner,          \
                      d.valid_inner, d.os, d.is, d.gos, d.gis, d.vocab, d.targets, d.tos, d.tis,  \
                      d.ignore_index, write_grad, ws)
-      if (per_thread <= 1) {
-        PT_CE_BATCHED(1);
-      } else if (per_thread <= 2) {
+      if (per_thread <= 2) {
         PT_CE_BATCHED(2);
       } else if (per_thread <= 4) {
         PT_CE_BATCHED(4);
