@@ -883,8 +883,8 @@ class CrossEntropyTrainFp16Workload(CrossEntropyTrainWorkload):
         self.leaf = self.leaf.detach().half().requires_grad_(True)
         rows = b * s
         self.bytes_per_step = 3 * rows * v * 2 + 16 * rows  # forward: read; backward: read + write
-        self.dominant = ("shifted cross-entropy fp16 forward + autograd backward (ce_prepare_kernel + "
-                         "ce_lse_kernel + ce_finish_kernel, then ce_scale_kernel writing the gradient)")
+        self.dominant = ("shifted cross-entropy fp16 forward + autograd backward (ce_lse_kernel + "
+                         "ce_finish_kernel, then ce_scale_kernel writing the gradient)")
         self.dominant_bytes = self.bytes_per_step
         self.description = (
             f"train-loop loss on fp16 model logits [{b}, {s}, {v}] ~N(0,2^2) against input_ids[:, 1:] "
@@ -965,8 +965,8 @@ class CrossEntropyDemoFp16Workload(CrossEntropyTrainFp16Workload):
         # rows written (the last position's rows as zeros)
         self.bytes_per_step = (2 * b * (s - 1) + b * s) * v * 2 + 16 * b * s
         self.tokens_per_step = b * (s - 1)
-        self.dominant = ("cross-entropy of the reference's call, fp16: ce_prepare_kernel + ce_lse_kernel + "
-                         "ce_finish_kernel, then ce_scale_kernel writing the scaled gradient to a new buffer")
+        self.dominant = ("cross-entropy of the reference's call, fp16: ce_lse_kernel + ce_finish_kernel, "
+                         "then ce_scale_kernel writing the scaled gradient to a new buffer")
         self.dominant_bytes = self.bytes_per_step
         self.description = (
             f"the reference's train-loop call on fp16 model logits [{b}, {s}, {v}] ~N(0,2^2): "

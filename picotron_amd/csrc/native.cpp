@@ -1,8 +1,8 @@
 // Launchers of the C ABI for torch tensors: shape and layout checks, output allocation and the
 // library call in one native function each, in place of the same steps in Python.
 //
-// What bounds a small call is the host: through Python and ctypes an RMSNorm forward takes 16 us
-// of host time and its backward 21, where the kernels take 2-7.  These functions take the plain
+// What bounds a small call is the host: through Python and ctypes an RMSNorm forward takes 11 us
+// of host time and its backward 15 ([64, 256] bf16), this way 6 and 9, where the kernels take 2-7.  These functions take the plain
 // case only -- ordinary dense GPU tensors in the layout that the kernels read -- and return None for
 // anything else (another layout, another dtype, a tensor without storage, an empty one, a shape
 // that does not match), untouched, so that the general route in ops.py copies, converts or raises

@@ -190,7 +190,7 @@ def _scan(optimizer: Optimizer) -> _Scan | None:
     """The fast form of :func:`_plan` and :func:`_prepare` for the usual step -- fp32 parameters,
     gradients and moments on one gfx950 device, every state in place, host step counts equal
     within a group.  None for anything else, which then goes through those two and their checks.
-    147 tensors take 60 us of host time this way, 640 through Python."""
+    A step of 147 tensors takes 43 us of host time this way and 580 through Python, clip + step 61 and 670."""
 
     if not isinstance(optimizer, torch.optim.AdamW) or not _lib.is_available():
         return None

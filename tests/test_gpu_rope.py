@@ -158,8 +158,9 @@ def test_module_shares_one_table_across_sequence_lengths(gpu):
 @pytest.mark.parametrize("heads,kv_heads", [(1, 1), (2, 3), (5, 2), (9, 3)])
 @pytest.mark.parametrize("memory", ["bshd", "bhsd", "sbhd"])
 def test_items_of_two_heads(gpu, dtype, heads, kv_heads, memory):
-    """Interleaved rows on 16-byte vectors take two heads per item: odd head counts leave an item
-    with one, and the heads lie at any stride order of the memory."""
+    """Interleaved rows on 16-byte vectors with odd head counts and the heads at any stride order of
+    the memory (of this size with one head per item; test_one_and_two_heads_per_item_agree has
+    the sizes with two, whose odd counts leave an item with one)."""
 
     b, s, d = 2, 5, 32
     order = {"bshd": (0, 2, 1, 3), "bhsd": (0, 1, 2, 3), "sbhd": (1, 2, 0, 3)}[memory]  # (b, h, s, d) from memory
