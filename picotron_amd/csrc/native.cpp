@@ -568,8 +568,9 @@ PT_FN(adamw_scan, 3)
       if (PyList_Append(g.steps, so) != 0) return nullptr;
       const int64_t n = p->numel(), blocks = (n + per - 1) / per;
       const auto at = [](const at::Tensor& x) { return reinterpret_cast<int64_t>(out(x)); };
-      g.rows.insert(g.rows.end(), {at(*p), at(grad), at(*m), at(*v), n, g.blocks});
-      grads.insert(grads.end(), {at(grad), at(grad), at(grad), at(grad), n, all});
+      const int64_t gp = at(grad);
+      g.rows.insert(g.rows.end(), {at(*p), gp, at(*m), at(*v), n, g.blocks});
+      grads.insert(grads.end(), {gp, gp, gp, gp, n, all});
       g.blocks += blocks;
       all += blocks;
     }
