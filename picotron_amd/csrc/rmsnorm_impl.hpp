@@ -288,11 +288,12 @@ __global__ __launch_bounds__(WAVES * 64) void rmsnorm_fwd_kernel(
 
   LaneWeights<T, WT, VPL, LANES, ALIGNED> wv;
   wv.load(w, wdt, rl, cols);
-  // Eight vectors per lane: every weight before the row.  Left alone, the compiler issues the first
-  // vectors' weights behind the row's loads, and the first store waits for them: [16384, 4096] fp32 88.4 us
-  // against 86.0, [2048, 4096] 13.8 against 13.2, [512, 8192] 8.1 against 7.2.  (Fewer vectors, and the
-  // residual form, gain and lose by it in turn.)
-  if constexpr (!ADD && VPL == 8) __builtin_amdgcn_sched_barrier(0);
+  // Long rows (eight vectors per lane, or four of several waves): every weight before the row.  Left alone,
+  // the compiler issues the first vectors' weights behind the row's loads, and the first store waits for
+  // them: [16384, 4096] fp32 88.4 us against 86.0, [2048, 4096] 13.8 against 13.2, [512, 8192] 8.1 against
+  // 7.2; bf16 [512, 16384] 8.2 against 7.8, [512, 12288] 6.8 against 6.5.  (Shorter rows, [512, 2048] bf16 2.6
+  // against 2.95, and the residual form gain and lose by it in turn.)
+  if constexpr (!ADD && (VPL == 8 || (VPL == 4 && WPR > 1))) __builtin_amdgcn_sched_barrier(0);
 
   using ResRegs = std::conditional_t<ADD, RowRegs<T, VPL>, NoRegs>;
   struct Row {
